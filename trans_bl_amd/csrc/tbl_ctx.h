@@ -29,6 +29,10 @@ struct tbl_ctx {
     std::vector<float *> qdy2_f;
     std::vector<double *> lu_d;   // [K][2][5][ld] per level
     std::vector<float *> lu_f;
+    // inverse line matrices of the coarsest level (coarse_inv_size per mode and
+    // centre/border), null where that form does not fit
+    double *inv_d = nullptr;
+    float *inv_f = nullptr;
     std::vector<tbl::LevelArgs<double>> la_d;
     std::vector<tbl::LevelArgs<float>> la_f;
     std::vector<int> G64, G32;    // lanes per line for each level

@@ -49,9 +49,19 @@ constexpr int kStripShape = 1000;
 // kXStagedShape + G (G lanes per line).
 constexpr int kXStagedShape = 2000;
 
-// Coarsest level only: shape kCoarseSeqShape selects the sequential kernels
-// (one or two threads per line, smooth_coarsest_2s/_reg); any G form there
-// selects the G-lane scan kernel (smooth_coarsest_kernel).
+// Tables of the coarsest level's inverse form, per (mode, centre/border): the
+// wall column g [M], G [M][N] and H [M][N] of x = G S + g v_0 - H X, zero
+// past the ny - 1 rows; N = 4 max(2, ceil((ny - 1) / 4)), M = N rounded up to 16.
+__host__ __device__ inline int coarse_inv_cols(int ny) { return ny <= 9 ? 8 : (ny + 2) / 4 * 4; }
+__host__ __device__ inline int coarse_inv_rows(int ny) { return (coarse_inv_cols(ny) + 15) / 16 * 16; }
+__host__ __device__ inline size_t coarse_inv_size(int ny)
+{
+    return static_cast<size_t>(coarse_inv_rows(ny)) * (1 + 2 * coarse_inv_cols(ny));
+}
+
+// Coarsest level only: shape kCoarseSeqShape selects the inverse form
+// (smooth_coarsest_inv_kernel) where it fits; any G form there selects the
+// G-lane scan kernel (smooth_coarsest_kernel).
 constexpr int kCoarseSeqShape = 1;
 // lanes for a colour-phase sweep on a level whose shape code may be the
 // sequential coarsest form
@@ -120,8 +130,9 @@ template <typename T>
 int strip_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps, T rf,
                  const int *active, int G, cx<T> *halo, hipStream_t st);
 template <typename T>
-int smooth_coarsest(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps,
-                    T rf, const int *active, int G, hipStream_t st);
+int smooth_coarsest(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, const T *inv,
+                    int sweeps, T rf, const int *active, int G, hipStream_t st);
+bool coarse_inv_fits(int nx, int ny);
 template <typename T, typename TO>
 void defect(const LevelArgs<T> &L, const cx<T> *V, const cx<T> *S, cx<TO> *out, T si,
             const int *active, double *resmax, hipStream_t st);

@@ -169,6 +169,20 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
         TRY(dalloc(&c->lu_f[l], luf.size()));
         TBL_HIP(hipMemcpy(c->lu_d[l], lu.data(), sizeof(double) * lu.size(), hipMemcpyHostToDevice));
         TBL_HIP(hipMemcpy(c->lu_f[l], luf.data(), sizeof(float) * luf.size(), hipMemcpyHostToDevice));
+        // the coarsest level's inverse form, from the factors of each line matrix
+        if (l == L - 1 && coarse_inv_fits(lv.nx, lv.ny)) {
+            const size_t sz = coarse_inv_size(lv.ny);
+            std::vector<double> inv(sz * 2 * K, 0.0);
+            for (int q = 0; q < 2 * K; ++q)
+                coarse_inverse(&lu[q * per], d, lv.ny, c->c.sp_poi[l], c->c.cp_poi[l],
+                               1.0 / (12.0 * c->m.dx2[l] * c->g.fac_y), coarse_inv_rows(lv.ny),
+                               coarse_inv_cols(lv.ny), &inv[q * sz]);
+            const std::vector<float> invf(inv.begin(), inv.end());
+            TRY(dalloc(&c->inv_d, inv.size()));
+            TRY(dalloc(&c->inv_f, invf.size()));
+            TBL_HIP(hipMemcpy(c->inv_d, inv.data(), sizeof(double) * inv.size(), hipMemcpyHostToDevice));
+            TBL_HIP(hipMemcpy(c->inv_f, invf.data(), sizeof(float) * invf.size(), hipMemcpyHostToDevice));
+        }
         c->G64[l] = default_G(lv.ny);
         c->G32[l] = default_G(lv.ny);
         // snapshot buffers for the fused-sweep strip smoother (not on the coarsest level)
@@ -179,7 +193,7 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
             if (h32) TRY(dalloc(&c->H32[l], h32));
         }
     }
-    // the coarsest level starts on its sequential kernels
+    // the coarsest level starts on its inverse form
     c->G64[L - 1] = c->G32[L - 1] = kCoarseSeqShape;
     c->la_d.resize(L);
     c->la_f.resize(L);
@@ -297,6 +311,7 @@ extern "C" int tbl_destroy(tbl_ctx *c)
     for (auto *p : c->qdy2_f) fr(p);
     for (auto *p : c->lu_d) fr(p);
     for (auto *p : c->lu_f) fr(p);
+    fr(c->inv_d); fr(c->inv_f);
     for (auto *p : c->H64) fr(p);
     for (auto *p : c->H32) fr(p);
     fr(c->d_active); fr(c->d_cycles); fr(c->d_nactive); fr(c->d_cycle);
@@ -434,7 +449,8 @@ int fas_cycle(tbl_ctx *c, const Sched &s, double tol)
         defect<double, double>(c->la_d[l + 1], c->V[l + 1], c->S[l + 1], c->S[l + 1], 1.0,
                                c->d_active, nullptr, st);
     }
-    TRY(smooth_coarsest<double>(c->la_d[L - 1], c->V[L - 1], c->S[L - 1], c->lu_d[L - 1], s.nc,
+    TRY(smooth_coarsest<double>(c->la_d[L - 1], c->V[L - 1], c->S[L - 1], c->lu_d[L - 1], c->inv_d,
+                                s.nc,
                                 rf_of(s.nc), c->d_active, c->G64[L - 1], st));
     for (int l = L - 1; l >= 1; --l) {
         prolong_level<double>(c->lv[l - 1], c->lv[l], K, c->V[l - 1], c->V[l], c->W[l], 1,
@@ -490,7 +506,7 @@ int correction_vcycle(tbl_ctx *c, const Sched &s, std::vector<cx<float> *> &e, i
             convert<float, float>(c->lv[l + 1].plane * K, e[l + 1], e[l + 1], 1, st);
     }
     // coarsest correction in FP32 too, from the zero the restriction left
-    TRY(smooth_coarsest<float>(c->la_f[L - 1], e[L - 1], c->S32[L - 1], c->lu_f[L - 1], s.nc,
+    TRY(smooth_coarsest<float>(c->la_f[L - 1], e[L - 1], c->S32[L - 1], c->lu_f[L - 1], c->inv_f, s.nc,
                                static_cast<float>(rf_of(s.nc)), c->d_active, c->G32[L - 1], st));
     for (int l = L - 1; l >= t + 1; --l) {
         prolong_level<float>(c->lv[l - 1], c->lv[l], K, e[l - 1], e[l], nullptr, 0, c->d_active,
@@ -551,7 +567,7 @@ int mixed_fmg_cycle(tbl_ctx *c, const Sched &s, double tol)
     for (int l = 0; l < L - 1; ++l)
         restrict_level<float>(c->lv[l], c->lv[l + 1], K, e[l], c->S32[l], e[l + 1], nullptr,
                               c->S32[l + 1], 0, c->d_active, st);
-    TRY(smooth_coarsest<float>(c->la_f[L - 1], e[L - 1], c->S32[L - 1], c->lu_f[L - 1], s.nc,
+    TRY(smooth_coarsest<float>(c->la_f[L - 1], e[L - 1], c->S32[L - 1], c->lu_f[L - 1], c->inv_f, s.nc,
                                static_cast<float>(rf_of(s.nc)), c->d_active, c->G32[L - 1], st));
     convert<float, float>(c->lv[0].plane * K, e[0], e[0], 1, st);
     const bool fused = fused_update(c, s);
@@ -837,10 +853,10 @@ extern "C" int tbl_time_smoother(tbl_ctx *c, int prec, int level, int sweeps, do
     TBL_HIP(hipEventRecord(c->ev0, st));
     if (level == c->L && prec)
         // the coarsest level's solve as each cycle runs it, one launch
-        TRY(smooth_coarsest<float>(c->la_f[l], c->E32[l], c->S32[l], c->lu_f[l], sweeps, 1.0f,
-                                   nullptr, c->G32[l], st));
+        TRY(smooth_coarsest<float>(c->la_f[l], c->E32[l], c->S32[l], c->lu_f[l], c->inv_f,
+                                   sweeps, 1.0f, nullptr, c->G32[l], st));
     else if (level == c->L)
-        TRY(smooth_coarsest<double>(c->la_d[l], c->V[l], c->S[l], c->lu_d[l], sweeps, 1.0,
+        TRY(smooth_coarsest<double>(c->la_d[l], c->V[l], c->S[l], c->lu_d[l], c->inv_d, sweeps, 1.0,
                                     nullptr, c->G64[l], st));
     else if (prec && shape_is_sweep(c->G32[l])) {
         cx<float> *cur = nullptr;

@@ -46,7 +46,7 @@ struct tbl_ctx {
     int last_need = 0;            // cycles the last solve needed (0: it did not converge)
 
     // derivatives
-    double *d_qdy = nullptr, *d_thomas = nullptr, *d_tseg = nullptr;
+    double *d_qdy = nullptr, *d_thomas = nullptr, *d_dtab = nullptr;
     tbl::DerivArgs dargs{};
 
     // staging for the host-pointer entry points (user layout)

@@ -2,299 +2,372 @@
 //
 // Arrays are in the caller's layout: complex (nx, ny, K), x fastest.  Each
 // kernel reads its input once, coalesced, into LDS and produces one or both
-// derivatives of a direction from it (the first and the second derivative
-// of one field share the load: 3 passes for the pair instead of 4).
+// derivatives of a direction from it (3 passes over memory for the pair).
+// The schemes are real, so a line's real and imaginary parts are two
+// independent lines: LDS holds them as two planes and a lane works on one
+// part -- half the registers per row, so twice the wavefronts per SIMD hide
+// the recurrences' latency.
 //  * x (derparx/derparxx, rhsx/rhsxx + tridparx at one rank,
-//    derivs_par.f:80-113, 259-397, 775-858): one wavefront per x-line (j, k);
-//    the line goes to LDS with lane-strided loads, lane t then owns points
-//    [t*R, t*R+R) and the tridiagonal Thomas solve is a per-lane affine map,
-//    a 6-step shuffle scan and a replay, forward and backward.
+//    derivs_par.f:80-113, 259-397, 775-858): a workgroup per x-line (j, k), W
+//    wavefronts per part, R consecutive points per lane.
 //  * y (dery/deryy/deryfv, rhsy/rhsyy/rhsyfv + tridy, derivs_par.f:116-177,
-//    400-611, 947-975): a workgroup holds a tile of 256/G columns x all ny
-//    rows of one mode in LDS (rows loaded coalesced); G lanes solve each
-//    column's line, R rows per lane, with the same scan form.  Results go
-//    back through the tile and out as coalesced rows.
-// The Thomas factors bet_j, gam_j (the reference's recurrence) and 1/bet_j
-// are precomputed on the host; the solve multiplies by 1/bet_j where tridy
-// divides by bet_j (last-bit rounding differs).
-#include "tbl_kernels.h"
+//    400-611, 947-975): a workgroup holds a tile of 8 columns x all ny rows of
+//    one mode; G lanes per column and part, R rows per lane.
+// Results go back through LDS and out as coalesced rows.
+//
+// Thomas solve: u_j = r_j / bet_j - p_j u_{j-1} and x_j = u_j - g_j x_{j+1},
+// p_j = a_j / bet_j, g_j = c_j / bet_j (gam_{j+1} of tridy), the factors from
+// the host.  Each direction is a local solve from a zero state, a scan of the
+// lanes' affine maps and the homogeneous response of the incoming state.  The
+// interior rows' weights are constants (also in y: the grid's ratio is), so
+// the factors converge within 64 rows to the last bit or its neighbour and
+// every row beyond reads one entry: the tables (kTriRows entries) sit in LDS.
+// (Read from global memory, as 6 lane-segmented loads per row or 3 of the
+// short tables, the address and data units were 85-98 % busy.)
+//
+// Both derivatives of 1025x193x64 (608 MB, 116 us at the rate of a copy): x
+// 230 -> 115 us, y 212 -> 160; of 2049x257x32 (809 MB): x 1526 -> 157, y 275 ->
+// 193.  x is bound by memory; y's rows of 128 bytes, mostly on two cache lines
+// each, keep it above that (three workgroups a CU instead of two: no faster).
+#include "tbl_relax.h"
 
 namespace tbl {
 
 using C = cx<double>;
 
-// a where c, else b (component-wise selects, no indexed lookup)
-__device__ __forceinline__ C sel(bool c, C a, C b)
-{
-    return {c ? a.re : b.re, c ? a.im : b.im};
-}
-__device__ __forceinline__ void lds_wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Thomas factors of a scheme in lane-segment order (built on the host for
-// the kernels' G lanes x R rows): entry r*G + t holds row t*R + r of a,
-// 1/bet and gam of the next row (rows past n: 0, 1, 0), so a lane's loads
-// of one r are coalesced across the lanes
-struct Thomas {
-    const double *a, *rbet, *gam1;
+// affine map of a line's scalar state: x -> m x + c
+struct Map {
+    double m, c;
 };
-__device__ __forceinline__ Thomas thomas_seg(const DerivArgs &A, int kind)
+// x after y
+__device__ __forceinline__ Map after(const Map &x, const Map &y)
 {
-    const bool x = kind <= 1;
-    const size_t per = static_cast<size_t>(x ? 64 * A.xR : A.yG * A.yR);
-    const double *t = A.tseg + (x ? kind * 3 * per
-                                   : 2 * 3 * static_cast<size_t>(64 * A.xR) + (kind - 2) * 3 * per);
-    return {t, t + per, t + 2 * per};
+    return {x.m * y.m, __builtin_fma(x.m, y.c, x.c)};
+}
+template <int CTRL>
+__device__ __forceinline__ Map dpp_map(const Map &x)
+{
+    return {dpp<CTRL>(1.0, x.m), dpp0<CTRL>(x.c)};
+}
+__device__ __forceinline__ Map shfl_map(const Map &x, int src, int G)
+{
+    return {__shfl(x.m, src, G), __shfl(x.c, src, G)};
+}
+// inclusive scans of the lanes' maps in lane order / reverse lane order: DPP
+// inside 16-lane rows, shuffles between rows
+template <int G>
+__device__ __forceinline__ Map scan_maps_up(Map x, int lane)
+{
+    x = after(x, dpp_map<0x111>(x));
+    x = after(x, dpp_map<0x112>(x));
+    x = after(x, dpp_map<0x114>(x));
+    x = after(x, dpp_map<0x118>(x));
+    if (G >= 32) {
+        const Map q = shfl_map(x, (lane & 32) + 15, G);
+        if (lane & 16) x = after(x, q);
+    }
+    if (G == 64) {
+        const Map h = shfl_map(x, 31, G);
+        if (lane & 32) x = after(x, h);
+    }
+    return x;
+}
+template <int G>
+__device__ __forceinline__ Map scan_maps_down(Map x, int lane)
+{
+    x = after(x, dpp_map<0x101>(x));
+    x = after(x, dpp_map<0x102>(x));
+    x = after(x, dpp_map<0x104>(x));
+    x = after(x, dpp_map<0x108>(x));
+    if (G >= 32) {
+        const Map q = shfl_map(x, (lane & 32) + 16, G);
+        if (!(lane & 16)) x = after(x, q);
+    }
+    if (G == 64) {
+        const Map h = shfl_map(x, 32, G);
+        if (!(lane & 32)) x = after(x, h);
+    }
+    return x;
 }
 
-// Tridiagonal solve of the n rows held R per lane by G lanes (lane t owns
-// rows t*R .. t*R+R-1; u holds their right-hand sides on entry and the
-// solution on exit): forward u_j = (r_j - a_j u_{j-1}) / bet_j and backward
-// x_j = u_j - gam_{j+1} x_{j+1} (tridy), each as a per-lane affine map of the
-// incoming state, an inclusive shuffle scan over the lanes and a replay.
-template <int G, int R>
-__device__ __forceinline__ void thomas_scan(const Thomas &T, int lane, C (&u)[R])
+// x: table entry of row i of n: converged rows share one, the last two have
+// their own, rows past n the zero entry
+__device__ __forceinline__ int tri_row(int i, int n)
 {
-    double M = 1.0;
-    C cc = {0, 0};
+    return i < n - 2 ? min(i, kTriRows - 4) : min(kTriRows - 3 + i - (n - 2), kTriRows - 1);
+}
+
+// One tridiagonal line held R rows per lane; u: the right-hand sides over bet
+// on entry, the solution on exit.  p(r), g(r): the factors of the lane's row
+// r.  Rows past the line's end lie behind row n - 1, whose g is 0: they reach
+// no row before them.
+template <int R, typename F>
+__device__ __forceinline__ Map line_forward(double (&u)[R], F p)
+{
+    Map m{1.0, 0.0};
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const double a = T.a[r * G + lane], rb = T.rbet[r * G + lane];
-        M = (-a * rb) * M;
-        cc = (u[r] - a * cc) * rb;
+        m.c = __builtin_fma(-p(r), m.c, u[r]);
+        m.m *= -p(r);
+        u[r] = m.c;
     }
-#pragma unroll
-    for (int d = 1; d < G; d <<= 1) {
-        const double Mo = __shfl_up(M, d, G);
-        const C co = shfl_up(cc, d, G);
-        if (lane >= d) {
-            cc = M * co + cc;
-            M = M * Mo;
-        }
-    }
-    C prev = shfl_up(cc, 1, G);
-    if (lane == 0) prev = {0, 0};
+    return m;
+}
+template <int R, typename F>
+__device__ __forceinline__ void line_forward_in(double (&u)[R], F p, double in)
+{
+    double h = 1.0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const double a = T.a[r * G + lane], rb = T.rbet[r * G + lane];
-        const C v = (u[r] - a * prev) * rb;
-        u[r] = v;
-        prev = v;
+        h *= -p(r);
+        u[r] = __builtin_fma(h, in, u[r]);
     }
-    M = 1.0;
-    cc = {0, 0};
+}
+template <int R, typename F>
+__device__ __forceinline__ Map line_backward(double (&u)[R], F g)
+{
+    Map m{1.0, 0.0};
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {
-        const double g = T.gam1[r * G + lane];
-        M = -g * M;
-        cc = u[r] - g * cc;
+        m.c = __builtin_fma(-g(r), m.c, u[r]);
+        m.m *= -g(r);
+        u[r] = m.c;
     }
-#pragma unroll
-    for (int d = 1; d < G; d <<= 1) {
-        const double Mo = __shfl_down(M, d, G);
-        const C co = shfl_down(cc, d, G);
-        if (lane + d < G) {
-            cc = M * co + cc;
-            M = M * Mo;
-        }
-    }
-    C next = shfl_down(cc, 1, G);
-    if (lane == G - 1) next = {0, 0};
+    return m;
+}
+template <int R, typename F>
+__device__ __forceinline__ void line_backward_in(double (&u)[R], F g, double in)
+{
+    double h = 1.0;
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {
-        const double g = T.gam1[r * G + lane];
-        const C v = u[r] - g * next;
-        u[r] = v;
-        next = v;
+        h *= -g(r);
+        u[r] = __builtin_fma(h, in, u[r]);
     }
 }
 
-// Right-hand sides of the x schemes (rhsx, derivs_par.f:259-302; rhsxx,
-// 351-397) on a line f of n points, in the reference's sums; the divisions
-// by 12 dx, 120 dx, ... are multiplications by their reciprocals.  The four
-// closure points (1-based 1, 2, n-1, n) are the same for every lane of the
-// line and are formed once per lane as wavefront-uniform values; interior
-// points take the centred stencil.
-struct XRhs {
-    C p1, p2, pn1, pn;   // closure points 1, 2, n-1, n
+// The two closure right-hand sides at a lane's end of the line (the start for
+// lanes of the first half, else the end): e the outermost point, s the next,
+// NE and NE + 1 terms in the reference's order over the values F[0], F[1], ...
+// from that end inwards; w: their weights, the scale last (8 each)
+struct Closure {
+    double e, s;
 };
-__device__ __forceinline__ XRhs rhs_x_closures(const C *f, int n, double dx, double dxx,
-                                               bool second)
+template <int NE>
+__device__ __forceinline__ Closure closure(const double *w, const double (&F)[7])
 {
-#define F(I) f[(I) - 1]
-    XRhs b;
-    if (!second) {
-        b.p1 = (-25.0 * F(1) + 48.0 * F(2) - 36.0 * F(3) + 16.0 * F(4) - 3.0 * F(5)) *
-               (1.0 / (12.0 * dx));
-        b.p2 = (-406.0 * F(1) - 300.0 * F(2) + 760.0 * F(3) - 80.0 * F(4) + 30.0 * F(5)
-                - 4.0 * F(6)) * (1.0 / (120.0 * dx));
-        b.pn1 = (-406.0 * F(n) - 300.0 * F(n - 1) + 760.0 * F(n - 2) - 80.0 * F(n - 3)
-                 + 30.0 * F(n - 4) - 4.0 * F(n - 5)) * (1.0 / (-120.0 * dx));
-        b.pn = (-74.0 * F(n) + 16.0 * F(n - 1) + 72.0 * F(n - 2) - 16.0 * F(n - 3)
-                + 2.0 * F(n - 4)) * (1.0 / (-24.0 * dx));
-    } else {
-        b.p1 = (9775.0 * F(1) - 20285.0 * F(2) + 11170.0 * F(3) - 550.0 * F(4) - 145.0 * F(5)
-                + 35.0 * F(6)) * (1.0 / (60.0 * dxx));
-        b.p2 = (4834.0 * F(1) - 8424.0 * F(2) + 1890.0 * F(3) + 2320.0 * F(4) - 810.0 * F(5)
-                + 216.0 * F(6) - 26.0 * F(7)) * (1.0 / (360.0 * dxx));
-        b.pn1 = (4834.0 * F(n) - 8424.0 * F(n - 1) + 1890.0 * F(n - 2) + 2320.0 * F(n - 3)
-                 - 810.0 * F(n - 4) + 216.0 * F(n - 5) - 26.0 * F(n - 6)) * (1.0 / (360.0 * dxx));
-        b.pn = (9775.0 * F(n) - 20285.0 * F(n - 1) + 11170.0 * F(n - 2) - 550.0 * F(n - 3)
-                - 145.0 * F(n - 4) + 35.0 * F(n - 5)) * (1.0 / (60.0 * dxx));
-    }
-#undef F
-    return b;
+    double e = w[0] * F[0], s = w[8] * F[0];
+#pragma unroll
+    for (int q = 1; q < NE; ++q) e = e + w[q] * F[q];
+#pragma unroll
+    for (int q = 1; q <= NE; ++q) s = s + w[8 + q] * F[q];
+    return {e * w[7], s * w[15]};
 }
-// interior point i (0-based, 2 <= i <= n-3) from f[i-2 .. i+2]
-__device__ __forceinline__ C rhs_x_centre(C m2, C m1, C c0, C p1, C p2, double s, bool second)
-{
-    if (!second) return (p2 - m2 + 28.0 * (p1 - m1)) * s;
-    return (3.0 * (p2 + m2) + 48.0 * (p1 + m1) - 102.0 * c0) * s;
-}
-
-// x-lines: o1 = d/dx, o2 = d2/dx2 of f (either may be null).  LDS: the
-// input lines of the workgroup's kDerivXLines wavefronts, ldx complex each,
-// then one output chunk of ch points (a multiple of 64) per wavefront.  A
-// solved line goes from the lanes' segments back to coalesced rows through
-// LDS: the last derivative of the call through its own input line (no
-// longer read once its right-hand side is formed), in one pass; the first
-// of two through the chunk buffer, ch points a pass.  The launch sizes ch
-// so that a workgroup stays within kDerivXWgLds, two workgroups a CU (two
-// wavefronts per SIMD, the occupancy the kernel's registers allow).
-constexpr int kDerivXLines = 4;
-constexpr int kDerivXWgLds = 80 * 1024;
-
+// the lane's closure points of u: rows 0, 1 or n - 1, n - 2
 template <int R>
-__global__ void __launch_bounds__(64 * kDerivXLines) deriv_x_kernel(DerivArgs A, int ldx, int ch,
-                                                                    const C *__restrict__ f,
-                                                                    C *o1, C *o2)
+__device__ __forceinline__ void put_closure(double (&u)[R], const Closure &b, int i0, int n)
 {
-    extern __shared__ C xline[];
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-    const int lane = threadIdx.x & 63;
-    const int nx = A.nx;
-    const size_t line = static_cast<size_t>(blockIdx.x) * kDerivXLines + w;
-    if (line >= static_cast<size_t>(A.ny) * A.K) return;   // whole wavefront
-    C *Ls = xline + static_cast<size_t>(w) * ldx;
-    const C *fl = f + line * nx;
-    {
-        // every load issued before the first is waited for (indices clamped
-        // into the line; a load under a lane mask would wait per point)
-        C v[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = fl[min(lane + 64 * r, nx - 1)];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (lane + 64 * r < nx) Ls[lane + 64 * r] = v[r];
+    if (i0 == 0) {
+        u[0] = b.e;
+        u[1] = b.s;
     }
-    lds_wave_sync();
-    const int i0 = lane * R;
-    C *Os = xline + static_cast<size_t>(kDerivXLines) * ldx + w * ch;   // output chunk
-#pragma unroll 1
-    for (int second = 0; second < 2; ++second) {
-        C *o = second ? o2 : o1;
-        if (!o) continue;
-        const XRhs b = rhs_x_closures(Ls, nx, A.dx, A.dxx, second);
-        const double s = second ? 1.0 / (4.0 * A.dxx) : 1.0 / (12.0 * A.dx);
-        // the lane's points and two more each side (clamped into the line)
-        C wv[R + 4];
+    const int re = (n - 1) % R, rs = (n - 2) % R;     // uniform
 #pragma unroll
-        for (int q = 0; q < R + 4; ++q) wv[q] = Ls[min(max(i0 + q - 2, 0), nx - 1)];
-        C u[R];
+    for (int r = 0; r < R; ++r) {
+        if (r == rs) u[r] = i0 + r == n - 2 ? b.s : u[r];
+        if (r == re) u[r] = i0 + r == n - 1 ? b.e : u[r];
+    }
+}
+// F and the weights' side for a lane whose first row is i0
+__device__ __forceinline__ int closure_points(const double *P, int i0, int n, double (&F)[7])
+{
+    const bool end = i0 >= n / 2;
+#pragma unroll
+    for (int q = 0; q < 7; ++q) F[q] = P[end ? n - 1 - q : q];
+    return end ? 16 : 0;
+}
+
+// Global rows go through buffer resources over the line (x) or the mode (y):
+// an access past the range reads zero or is dropped, so no access needs a
+// branch.  A plane holds two values each side of its rows, zero where nothing
+// was read, so the stencil windows need no clamp.
+// (The whole offset is in the vector operand: the range check does not cover
+// a scalar offset past the range.)
+template <bool NT>
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, unsigned off, C v)
+{
+    u32x4 x;
+    __builtin_memcpy(&x, &v, sizeof(x));
+    __builtin_amdgcn_raw_buffer_store_b128(x, r, off, 0, NT ? 2 : 0);
+}
+// a workgroup's tables: `n` doubles, loads issued here, into LDS by the result
+template <int NT, int M>
+struct TableCopy {
+    double v[M];
+    int n;
+    __device__ __forceinline__ TableCopy(const double *src, int count, int t) : n(count)
+    {
+#pragma unroll
+        for (int q = 0; q < M; ++q) v[q] = src[min(t + NT * q, n - 1)];
+    }
+    __device__ __forceinline__ void store(double *dst, int t) const
+    {
+#pragma unroll
+        for (int q = 0; q < M; ++q)
+            if (t + NT * q < n) dst[t + NT * q] = v[q];
+    }
+};
+
+// x-lines: o1 = d/dx (D1), o2 = d2/dx2 (D2) of f.  Workgroup: one line, W
+// wavefronts per part; LDS: the two planes (LP values each; their reads at a
+// lane stride of R, odd but for the shortest lines, are conflict-free), the
+// wavefronts' maps, the tables.  Interior points: rhsx, rhsxx in the
+// reference's sums, over 12 dx or 4 dx^2 and the pivot in one multiplication.
+// The stores stream (nt): whole cache lines that the launch does not read
+// again (1025x193x64, both derivatives: 130 -> 116 us).
+// From 3 wavefronts per part the registers are held to 4 wavefronts a SIMD: two
+// workgroups a CU (2049x257x32: 276 -> 198 us; below that it only spilled).
+template <int R, int W, bool D1, bool D2>
+__global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
+    deriv_x_kernel(DerivArgs A, const C *__restrict__ f, C *__restrict__ o1, C *__restrict__ o2)
+{
+    constexpr int NT = 128 * W, N = (R + 1) / 2, LP = 64 * R * W + 4;
+    __shared__ double planes[2 * LP], maps[16 * W], tab[kXTab];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int part = wv / W, w = wv % W;
+    const int nx = A.nx;
+    const size_t line = static_cast<size_t>(blockIdx.x) * nx;
+    {
+        const __amdgpu_buffer_rsrc_t fr = buf_rsrc(f + line, static_cast<size_t>(nx) * sizeof(C));
+        C v[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) v[q] = buf_load(fr, (t + NT * q) * sizeof(C), 0.0);
+        const TableCopy<NT, (kXTab + NT - 1) / NT> tc(A.xtab, kXTab, t);
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+            if ((q + 1) * NT <= 64 * R * W || wv < W) {
+                planes[2 + t + NT * q] = v[q].re;
+                planes[LP + 2 + t + NT * q] = v[q].im;
+            }
+        if (t < 8) planes[t / 4 * LP + (t % 4 < 2 ? t % 4 : LP - 4 + t % 4)] = 0.0;
+        tc.store(tab, t);
+    }
+    __syncthreads();
+    double *P = planes + part * LP + 2, *tot = maps + part * 8 * W;
+    const int i0 = (w * 64 + lane) * R;
+    const double *ta = tab, *tb = tab + 3 * kTriRows, *tc = tab + 6 * kTriRows;
+    double a[R], b[R];
+    int row[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) row[r] = tri_row(i0 + r, nx);
+    {
+        double x[R + 4];
+#pragma unroll
+        for (int q = 0; q < R + 4; ++q) x[q] = P[i0 + q - 2];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int i = i0 + r;
-            C v = rhs_x_centre(wv[r], wv[r + 1], wv[r + 2], wv[r + 3], wv[r + 4], s, second);
-            v = sel(i == 0, b.p1, v);
-            v = sel(i == 1, b.p2, v);
-            v = sel(i == nx - 2, b.pn1, v);
-            v = sel(i == nx - 1, b.pn, v);
-            u[r] = sel(i < nx, v, C{0, 0});
+            if constexpr (D1) a[r] = (x[r + 4] - x[r] + 28.0 * (x[r + 3] - x[r + 1])) * ta[row[r]];
+            if constexpr (D2)
+                b[r] = (3.0 * (x[r + 4] + x[r]) + 48.0 * (x[r + 3] + x[r + 1]) - 102.0 * x[r + 2]) *
+                       tb[row[r]];
         }
-        thomas_scan<64, R>(thomas_seg(A, second), lane, u);
-        C *ol = o + line * nx;
-        if (second || !o2) {
-            // the call's last derivative: out through the input line
-            lds_wave_sync();
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (i0 + r < nx) Ls[i0 + r] = u[r];
-            lds_wave_sync();
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (lane + 64 * r < nx) ol[lane + 64 * r] = Ls[lane + 64 * r];
-            break;
-        }
-        // the lane's points through the output chunk, out as coalesced stores
-#pragma unroll 1
-        for (int c0 = 0; c0 < nx; c0 += ch) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int e = i0 + r - c0;
-                if (e >= 0 && e < ch && i0 + r < nx) Os[e] = u[r];
-            }
-            lds_wave_sync();
-#pragma unroll 1
-            for (int e = lane; e < ch; e += 64)
-                if (c0 + e < nx) ol[c0 + e] = Os[e];
-            lds_wave_sync();
+        // the wavefronts that hold the line's first or last two points
+        if (w == 0 || (w + 1) * 64 * R > nx - 2) {
+            double F[7];
+            const int side = closure_points(P, i0, nx, F);
+            if constexpr (D1) put_closure<R>(a, closure<5>(tc + side, F), i0, nx);
+            if constexpr (D2) put_closure<R>(b, closure<6>(tc + 32 + side, F), i0, nx);
         }
     }
+    // incoming state of a lane: its wavefront's (0, or through the maps of the
+    // wavefronts before it) sent through the lanes before it
+    auto solve_dir = [&](bool up) {
+        const int field = (up ? 1 : 2) * kTriRows;
+        double pa[R], pb[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (D1) pa[r] = ta[field + row[r]];
+            if constexpr (D2) pb[r] = tb[field + row[r]];
+        }
+        auto fa = [&](int r) { return pa[r]; };
+        auto fb = [&](int r) { return pb[r]; };
+        Map ma{1.0, 0.0}, mb{1.0, 0.0};
+        if constexpr (D1) ma = up ? line_forward<R>(a, fa) : line_backward<R>(a, fa);
+        if constexpr (D2) mb = up ? line_forward<R>(b, fb) : line_backward<R>(b, fb);
+        if constexpr (D1) ma = up ? scan_maps_up<64>(ma, lane) : scan_maps_down<64>(ma, lane);
+        if constexpr (D2) mb = up ? scan_maps_up<64>(mb, lane) : scan_maps_down<64>(mb, lane);
+        double sa = 0.0, sb = 0.0;
+        if constexpr (W > 1) {
+            double *tt = tot + (up ? 0 : 4 * W);
+            if (lane == (up ? 63 : 0)) {
+                tt[4 * w] = ma.m;
+                tt[4 * w + 1] = ma.c;
+                tt[4 * w + 2] = mb.m;
+                tt[4 * w + 3] = mb.c;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < W - 1; ++q) {
+                const int s = up ? q : W - 1 - q;
+                if (up ? s < w : s > w) {
+                    if constexpr (D1) sa = __builtin_fma(tt[4 * s], sa, tt[4 * s + 1]);
+                    if constexpr (D2) sb = __builtin_fma(tt[4 * s + 2], sb, tt[4 * s + 3]);
+                }
+            }
+        }
+        const bool first = lane == (up ? 0 : 63);
+        if constexpr (D1) {
+            const Map e = up ? dpp_map<0x138>(ma) : dpp_map<0x130>(ma);
+            const double in = first ? sa : __builtin_fma(e.m, sa, e.c);
+            up ? line_forward_in<R>(a, fa, in) : line_backward_in<R>(a, fa, in);
+        }
+        if constexpr (D2) {
+            const Map e = up ? dpp_map<0x138>(mb) : dpp_map<0x130>(mb);
+            const double in = first ? sb : __builtin_fma(e.m, sb, e.c);
+            up ? line_forward_in<R>(b, fb, in) : line_backward_in<R>(b, fb, in);
+        }
+    };
+    solve_dir(true);
+    solve_dir(false);
+    // out through the planes (a plane's readers are its own part's wavefronts:
+    // past the maps' barriers, or this wavefront itself)
+    auto out = [&](const double (&u)[R], C *o) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) P[i0 + r] = u[r];
+        __syncthreads();
+        const __amdgpu_buffer_rsrc_t ro = buf_rsrc(o + line, static_cast<size_t>(nx) * sizeof(C));
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+            if ((q + 1) * NT <= 64 * R * W || wv < W)
+                buf_store<true>(ro, (t + NT * q) * sizeof(C),
+                                C{planes[2 + t + NT * q], planes[LP + 2 + t + NT * q]});
+    };
+    if constexpr (D1) out(a, o1);
+    if constexpr (D1 && D2) __syncthreads();
+    if constexpr (D2) out(b, o2);
 }
 
-// Right-hand sides of the y schemes (rhsy 400-449, rhsyfv 504-549 with the
-// wall row 0, rhsyy 552-611) on a column f of n rows: the four closure rows
-// per column (wavefront-uniform for the column's lanes) and the centred rows
-// j (0-based, 2 <= j <= n-3), with the metric of the spacing the generator
-// normalised to (v_qdy(j-2), v_qdy2(j-2, 1); 1-based j in the reference).
-__device__ __forceinline__ XRhs rhs_y1_closures(const DerivArgs &A, const C *f, int n, bool fv)
+// y-lines: o1 = d/dy (fv: with the wall row forced, deryfv), o2 = d2/dy2 of f.
+// Workgroup: 8 columns x all rows of one mode, both parts, in LDS (column
+// stride LP, 4 past a multiple of 32 values: the 8 columns x 4 rows of half a
+// wavefront's tile accesses fall on different banks); G lanes per column and
+// part.  Interior rows: rhsy, rhsyy in the reference's sums, times the metric
+// of the spacing the generator normalised to (v_qdy(j-2), v_qdy2(j-2, 1);
+// 1-based j) over the pivot; every row has its own table entry, at a constant
+// offset from the lane's first.  The stores do not stream: a row's 128 bytes
+// are rarely one cache line (with nt 8 of 9 sizes were up to 50 % slower).
+constexpr int kDerivYCols = 8;
+template <int G, int R, bool D1, bool D2>
+__global__ void __launch_bounds__(16 * G) deriv_y_kernel(DerivArgs A, const C *__restrict__ f,
+                                                         C *__restrict__ o1, int fv,
+                                                         C *__restrict__ o2)
 {
-    const double *qdy = A.qdy;
-    const double *sp = A.sp_fd, *pp = A.pp_fd, *lp = A.lp_fd, *fe = A.fp_e;
-#define FY(J) f[(J) - 1]
-    XRhs b;
-    b.p1 = fv ? C{0, 0}
-              : qdy[0] * (fe[1] * FY(1) + fe[2] * FY(2) + fe[3] * FY(3) + fe[4] * FY(4)
-                          + fe[5] * FY(5));
-    b.p2 = qdy[0] * (sp[3] * FY(1) + sp[4] * FY(2) + sp[5] * FY(3) + sp[6] * FY(4)
-                     + sp[7] * FY(5) + sp[8] * FY(6));
-    b.pn1 = qdy[n - 6] * (pp[3] * FY(n) + pp[4] * FY(n - 1) + pp[5] * FY(n - 2)
-                          + pp[6] * FY(n - 3) + pp[7] * FY(n - 4) + pp[8] * FY(n - 5));
-    b.pn = qdy[n - 5] * (lp[2] * FY(n) + lp[3] * FY(n - 1) + lp[4] * FY(n - 2)
-                         + lp[5] * FY(n - 3) + lp[6] * FY(n - 4));
-    return b;
-}
-__device__ __forceinline__ XRhs rhs_y2_closures(const DerivArgs &A, const C *f, int n)
-{
-    const double *qdy2 = A.qdy2;
-    const double *fp = A.fp_sd, *sp = A.sp_sd, *pp = A.pp_sd, *lp = A.lp_sd;
-    XRhs b;
-    b.p1 = (fp[2] * FY(1) + fp[3] * FY(2) + fp[4] * FY(3) + fp[5] * FY(4) + fp[6] * FY(5)
-            + fp[7] * FY(6)) * qdy2[0];
-    b.p2 = (sp[3] * FY(1) + sp[4] * FY(2) + sp[5] * FY(3) + sp[6] * FY(4) + sp[7] * FY(5)
-            + sp[8] * FY(6) + sp[9] * FY(7)) * qdy2[0];
-    b.pn1 = (pp[3] * FY(n) + pp[4] * FY(n - 1) + pp[5] * FY(n - 2) + pp[6] * FY(n - 3)
-             + pp[7] * FY(n - 4) + pp[8] * FY(n - 5) + pp[9] * FY(n - 6)) * qdy2[n - 7];
-    b.pn = (lp[2] * FY(n) + lp[3] * FY(n - 1) + lp[4] * FY(n - 2) + lp[5] * FY(n - 3)
-            + lp[6] * FY(n - 4) + lp[7] * FY(n - 5)) * qdy2[n - 6];
-#undef FY
-    return b;
-}
-
-// y-lines: o1 = d/dy (fv: with the wall row forced, deryfv), o2 = d2/dy2 of
-// f (either may be null).  Workgroup: TX = 256/G columns x all rows of one
-// mode in LDS, column-major with stride ldy (odd, against bank conflicts).
-template <int G, int R>
-__global__ void __launch_bounds__(256) deriv_y_kernel(DerivArgs A, int ldy, const C *__restrict__ f,
-                                                      C *o1, int fv, C *o2)
-{
-    constexpr int TX = 256 / G;
-    extern __shared__ C ytile[];
-    const int nx = A.nx, ny = A.ny;
+    constexpr int TX = kDerivYCols, NT = 2 * TX * G, N = (R + 1) / 2, M = G * R, LP = M + 4;
+    constexpr int NTAB = 6 * M + 64;
+    extern __shared__ double ylds[];
+    double *planes = ylds, *tab = ylds + 2 * TX * LP;
+    const int nx = A.nx, ny = A.ny, t = threadIdx.x;
     // workgroup n takes tile (n mod 8) * ceil(B/8) + n / 8 of the B tiles
     // (x fastest, then mode): the hardware deals workgroups to the 8 XCDs
     // round-robin, so neighbouring tiles -- whose rows share the cache line
@@ -304,214 +377,95 @@ __global__ void __launch_bounds__(256) deriv_y_kernel(DerivArgs A, int ldy, cons
     const int m = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
     if (m >= B) return;
     const int x0 = (m % tiles_x) * TX, k = m / tiles_x;
-    const size_t mb = static_cast<size_t>(k) * nx * ny;
-    // tile load: TX consecutive x of each row (one contiguous run per row);
-    // TX * ny <= 256 R, so R steps of the workgroup cover the tile, and all
-    // of a thread's loads are issued before the first is waited for
+    const size_t plane = static_cast<size_t>(nx) * ny, mb = plane * k;
+    // thread: column x0 + t % 8, rows t / 8 + 2 G q
+    const int tx = t % TX, tj = t / TX;
+    const unsigned off = x0 + tx < nx ? static_cast<unsigned>((tj * nx + x0 + tx) * sizeof(C)) : kBufOff;
+    const unsigned step = 2 * G * nx * static_cast<unsigned>(sizeof(C));
+    double *re = planes + tx * LP + 2 + tj, *im = re + TX * LP;
     {
-        C v[R];
+        const __amdgpu_buffer_rsrc_t fr = buf_rsrc(f + mb, plane * sizeof(C));
+        C v[N];
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int e = min(static_cast<int>(threadIdx.x) + 256 * q, TX * ny - 1);
-            const int x = e % TX, j = e / TX;
-            const int xi = x0 + x < nx ? x0 + x : nx - 1;
-            v[q] = f[mb + static_cast<size_t>(j) * nx + xi];
-        }
+        for (int q = 0; q < N; ++q) v[q] = buf_load(fr, off + step * q, 0.0);
+        const TableCopy<NT, (NTAB + NT - 1) / NT> tc(A.ytab + (fv ? NTAB : 0), NTAB, t);
 #pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int e = static_cast<int>(threadIdx.x) + 256 * q;
-            if (e < TX * ny) {
-                const int x = e % TX, j = e / TX;
-                ytile[x * ldy + j] = x0 + x < nx ? v[q] : C{0, 0};
+        for (int q = 0; q < N; ++q)
+            if ((q + 1) * 2 * G <= M || tj + 2 * G * q < M) {
+                re[2 * G * q] = v[q].re;
+                im[2 * G * q] = v[q].im;
             }
-        }
+        if (t < 64) planes[t / 4 * LP + (t % 4 < 2 ? t % 4 : M + t % 4)] = 0.0;
+        tc.store(tab, t);
     }
     __syncthreads();
-    const int col = threadIdx.x / G, lane = threadIdx.x % G;
-    const C *Tc = ytile + col * ldy;
+    const int lane = t % G, col = t / G;       // col: column, then part
     const int j0 = lane * R;
-    // the lane's rows and two more each side (clamped into the column)
-    C wv[R + 4];
+    double *P = planes + col * LP + 2;
+    const double *ta = tab + j0, *tb = ta + 3 * M, *tc = tab + 6 * M;
+    double a[R], b[R];
+    {
+        double x[R + 4];
 #pragma unroll
-    for (int q = 0; q < R + 4; ++q) wv[q] = Tc[min(max(j0 + q - 2, 0), ny - 1)];
-    const double *cp1 = A.cp_fd, *cp2 = A.cp_sd;
-    C u1[R], u2[R];
-    if (o1) {
-        const XRhs b = rhs_y1_closures(A, Tc, ny, fv != 0);
+        for (int q = 0; q < R + 4; ++q) x[q] = P[j0 + q - 2];
+        const double *c1 = A.cp_fd, *c2 = A.cp_sd;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int j = j0 + r;
-            const double q = A.qdy[min(max(j - 2, 0), ny - 1)];
-            C v = q * (cp1[3] * wv[r] + cp1[4] * wv[r + 1] + cp1[5] * wv[r + 2]
-                       + cp1[6] * wv[r + 3] + cp1[7] * wv[r + 4]);
-            v = sel(j == 0, b.p1, v);
-            v = sel(j == 1, b.p2, v);
-            v = sel(j == ny - 2, b.pn1, v);
-            v = sel(j == ny - 1, b.pn, v);
-            u1[r] = sel(j < ny, v, C{0, 0});
+            if constexpr (D1)
+                a[r] = (c1[3] * x[r] + c1[4] * x[r + 1] + c1[5] * x[r + 2] + c1[6] * x[r + 3]
+                        + c1[7] * x[r + 4]) * ta[r];
+            if constexpr (D2)
+                b[r] = (c2[3] * x[r] + c2[4] * x[r + 1] + c2[5] * x[r + 2] + c2[6] * x[r + 3]
+                        + c2[7] * x[r + 4]) * tb[r];
         }
+        double F[7];
+        const int side = closure_points(P, j0, ny, F);
+        if constexpr (D1) {
+            Closure c = closure<5>(tc + side, F);
+            if (fv && side == 0) c.e = 0.0;
+            put_closure<R>(a, c, j0, ny);
+        }
+        if constexpr (D2) put_closure<R>(b, closure<6>(tc + 32 + side, F), j0, ny);
     }
-    if (o2) {
-        const XRhs b = rhs_y2_closures(A, Tc, ny);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int j = j0 + r;
-            const double q = A.qdy2[min(max(j - 2, 0), ny - 1)];
-            C v = (cp2[3] * wv[r] + cp2[4] * wv[r + 1] + cp2[5] * wv[r + 2] + cp2[6] * wv[r + 3]
-                   + cp2[7] * wv[r + 4]) * q;
-            v = sel(j == 0, b.p1, v);
-            v = sel(j == 1, b.p2, v);
-            v = sel(j == ny - 2, b.pn1, v);
-            v = sel(j == ny - 1, b.pn, v);
-            u2[r] = sel(j < ny, v, C{0, 0});
-        }
+    auto pa = [&](int r) { return ta[M + r]; };
+    auto pb = [&](int r) { return tb[M + r]; };
+    auto ga = [&](int r) { return ta[2 * M + r]; };
+    auto gb = [&](int r) { return tb[2 * M + r]; };
+    if constexpr (D1) {
+        const Map e = dpp_map<0x138>(scan_maps_up<G>(line_forward<R>(a, pa), lane));
+        line_forward_in<R>(a, pa, lane == 0 ? 0.0 : e.c);
     }
-    __syncthreads();   // the tile is rewritten with the results below
-    // solve, results through the tile, coalesced rows out
-    auto finish = [&](C(&u)[R], const Thomas &T, C *o) {
-        thomas_scan<G, R>(T, lane, u);
-        C *Tw = ytile + col * ldy;
+    if constexpr (D2) {
+        const Map e = dpp_map<0x138>(scan_maps_up<G>(line_forward<R>(b, pb), lane));
+        line_forward_in<R>(b, pb, lane == 0 ? 0.0 : e.c);
+    }
+    if constexpr (D1) {
+        const Map e = dpp_map<0x130>(scan_maps_down<G>(line_backward<R>(a, ga), lane));
+        line_backward_in<R>(a, ga, lane == G - 1 ? 0.0 : e.c);
+    }
+    if constexpr (D2) {
+        const Map e = dpp_map<0x130>(scan_maps_down<G>(line_backward<R>(b, gb), lane));
+        line_backward_in<R>(b, gb, lane == G - 1 ? 0.0 : e.c);
+    }
+    // out through the tile (a column's group of lanes lies in one wavefront
+    // and is its only reader until the barrier)
+    auto out = [&](const double (&u)[R], C *o) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int j = lane * R + r;
-            if (j < ny) Tw[j] = u[r];
-        }
+        for (int r = 0; r < R; ++r) P[j0 + r] = u[r];
         __syncthreads();
-        for (int e = threadIdx.x; e < TX * ny; e += 256) {
-            const int x = e % TX, j = e / TX;
-            if (x0 + x < nx) o[mb + static_cast<size_t>(j) * nx + x0 + x] = ytile[x * ldy + j];
-        }
-        __syncthreads();
+        const __amdgpu_buffer_rsrc_t ro = buf_rsrc(o + mb, plane * sizeof(C));
+#pragma unroll
+        for (int q = 0; q < N; ++q)
+            if ((q + 1) * 2 * G <= M || tj + 2 * G * q < M)
+                buf_store<false>(ro, off + step * q, C{re[2 * G * q], im[2 * G * q]});
     };
-    if (o1) finish(u1, thomas_seg(A, fv ? 4 : 2), o1);
-    if (o2) finish(u2, thomas_seg(A, 3), o2);
+    if constexpr (D1) out(a, o1);
+    if constexpr (D1 && D2) __syncthreads();
+    if constexpr (D2) out(b, o2);
 }
 
-// ---------------------------------------------------------------------------
-// Long lines: x-lines of more than 64 * 17 points and y-lines of more than
-// 64 * 9 rows take these kernels (no LDS stage; the LDS-staged forms would
-// need more than 256 registers per lane there).  x: one wavefront per line,
-// lane t owns points [t*R, t*R+R) read from global memory, divisions as in
-// tridparx; y: one thread per column, the forward sweep stored in the output
-// and re-read by the backward sweep (tridy's order).
-// ---------------------------------------------------------------------------
-// d/dx right-hand side (rhsx, derivs_par.f:259-302) and d2/dx2 (rhsxx, 351-397)
-__device__ __forceinline__ C rhs_x_point(const C *__restrict__ f, int i, int n, double dx, double dxx,
-                                   bool second)
-{
-#define F(I) f[(I) - 1]
-    const int I = i + 1;   // 1-based
-    if (!second) {
-        if (I == 1)
-            return (-25.0 * F(1) + 48.0 * F(2) - 36.0 * F(3) + 16.0 * F(4) - 3.0 * F(5)) / (12.0 * dx);
-        if (I == 2)
-            return (-406.0 * F(1) - 300.0 * F(2) + 760.0 * F(3) - 80.0 * F(4) + 30.0 * F(5)
-                    - 4.0 * F(6)) / (120.0 * dx);
-        if (I == n - 1)
-            return (-406.0 * F(n) - 300.0 * F(n - 1) + 760.0 * F(n - 2) - 80.0 * F(n - 3)
-                    + 30.0 * F(n - 4) - 4.0 * F(n - 5)) / (-120.0 * dx);
-        if (I == n)
-            return (-74.0 * F(n) + 16.0 * F(n - 1) + 72.0 * F(n - 2) - 16.0 * F(n - 3)
-                    + 2.0 * F(n - 4)) / (-24.0 * dx);
-        return (F(I + 2) - F(I - 2) + 28.0 * (F(I + 1) - F(I - 1))) / (12.0 * dx);
-    }
-    if (I == 1)
-        return (9775.0 * F(1) - 20285.0 * F(2) + 11170.0 * F(3) - 550.0 * F(4) - 145.0 * F(5)
-                + 35.0 * F(6)) / (60.0 * dxx);
-    if (I == 2)
-        return (4834.0 * F(1) - 8424.0 * F(2) + 1890.0 * F(3) + 2320.0 * F(4) - 810.0 * F(5)
-                + 216.0 * F(6) - 26.0 * F(7)) / (360.0 * dxx);
-    if (I == n - 1)
-        return (4834.0 * F(n) - 8424.0 * F(n - 1) + 1890.0 * F(n - 2) + 2320.0 * F(n - 3)
-                - 810.0 * F(n - 4) + 216.0 * F(n - 5) - 26.0 * F(n - 6)) / (360.0 * dxx);
-    if (I == n)
-        return (9775.0 * F(n) - 20285.0 * F(n - 1) + 11170.0 * F(n - 2) - 550.0 * F(n - 3)
-                - 145.0 * F(n - 4) + 35.0 * F(n - 5)) / (60.0 * dxx);
-    return (3.0 * (F(I + 2) + F(I - 2)) + 48.0 * (F(I + 1) + F(I - 1)) - 102.0 * F(I)) / (4.0 * dxx);
-#undef F
-}
-
-template <int R>
-__global__ void __launch_bounds__(256) deriv_x_line_kernel(DerivArgs A, int second, const C *f, C *out)
-{
-    const int lane = threadIdx.x & 63;
-    const size_t line = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (line >= static_cast<size_t>(A.ny) * A.K) return;
-    const int n = A.nx;
-    const C *fl = f + line * n;
-    C *ol = out + line * n;
-    const double *ta = A.thomas + static_cast<size_t>(second) * kThomasFields * A.nmax;
-    const double *tb = ta + A.nmax, *tg = tb + A.nmax;
-    const int i0 = lane * R;
-    C u[R];
-    // forward sweep u_i = (r_i - a_i u_{i-1}) / bet_i as an affine map of u_{i0-1}
-    double M = 1.0;
-    C cc = {0, 0};
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int i = i0 + r;
-        C rr = {0, 0};
-        double a = 0.0, bet = 1.0;
-        if (i < n) {
-            rr = rhs_x_point(fl, i, n, A.dx, A.dxx, second);
-            a = ta[i];
-            bet = tb[i];
-        }
-        u[r] = rr;
-        const double m = -a / bet;
-        M = m * M;
-        cc = (rr - a * cc) / bet;
-    }
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Mo = __shfl_up(M, d, 64);
-        const C co = shfl_up(cc, d, 64);
-        if (lane >= d) {
-            cc = M * co + cc;
-            M = M * Mo;
-        }
-    }
-    C prev = shfl_up(cc, 1, 64);
-    if (lane == 0) prev = {0, 0};
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int i = i0 + r;
-        const double a = (i < n) ? ta[i] : 0.0, bet = (i < n) ? tb[i] : 1.0;
-        const C v = (u[r] - a * prev) / bet;
-        u[r] = v;
-        prev = v;
-    }
-    // backward sweep x_i = u_i - gam_{i+1} x_{i+1}
-    M = 1.0;
-    cc = {0, 0};
-#pragma unroll
-    for (int r = R - 1; r >= 0; --r) {
-        const int i = i0 + r;
-        const double g = (i + 1 < n) ? tg[i + 1] : 0.0;
-        M = -g * M;
-        cc = u[r] - g * cc;
-    }
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double Mo = __shfl_down(M, d, 64);
-        const C co = shfl_down(cc, d, 64);
-        if (lane + d < 64) {
-            cc = M * co + cc;
-            M = M * Mo;
-        }
-    }
-    C next = shfl_down(cc, 1, 64);
-    if (lane == 63) next = {0, 0};
-#pragma unroll
-    for (int r = R - 1; r >= 0; --r) {
-        const int i = i0 + r;
-        const double g = (i + 1 < n) ? tg[i + 1] : 0.0;
-        const C v = u[r] - g * next;
-        next = v;
-        if (i < n) ol[i] = v;
-    }
-}
-
+// y-lines of more than 64 * 9 rows: one thread per column, the forward sweep
+// stored in the output and re-read by the backward sweep (tridy's order).
 // d/dy (rhsy 400-449), d2/dy2 (rhsyy 552-611), d/dy with wall row 0
 // (rhsyfv 504-549); kind 2, 3, 4
 __global__ void __launch_bounds__(64) deriv_y_line_kernel(DerivArgs A, int kind, const C *f, C *out)
@@ -587,86 +541,101 @@ __global__ void __launch_bounds__(64) deriv_y_line_kernel(DerivArgs A, int kind,
 }
 
 
-#define TBL_XR(X) X(1) X(2) X(3) X(5) X(7) X(9) X(17)
-#define TBL_YR(X) X(1) X(2) X(3) X(4) X(5) X(7) X(9)
+// x shapes (R, W): the fewest wavefronts per part with at most 9 points per
+// lane, then the fewest points (17 points per lane took the registers of the
+// wavefronts that hide the recurrences' latency)
+#define TBL_X_SHAPES(X) \
+    X(2, 1) X(3, 1) X(5, 1) X(7, 1) X(9, 1) X(5, 2) X(7, 2) X(9, 2) X(7, 3) X(9, 3) X(7, 4) X(9, 4)
+// y shapes (G, R): the first that holds the rows; R odd (an even lane stride
+// puts the lanes of a column on few banks: 97 rows as 32 x 4 took 252 us for
+// both derivatives of 1025x97x128, as 16 x 7 149)
+#define TBL_Y_SHAPES(X) \
+    X(16, 3) X(16, 5) X(16, 7) X(16, 9) X(32, 5) X(32, 7) X(32, 9) X(64, 5) X(64, 7) X(64, 9)
 
-
-// Lane shapes of the LDS-staged kernels: x: 64 lanes, R = xR rows (0: the
-// long-line kernel); y: yG lanes, yR rows (0: the long-line kernel)
-void deriv_shapes(int nx, int ny, int *xR, int *yG, int *yR)
+// longest x-line accepted (ptsx), below the 64 * 9 * 4 points the shapes hold
+constexpr int kDerivMaxNx = 2112;
+static bool x_shape(int nx, int *R, int *W)
 {
-    const int needx = (nx + 63) / 64;
-    *xR = 0;
-    for (int r : {1, 2, 3, 5, 7, 9, 17})
-        if (needx <= r) { *xR = r; break; }
-    *yG = (ny + 31) / 32 <= 9 ? 32 : 64;
-    const int needy = (ny + *yG - 1) / *yG;
-    *yR = 0;
-    if (ny <= 64 * 9)
-        for (int r : {1, 2, 3, 4, 5, 7, 9})
-            if (needy <= r) { *yR = r; break; }
-}
-
-// output chunk of deriv_x_kernel: the largest multiple of 64 points (at
-// least 64, at most the line rounded up) that keeps a workgroup's LDS within
-// kDerivXWgLds; lines up to 1088 points leave at least 128
-int deriv_x_chunk(int nx)
-{
-    const int ldx = nx | 1;
-    const int room = kDerivXWgLds / static_cast<int>(sizeof(C)) / kDerivXLines - ldx;
-    return std::max(64, std::min((nx + 63) / 64 * 64, room / 64 * 64));
+    bool found = false;
+    if (nx > kDerivMaxNx) return false;
+#define X(RR, WW)                                                                   \
+    if (64 * RR * WW >= nx && (!found || WW < *W || (WW == *W && RR < *R))) {       \
+        found = true;                                                               \
+        *R = RR;                                                                    \
+        *W = WW;                                                                    \
+    }
+    TBL_X_SHAPES(X)
+#undef X
+    return found;
 }
 
 static int deriv_x(const DerivArgs &A, const C *f, C *o1, C *o2, hipStream_t st)
 {
-    const int need = (A.nx + 63) / 64;
-    const size_t lines = static_cast<size_t>(A.ny) * A.K;
-    if (A.xR == 0) {
-        if (need > 33) return TBL_ERR_GRID;
-        const dim3 g4(static_cast<unsigned>((lines + 3) / 4));
-        if (o1) hipLaunchKernelGGL(deriv_x_line_kernel<33>, g4, dim3(256), 0, st, A, 0, f, o1);
-        if (o2) hipLaunchKernelGGL(deriv_x_line_kernel<33>, g4, dim3(256), 0, st, A, 1, f, o2);
-        return TBL_OK;
+    int R = 0, W = 0;
+    if (!x_shape(A.nx, &R, &W)) return TBL_ERR_GRID;
+    const dim3 grid(static_cast<unsigned>(A.ny) * static_cast<unsigned>(A.K));
+#define X(RR, WW)                                                                              \
+    if (R == RR && W == WW) {                                                                  \
+        const dim3 block(128 * WW);                                                            \
+        if (o1 && o2)                                                                          \
+            hipLaunchKernelGGL((deriv_x_kernel<RR, WW, true, true>), grid, block, 0, st, A,    \
+                               f, o1, o2);                                                     \
+        else if (o1)                                                                           \
+            hipLaunchKernelGGL((deriv_x_kernel<RR, WW, true, false>), grid, block, 0, st, A,   \
+                               f, o1, o2);                                                     \
+        else                                                                                   \
+            hipLaunchKernelGGL((deriv_x_kernel<RR, WW, false, true>), grid, block, 0, st, A,   \
+                               f, o1, o2);                                                     \
+        return TBL_OK;                                                                         \
     }
-    const dim3 grid(static_cast<unsigned>((lines + kDerivXLines - 1) / kDerivXLines));
-    const int ldx = A.nx | 1;
-    const int ch = deriv_x_chunk(A.nx);
-    const size_t lds = static_cast<size_t>(kDerivXLines) * (ldx + ch) * sizeof(C);
-#define X(RR)                                                                             \
-    if (A.xR == RR) {                                                                     \
-        hipLaunchKernelGGL(deriv_x_kernel<RR>, grid, dim3(64 * kDerivXLines), lds, st, A, \
-                           ldx, ch, f, o1, o2);                                           \
-        return TBL_OK;                                                                    \
-    }
-    TBL_XR(X)
+    TBL_X_SHAPES(X)
 #undef X
     return TBL_ERR_GRID;
 }
 
+// rows the y shape of ny holds (0: the one-thread-per-column kernel)
+int deriv_y_rows(int ny, int *G, int *R)
+{
+    *G = *R = 0;
+#define X(GG, RR)             \
+    if (!*R && GG * RR >= ny) { \
+        *G = GG;              \
+        *R = RR;              \
+    }
+    TBL_Y_SHAPES(X)
+#undef X
+    return *G * *R;
+}
+
 static int deriv_y(const DerivArgs &A, const C *f, C *o1, int fv, C *o2, hipStream_t st)
 {
-    const int ldy = A.ny | 1;
-    if (A.yR == 0) {
+    int G, R;
+    const int rows = deriv_y_rows(A.ny, &G, &R);
+    if (!R) {
         const dim3 g2((A.nx + 63) / 64, A.K);
         if (o1) hipLaunchKernelGGL(deriv_y_line_kernel, g2, dim3(64), 0, st, A, fv ? 4 : 2, f, o1);
         if (o2) hipLaunchKernelGGL(deriv_y_line_kernel, g2, dim3(64), 0, st, A, 3, f, o2);
         return TBL_OK;
     }
-    const int G = A.yG;
-    const int tiles = (A.nx + 256 / G - 1) / (256 / G) * A.K;
+    const int tiles = (A.nx + kDerivYCols - 1) / kDerivYCols * A.K;
     const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8));
-    const size_t lds = static_cast<size_t>(256 / G) * ldy * sizeof(C);
-#define X(RR)                                                                                \
-    if (A.yR == RR) {                                                                        \
-        if (G == 32)                                                                         \
-            hipLaunchKernelGGL((deriv_y_kernel<32, RR>), grid, dim3(256), lds, st, A, ldy, f, \
-                               o1, fv, o2);                                                   \
-        else                                                                                 \
-            hipLaunchKernelGGL((deriv_y_kernel<64, RR>), grid, dim3(256), lds, st, A, ldy, f, \
-                               o1, fv, o2);                                                   \
-        return TBL_OK;                                                                       \
+    const size_t lds =
+        (static_cast<size_t>(2 * kDerivYCols) * (rows + 4) + 6 * rows + 64) * sizeof(double);
+#define X(GG, RR)                                                                               \
+    if (G == GG && R == RR) {                                                                   \
+        const dim3 block(16 * GG);                                                              \
+        if (o1 && o2)                                                                           \
+            hipLaunchKernelGGL((deriv_y_kernel<GG, RR, true, true>), grid, block, lds, st, A,   \
+                               f, o1, fv, o2);                                                  \
+        else if (o1)                                                                            \
+            hipLaunchKernelGGL((deriv_y_kernel<GG, RR, true, false>), grid, block, lds, st, A,  \
+                               f, o1, fv, o2);                                                  \
+        else                                                                                    \
+            hipLaunchKernelGGL((deriv_y_kernel<GG, RR, false, true>), grid, block, lds, st, A,  \
+                               f, o1, fv, o2);                                                  \
+        return TBL_OK;                                                                          \
     }
-    TBL_YR(X)
+    TBL_Y_SHAPES(X)
 #undef X
     return TBL_ERR_GRID;
 }
@@ -700,23 +669,16 @@ int derivs4(const DerivArgs &A, const double *f, double *dx, double *dxx, double
 int deriv_kernel_attributes()
 {
     hipError_t e = hipSuccess;
-#define X(RR)                                                                                  \
-    {                                                                                          \
-        hipError_t r = hipFuncSetAttribute(reinterpret_cast<const void *>(&deriv_x_kernel<RR>), \
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,         \
-                                           160 * 1024);                                        \
-        if (r != hipSuccess) e = r;                                                            \
-    }
-    TBL_XR(X)
-#undef X
-#define X(RR)                                                                                  \
-    for (const void *fn : {reinterpret_cast<const void *>(&deriv_y_kernel<32, RR>),            \
-                           reinterpret_cast<const void *>(&deriv_y_kernel<64, RR>)}) {         \
-        hipError_t r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,     \
-                                           160 * 1024);                                        \
-        if (r != hipSuccess) e = r;                                                            \
-    }
-    TBL_YR(X)
+    auto allow = [&](const void *fn) {
+        const hipError_t r =
+            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (r != hipSuccess) e = r;
+    };
+#define X(GG, RR)                                                                  \
+    allow(reinterpret_cast<const void *>(&deriv_y_kernel<GG, RR, true, true>));    \
+    allow(reinterpret_cast<const void *>(&deriv_y_kernel<GG, RR, true, false>));   \
+    allow(reinterpret_cast<const void *>(&deriv_y_kernel<GG, RR, false, true>));
+    TBL_Y_SHAPES(X)
 #undef X
     return e == hipSuccess ? TBL_OK : TBL_ERR_HIP;
 }

@@ -429,6 +429,43 @@ void thomas_factors(const std::vector<double> &a, const std::vector<double> &b,
     }
 }
 
+// The right-hand sides of the first two and last two points of each scheme
+// (rhsx 259-302, rhsxx 351-397, rhsy 400-449, rhsyy 552-611).
+std::vector<double> deriv_closures(const tbl_grid &g, const tbl_coefs &c, const Metrics &m,
+                                   const double *rbet, size_t stride)
+{
+    std::vector<double> out(5 * 32, 0.0);
+    auto set = [&](int kind, int side, int next, const std::vector<double> &w, double scale) {
+        double *o = &out[kind * 32 + side * 16 + next * 8];
+        std::copy(w.begin(), w.end(), o);
+        const int n = kind <= 1 ? g.nx : g.ny;
+        o[7] = scale * rbet[kind * stride + (side ? n - 1 - next : next)];
+    };
+    const double dx = g.dx, dxx = g.dx * g.dx;
+    set(0, 0, 0, {-25, 48, -36, 16, -3}, 1.0 / (12.0 * dx));
+    set(0, 0, 1, {-406, -300, 760, -80, 30, -4}, 1.0 / (120.0 * dx));
+    set(0, 1, 0, {-74, 16, 72, -16, 2}, 1.0 / (-24.0 * dx));
+    set(0, 1, 1, {-406, -300, 760, -80, 30, -4}, 1.0 / (-120.0 * dx));
+    for (int side = 0; side < 2; ++side) {
+        set(1, side, 0, {9775, -20285, 11170, -550, -145, 35}, 1.0 / (60.0 * dxx));
+        set(1, side, 1, {4834, -8424, 1890, 2320, -810, 216, -26}, 1.0 / (360.0 * dxx));
+    }
+    const int n = g.ny;
+    auto fd = [](const double *w, int k) { return std::vector<double>(w, w + k); };
+    const double *q = m.qdy.data(), *q2 = m.qdy2.data();
+    for (int kind : {2, 4}) {
+        if (kind == 2) set(2, 0, 0, fd(c.fp_fd_e + 1, 5), q[0]);   // deryfv: a zero row
+        set(kind, 0, 1, fd(c.sp_fd + 3, 6), q[0]);
+        set(kind, 1, 0, fd(c.lp_fd + 2, 5), q[n - 5]);
+        set(kind, 1, 1, fd(c.pp_fd + 3, 6), q[n - 6]);
+    }
+    set(3, 0, 0, fd(c.fp_sd + 2, 6), q2[0]);
+    set(3, 0, 1, fd(c.sp_sd + 3, 7), q2[0]);
+    set(3, 1, 0, fd(c.lp_sd + 2, 6), q2[n - 6]);
+    set(3, 1, 1, fd(c.pp_sd + 3, 7), q2[n - 7]);
+    return out;
+}
+
 // coefx / coeffx (derivs_par.f:1145-1210), coefy / coefy_fv / coeffy
 // (derivs_par.f:1040-1142).  kind: 0 x first, 1 x second, 2 y first,
 // 3 y second, 4 y first with the wall row forced (deryfv).

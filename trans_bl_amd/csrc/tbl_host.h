@@ -35,4 +35,11 @@ int read_coefs_bin(const char *path, int levels, tbl_coefs *c, std::string *err)
 void deriv_lhs(const tbl_grid &g, const tbl_coefs &c, int kind, std::vector<double> &a,
                std::vector<double> &b, std::vector<double> &cc);
 
+// right-hand sides of the first and last two points of the derivative kinds
+// 0..4: [kind][start, end][outermost point, next][7 weights from that end
+// inwards, scale over the row's pivot]; rbet: 1/pivot per row, kinds `stride`
+// apart
+std::vector<double> deriv_closures(const tbl_grid &g, const tbl_coefs &c, const Metrics &m,
+                                   const double *rbet, size_t stride);
+
 }  // namespace tbl

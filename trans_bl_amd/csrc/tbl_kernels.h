@@ -174,15 +174,16 @@ struct DerivArgs {
     // Thomas factors per scheme: a, bet, gam, 1/bet (kind-major, stride nmax)
     const double *thomas;  // [kind][kThomasFields][nmax]
     int nmax;
-    // the same factors in lane-segment order for the LDS-staged kernels:
-    // x kinds 0, 1 ([kind][a, 1/bet, next gam][xR][64]), then y kinds 2, 3, 4
-    // ([kind][3][yR][yG]); xR / yR = 0: that direction takes the long-line
-    // kernel
-    const double *tseg;
-    int xR, yG, yR;
+    // tables of the LDS-staged kernels, per kind: interior scale/bet, a/bet, c/bet
+    // (gam of the next row), then the closures (deriv_closures).  xtab: kinds 0
+    // and 1, kTriRows entries a field (rows 0..63, converged beyond, the last
+    // two, a zero), closures.  ytab: kinds 2 and 3, then kinds 4 and 3, one entry
+    // per row of the y shape (deriv_y_rows; zero past ny), closures.
+    const double *xtab, *ytab;
 };
 constexpr int kThomasFields = 4;
-void deriv_shapes(int nx, int ny, int *xR, int *yG, int *yR);
+constexpr int kTriRows = 67, kXTab = 6 * kTriRows + 64;
+int deriv_y_rows(int ny, int *G, int *R);
 
 int deriv(const DerivArgs &A, int kind, const double *f, double *out, hipStream_t st);
 // d/dx, d2/dx2, d/dy, d2/dy2 of one field (any output may be null): two

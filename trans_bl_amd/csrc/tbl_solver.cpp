@@ -224,29 +224,44 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
             t[3 * nmax + j] = 1.0 / bet[j];
         }
     }
-    // lane-segment copies for the LDS-staged kernels
-    int xR = 0, yG = 0, yR = 0;
-    deriv_shapes(c->g.nx, c->g.ny, &xR, &yG, &yR);
-    std::vector<double> ts;
-    for (int kind = 0; kind < 5; ++kind) {
-        const bool x = kind <= 1;
-        const int G = x ? 64 : yG, R = x ? xR : yR, n = x ? c->g.nx : c->g.ny;
+    // the LDS-staged kernels' tables (DerivArgs)
+    int yG, yR;
+    const int yrows = deriv_y_rows(c->g.ny, &yG, &yR);
+    std::vector<double> dtab;
+    auto kind_table = [&](int kind, int rows, bool sparse) {
+        const int n = kind <= 1 ? c->g.nx : c->g.ny;
         const double *t = &th[static_cast<size_t>(kind) * kThomasFields * nmax];
-        const size_t base = ts.size(), per = static_cast<size_t>(G) * R;
-        ts.resize(base + 3 * per);
-        for (int r = 0; r < R; ++r)
-            for (int lane = 0; lane < G; ++lane) {
-                const int i = lane * R + r;
-                const size_t e = base + static_cast<size_t>(r) * G + lane;
-                ts[e] = i < n ? t[i] : 0.0;                            // a
-                ts[e + per] = i < n ? t[3 * nmax + i] : 1.0;           // 1/bet
-                ts[e + 2 * per] = i + 1 < n ? t[2 * nmax + i + 1] : 0.0;   // gam of row i+1
+        auto scale = [&](int j) {
+            return kind == 0   ? 1.0 / (12.0 * c->g.dx)
+                   : kind == 1 ? 1.0 / (4.0 * (c->g.dx * c->g.dx))
+                   : kind == 3 ? c->m.qdy2[std::max(j - 2, 0)]
+                               : c->m.qdy[std::max(j - 2, 0)];
+        };
+        for (int f = 0; f < 3; ++f)
+            for (int e = 0; e < rows; ++e) {
+                // sparse: rows 0.., then the last two and a zero; zero past n
+                const int j = sparse && e >= rows - 3 ? n - (rows - 1 - e) : e;
+                if (j >= n) {
+                    dtab.push_back(0.0);
+                    continue;
+                }
+                const double rb = t[3 * nmax + j];
+                dtab.push_back(f == 0 ? scale(j) * rb : f == 1 ? t[j] * rb
+                                        : j + 1 < n ? t[2 * nmax + j + 1] : 0.0);
             }
+    };
+    const std::vector<double> clos = deriv_closures(c->g, c->c, c->m, &th[3 * nmax],
+                                                    static_cast<size_t>(kThomasFields) * nmax);
+    auto closures = [&](int kind) {
+        dtab.insert(dtab.end(), clos.begin() + 32 * kind, clos.begin() + 32 * (kind + 1));
+    };
+    for (int first : {0, 2, 4}) {
+        const int second = first == 0 ? 1 : 3;
+        for (int kind : {first, second}) kind_table(kind, first == 0 ? kTriRows : yrows, first == 0);
+        for (int kind : {first, second}) closures(kind);
     }
-    if (!ts.empty()) {
-        TRY(dalloc(&c->d_tseg, ts.size()));
-        TBL_HIP(hipMemcpy(c->d_tseg, ts.data(), sizeof(double) * ts.size(), hipMemcpyHostToDevice));
-    }
+    TRY(dalloc(&c->d_dtab, dtab.size()));
+    TBL_HIP(hipMemcpy(c->d_dtab, dtab.data(), sizeof(double) * dtab.size(), hipMemcpyHostToDevice));
     TRY(dalloc(&c->d_thomas, th.size()));
     TBL_HIP(hipMemcpy(c->d_thomas, th.data(), sizeof(double) * th.size(), hipMemcpyHostToDevice));
     TRY(dalloc(&c->d_qdy, c->g.ny));
@@ -271,10 +286,8 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
     A.qdy2 = c->qdy2_d[0];
     A.thomas = c->d_thomas;
     A.nmax = nmax;
-    A.tseg = c->d_tseg;
-    A.xR = xR;
-    A.yG = yG;
-    A.yR = yR;
+    A.xtab = c->d_dtab;
+    A.ytab = c->d_dtab + kXTab;
     TBL_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamDefault));
     c->stream = c->own_stream;
     TBL_HIP(hipEventCreate(&c->ev0));
@@ -315,7 +328,7 @@ extern "C" int tbl_destroy(tbl_ctx *c)
     for (auto *p : c->H64) fr(p);
     for (auto *p : c->H32) fr(p);
     fr(c->d_active); fr(c->d_cycles); fr(c->d_nactive); fr(c->d_cycle);
-    fr(c->d_resmax); fr(c->d_lastres); fr(c->d_qdy); fr(c->d_thomas); fr(c->d_tseg);
+    fr(c->d_resmax); fr(c->d_lastres); fr(c->d_qdy); fr(c->d_thomas); fr(c->d_dtab);
     fr(c->d_u0); fr(c->d_u1); fr(c->d_u2);
     fr(c->d_xpenta); fr(c->d_xinteg); fr(c->d_xfilter);
     fr(c->d_t1); fr(c->d_t2); fr(c->d_lapv); fr(c->d_dwydy); fr(c->d_d2wy);

@@ -76,3 +76,50 @@ def test_derivatives_at_every_shape(torch_mod, nx, ny):
     for kind, v in got.items():
         assert rel(v, oracle.deriv(p, kind, f)) < 1e-12, kind
 
+
+
+@pytest.mark.parametrize("n, H, W", [(2, 8, 8), (3, 8, 40), (1, 40, 56), (2, 32, 136), (1, 16, 264), (1, 8, 1024)],
+                         ids=lambda v: str(v))
+def test_network_gradients_at_image_shapes(torch_mod, n, H, W):
+    """Parameter and input gradients against the numpy network: one-column
+    coarsest images, rows that do not fill a group, several images in a group,
+    and a width whose finest levels take the im2col form.  Every output
+    channel copies one (tap, channel) and inputs are small integers, so every value before a bf16 rounding is exact in both and rounds
+    alike; what is left are the fp32 sums over up to 2^13 pixels (1e-5)."""
+    torch = torch_mod
+    from oracle import unet_ref as U
+    from trans_bl_amd import guess
+    rng = np.random.default_rng(H * W + n)
+    x = rng.integers(0, 5, size=(n, H, W, 4)).astype(np.float32)
+    t = rng.integers(-4, 5, size=(n, H, W, 2)).astype(np.float32)
+    theta = []
+    for name, cin, cout, ks, lvl, relu in U.layers():
+        w = np.zeros((ks * ks, cin, cout))
+        o = np.arange(cout)
+        tap = np.where(o % 2 > 0, ks * ks // 2, rng.integers(0, ks * ks, cout))
+        w[tap, 3 * o % cin, o] = 1.0
+        if name == "OUT":
+            w[:] = 1.0                            # the gradient reaches every layer
+        theta += [w.ravel(), rng.integers(0, 2, cout)]
+    theta = np.concatenate(theta)
+    net = guess.Net(H, W, n + 1, seed=7)          # a batch below the capacity
+    net.set_params(theta.astype(np.float32))
+    xd, td = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    gx = torch.zeros_like(xd)
+    torch.cuda.synchronize()
+    loss, g = net.gradients(xd.data_ptr(), td.data_ptr(), n, gx.data_ptr())
+    again = net.gradients(xd.data_ptr(), td.data_ptr(), n, gx.data_ptr())[1]
+    ref = U.UNet(theta, bf16=True)
+    rloss, dout = U.mse_loss_and_grad(ref.forward(x), t)
+    rg, rdx = ref.backward(dout)
+    assert abs(loss - rloss) / rloss < 1e-5
+    off, errs = 0, {}
+    for name, cin, cout, ks, lvl, relu in U.layers():
+        m = ks * ks * cin * cout + cout
+        assert np.any(rg[off:off + m])
+        errs[name] = np.linalg.norm(g[off:off + m] - rg[off:off + m]) / np.linalg.norm(rg[off:off + m])
+        off += m
+    assert max(errs.values()) < 1e-5, errs
+    assert np.linalg.norm(gx.cpu().numpy() - rdx) <= 1e-5 * np.linalg.norm(rdx)
+    if W < 500:
+        assert np.array_equal(g, again)           # no atomics in the direct forms

@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <random>
 #include <string>
 #include <vector>
@@ -73,6 +74,8 @@ struct tbl_net {
     bf16 *col = nullptr;         // im2col scratch
     float *dcol = nullptr;       // dcol scratch
     bf16 *dzb = nullptr;         // bf16 gradient of the current conv
+    float *ws = nullptr;         // partial sums of the current weight gradient
+    float *bs = nullptr;         // and of the bias gradient
     // fp32 gradients of activations
     float *d_act[NCONV] = {nullptr};
     float *d_pool[3] = {nullptr};
@@ -119,11 +122,20 @@ int net_alloc(tbl_net *n)
     }
     A_(n->wp, npk);
     const long N = n->nmax;
-    long maxz = 0, maxcol = 0;
+    // gradients of every layer; the im2col scratch only for layers without a
+    // direct backward form
+    long maxz = 0, maxcol = 0, maxws = 64L * relu_back_slices(N * n->hw(0)), maxbs = 0;
     for (auto &c : n->L) {
+        const int h = n->H >> c.lvl, w = n->W >> c.lvl;
         const long P = N * n->hw(c.lvl);
         maxz = std::max(maxz, P * c.cout);
-        maxcol = std::max(maxcol, P * c.ks * c.ks * c.cin);
+        maxbs = std::max(maxbs, 1L * c.cout * relu_back_slices(P));
+        if (c.ks != 3) continue;
+        if (conv3x3_back_fits(w, c.cin, c.cout))
+            maxws = std::max(maxws, 9L * c.cin * c.cout *
+                                        conv3x3_dw_slices(static_cast<int>(N), h, w, c.cin, c.cout));
+        else
+            maxcol = std::max(maxcol, P * 9 * c.cin);
     }
     A_(n->x_in, N * n->hw(0) * 4);
     A_(n->d_xin, N * n->hw(0) * 4);
@@ -148,6 +160,8 @@ int net_alloc(tbl_net *n)
     A_(n->col, maxcol);
     A_(n->dcol, maxcol);
     A_(n->dzb, maxz);
+    A_(n->ws, maxws);
+    A_(n->bs, maxbs);
     A_(n->d_loss, 1);
 #undef A_
     return TBL_OK;
@@ -185,35 +199,39 @@ void conv_fwd(tbl_net *n, int id, const bf16 *x, int N, hipStream_t st)
 }
 
 // conv backward.  dy: fp32 gradient w.r.t. this conv's output; dx: fp32
-// gradient w.r.t. its input (written, or added when acc); x: its input
-void conv_bwd(tbl_net *n, int id, const bf16 *x, const float *dy, float *dx, int acc, int N,
-              hipStream_t st)
+// gradient w.r.t. its input (written; may be null); x: its input
+void conv_bwd(tbl_net *n, int id, const bf16 *x, const float *dy, float *dx, int N, hipStream_t st)
 {
     const Conv &c = n->L[id];
     const int h = n->H >> c.lvl, w = n->W >> c.lvl;
     const long P = static_cast<long>(N) * h * w;
     const int kk = c.ks * c.ks * c.cin;
-    relu_back(P * c.cout, dy, id == OUT ? nullptr : n->act[id], n->dzb, c.relu, st);
-    bias_grad(P, c.cout, n->dzb, n->g + c.boff, st);
-    const bf16 *col = x;
-    if (c.ks == 3) {
-        im2col(N, h, w, c.cin, x, n->col, st);
-        col = n->col;
+    if (id == OUT) {
+        const int s = relu_back_slices(P);
+        out_back(P, dy, x, n->wb + c.woff, dx, n->ws, n->bs, st);
+        wgrad_reduce(kk * c.cout, s, n->ws, n->g + c.woff, c.cout, s, n->bs, n->g + c.boff, st);
+        return;
     }
+    if (conv3x3_back_fits(w, c.cin, c.cout)) {
+        relu_back_bias(P, c.cout, dy, n->act[id], n->dzb, n->bs, st);
+        conv3x3_dw(N, h, w, c.cin, c.cout, x, n->dzb, n->ws, st);
+        wgrad_reduce(kk * c.cout, conv3x3_dw_slices(N, h, w, c.cin, c.cout), n->ws, n->g + c.woff,
+                     c.cout, relu_back_slices(P), n->bs, n->g + c.boff, st);
+        if (dx) conv3x3_dx(N, h, w, c.cin, c.cout, n->dzb, n->wb + c.woff, dx, st);
+        return;
+    }
+    relu_back(P * c.cout, dy, n->act[id], n->dzb, c.relu, st);
+    bias_grad(P, c.cout, n->dzb, n->g + c.boff, st);
+    im2col(N, h, w, c.cin, x, n->col, st);
     // dW[kk, cout] = col^T dZ   (K = P, split over blocks)
     const long blocks = ((kk + 63) / 64) * ((c.cout + 63) / 64);
     int split = static_cast<int>(std::max(1L, std::min(1024L / std::max(1L, blocks), P / 512)));
-    gemm(kk, c.cout, static_cast<int>(P), col, 1, kk, n->dzb, c.cout, 1, n->g + c.woff, c.cout,
+    gemm(kk, c.cout, static_cast<int>(P), n->col, 1, kk, n->dzb, c.cout, 1, n->g + c.woff, c.cout,
          1.f, 0.f, st, split);
     if (!dx) return;
-    if (c.ks == 3) {
-        gemm(static_cast<int>(P), kk, c.cout, n->dzb, c.cout, 1, n->wb + c.woff, 1, c.cout,
-             n->dcol, kk, 1.f, 0.f, st);
-        col2im(N, h, w, c.cin, n->dcol, dx, acc, st);
-    } else {
-        gemm(static_cast<int>(P), kk, c.cout, n->dzb, c.cout, 1, n->wb + c.woff, 1, c.cout, dx, kk,
-             1.f, acc ? 1.f : 0.f, st);
-    }
+    gemm(static_cast<int>(P), kk, c.cout, n->dzb, c.cout, 1, n->wb + c.woff, 1, c.cout, n->dcol, kk,
+         1.f, 0.f, st);
+    col2im(N, h, w, c.cin, n->dcol, dx, 0, st);
 }
 
 void forward(tbl_net *n, int N, hipStream_t st)
@@ -252,29 +270,29 @@ void forward(tbl_net *n, int N, hipStream_t st)
 void backward(tbl_net *n, int N, bool input_grad, hipStream_t st)
 {
     const int B = n->base;
-    conv_bwd(n, OUT, n->act[D0B], n->d_out, n->d_act[D0B], 0, N, st);
-    conv_bwd(n, D0B, n->act[D0A], n->d_act[D0B], n->d_act[D0A], 0, N, st);
-    conv_bwd(n, D0A, n->cat[0], n->d_act[D0A], n->d_cat[0], 0, N, st);
+    conv_bwd(n, OUT, n->act[D0B], n->d_out, n->d_act[D0B], N, st);
+    conv_bwd(n, D0B, n->act[D0A], n->d_act[D0B], n->d_act[D0A], N, st);
+    conv_bwd(n, D0A, n->cat[0], n->d_act[D0A], n->d_cat[0], N, st);
     up_concat_back(N, n->H, n->W, 2 * B, B, n->d_cat[0], n->d_act[D1B], n->d_act[E0B], 0, st);
-    conv_bwd(n, D1B, n->act[D1A], n->d_act[D1B], n->d_act[D1A], 0, N, st);
-    conv_bwd(n, D1A, n->cat[1], n->d_act[D1A], n->d_cat[1], 0, N, st);
+    conv_bwd(n, D1B, n->act[D1A], n->d_act[D1B], n->d_act[D1A], N, st);
+    conv_bwd(n, D1A, n->cat[1], n->d_act[D1A], n->d_cat[1], N, st);
     up_concat_back(N, n->H >> 1, n->W >> 1, 4 * B, 2 * B, n->d_cat[1], n->d_act[D2B],
                    n->d_act[E1B], 0, st);
-    conv_bwd(n, D2B, n->act[D2A], n->d_act[D2B], n->d_act[D2A], 0, N, st);
-    conv_bwd(n, D2A, n->cat[2], n->d_act[D2A], n->d_cat[2], 0, N, st);
+    conv_bwd(n, D2B, n->act[D2A], n->d_act[D2B], n->d_act[D2A], N, st);
+    conv_bwd(n, D2A, n->cat[2], n->d_act[D2A], n->d_cat[2], N, st);
     up_concat_back(N, n->H >> 2, n->W >> 2, 8 * B, 4 * B, n->d_cat[2], n->d_act[E3B],
                    n->d_act[E2B], 0, st);
-    conv_bwd(n, E3B, n->act[E3A], n->d_act[E3B], n->d_act[E3A], 0, N, st);
-    conv_bwd(n, E3A, n->pool_out[2], n->d_act[E3A], n->d_pool[2], 0, N, st);
+    conv_bwd(n, E3B, n->act[E3A], n->d_act[E3B], n->d_act[E3A], N, st);
+    conv_bwd(n, E3A, n->pool_out[2], n->d_act[E3A], n->d_pool[2], N, st);
     pool_back(N, n->H >> 2, n->W >> 2, 4 * B, n->d_pool[2], n->d_act[E2B], 1, st);
-    conv_bwd(n, E2B, n->act[E2A], n->d_act[E2B], n->d_act[E2A], 0, N, st);
-    conv_bwd(n, E2A, n->pool_out[1], n->d_act[E2A], n->d_pool[1], 0, N, st);
+    conv_bwd(n, E2B, n->act[E2A], n->d_act[E2B], n->d_act[E2A], N, st);
+    conv_bwd(n, E2A, n->pool_out[1], n->d_act[E2A], n->d_pool[1], N, st);
     pool_back(N, n->H >> 1, n->W >> 1, 2 * B, n->d_pool[1], n->d_act[E1B], 1, st);
-    conv_bwd(n, E1B, n->act[E1A], n->d_act[E1B], n->d_act[E1A], 0, N, st);
-    conv_bwd(n, E1A, n->pool_out[0], n->d_act[E1A], n->d_pool[0], 0, N, st);
+    conv_bwd(n, E1B, n->act[E1A], n->d_act[E1B], n->d_act[E1A], N, st);
+    conv_bwd(n, E1A, n->pool_out[0], n->d_act[E1A], n->d_pool[0], N, st);
     pool_back(N, n->H, n->W, B, n->d_pool[0], n->d_act[E0B], 1, st);
-    conv_bwd(n, E0B, n->act[E0A], n->d_act[E0B], n->d_act[E0A], 0, N, st);
-    conv_bwd(n, E0A, n->x_in, n->d_act[E0A], input_grad ? n->d_xin : nullptr, 0, N, st);
+    conv_bwd(n, E0B, n->act[E0A], n->d_act[E0B], n->d_act[E0A], N, st);
+    conv_bwd(n, E0A, n->x_in, n->d_act[E0A], input_grad ? n->d_xin : nullptr, N, st);
 }
 
 int check_n(const tbl_net *n, int N)
@@ -297,7 +315,11 @@ extern "C" int tbl_net_create(int H, int W, int max_batch, unsigned seed, tbl_ne
     n->H = H;
     n->W = W;
     n->nmax = max_batch;
-    int rc = net_alloc(n);
+    static std::once_flag attr_once;
+    static int attr_rc = TBL_OK;
+    std::call_once(attr_once, [] { attr_rc = nn_kernel_attributes(); });
+    int rc = attr_rc;
+    if (rc == TBL_OK) rc = net_alloc(n);
     if (rc == TBL_OK) {
         std::vector<float> h;
         init_params(n, seed, h);
@@ -327,7 +349,7 @@ extern "C" int tbl_net_destroy(tbl_net *n)
     fr(n->w); fr(n->g); fr(n->m); fr(n->v); fr(n->wb); fr(n->wp); fr(n->x_in); fr(n->d_xin);
     for (int i = 0; i < NCONV; ++i) { fr(n->act[i]); fr(n->d_act[i]); }
     for (int l = 0; l < 3; ++l) { fr(n->pool_out[l]); fr(n->d_pool[l]); fr(n->cat[l]); fr(n->d_cat[l]); }
-    fr(n->z); fr(n->out); fr(n->d_out); fr(n->col); fr(n->dcol); fr(n->dzb); fr(n->d_loss);
+    fr(n->z); fr(n->out); fr(n->d_out); fr(n->col); fr(n->dcol); fr(n->dzb); fr(n->d_loss); fr(n->ws); fr(n->bs);
     if (n->own) (void)hipStreamDestroy(n->own);
     delete n;
     return TBL_OK;

@@ -37,5 +37,24 @@ void pack_conv3x3(int cin, int cout, const bf16 *w, bf16 *wp, hipStream_t st);
 void conv3x3(int n, int h, int w, int cin, int cout, const bf16 *x, const bf16 *wp,
              const float *bias, bf16 *y, int relu, hipStream_t st);
 
+// direct backward of a 3x3 convolution (where conv3x3_back_fits): dz = dy * (y >
+// 0) with bias partials bs [relu_back_slices][c], weight-gradient partials ws
+// [conv3x3_dw_slices][9 cin cout], their sums, and the input's gradient from
+// the unpacked weights [tap][cin][cout]
+bool conv3x3_back_fits(int w, int cin, int cout);
+int conv3x3_dw_slices(int n, int h, int w, int cin, int cout);
+int relu_back_slices(long P);
+void relu_back_bias(long P, int c, const float *dy, const bf16 *y, bf16 *dz, float *bs, hipStream_t st);
+void conv3x3_dw(int n, int h, int w, int cin, int cout, const bf16 *x, const bf16 *dz, float *ws,
+                hipStream_t st);
+void wgrad_reduce(int n, int slices, const float *ws, float *g, int cout, int bslices, const float *bs,
+                  float *gb, hipStream_t st);
+void conv3x3_dx(int n, int h, int w, int cin, int cout, const bf16 *dz, const bf16 *wb, float *dx,
+                hipStream_t st);
+// the 1x1 output layer (32 channels in, 2 out): dx, and partials ws [][64], bs [][2]
+void out_back(long P, const float *dy, const bf16 *x, const bf16 *w, float *dx, float *ws, float *bs,
+              hipStream_t st);
+int nn_kernel_attributes();
+
 }  // namespace nn
 }  // namespace tbl

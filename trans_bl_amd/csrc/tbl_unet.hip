@@ -1,10 +1,12 @@
 // BF16 U-Net kernels for the learned multigrid initial guess (gfx950).
 //
-// Activations are NHWC (channels fastest).  A 3x3 convolution is an
-// im2col gather followed by a GEMM on the matrix cores
-// (v_mfma_f32_32x32x8_bf16: bf16 operands, fp32 accumulation); the
-// backward pass is two more GEMMs (weights: col^T x dZ, data: dZ x W^T)
-// and a col2im gather.  Weights keep an fp32 master copy for Adam.
+// Activations are NHWC (channels fastest).  3x3 convolutions run directly on the
+// matrix cores (bf16 operands, fp32 accumulation), forward and backward, from
+// input tiles in LDS; images too wide for those tiles take an im2col gather
+// and a GEMM (weights: col^T x dZ, data: dZ x W^T and a col2im gather).
+// Weights keep an fp32 master copy for Adam.
+#include <algorithm>
+
 #include "tbl_buf.h"
 #include "tbl_nn.h"
 
@@ -13,6 +15,7 @@ namespace nn {
 
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf2f(bf16 h)
 {
@@ -366,6 +369,422 @@ __global__ void __launch_bounds__(256) conv3x3s_kernel(long NP, int H, int W, in
 }
 
 // ---------------------------------------------------------------------------
+// Backward of a 3x3 convolution without the im2col and col2im matrices (9
+// times the activations, bf16 and fp32, each written and read once), which
+// with the GEMM's scalar loads were the time of a training step.
+//
+// Gradient of the input: dX[p, ci] = sum_t sum_co dZ[p - shift(t), co] W[t, ci,
+// co].  Workgroup: 4 wavefronts x MT tiles of 32 flattened pixels x CT = 32 NT
+// input channels; LDS: the dZ pixels its taps reach, all COUT channels, and
+// one tap's weights (the next tap's loads are in flight meanwhile; the bf16
+// weights [tap][ci][co] need no packing).  Each tap is summed over the channels on
+// its own and the taps are added in fp32 in their order, as the GEMM and
+// col2im did: the same values bit for bit (the K = 16 instruction adds as two
+// of K = 8 do), so no bf16 rounding downstream changes.
+// ---------------------------------------------------------------------------
+template <int MT, int NT, int COUT>
+__global__ void __launch_bounds__(256) conv3x3_dx_kernel(long NP, int H, int W, int cin,
+                                                         const bf16 *__restrict__ dZ,
+                                                         const bf16 *__restrict__ wb,
+                                                         float *__restrict__ dX)
+{
+    constexpr int CT = 32 * NT, PX = 128 * MT, ROW = COUT + 8, G = COUT / 8;
+    constexpr int WP = CT * G / 256 > 0 ? CT * G / 256 : 1;
+    extern __shared__ __attribute__((aligned(16))) unsigned char conv_smem[];
+    bf16 *Ws = reinterpret_cast<bf16 *>(conv_smem), *Zs = Ws + CT * ROW;
+    const int NQ = PX + 2 * W + 2;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const long p0 = static_cast<long>(blockIdx.x) * PX, q0 = p0 - W - 1;
+    const int o0 = blockIdx.y * CT;
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    // weights of tap t, rows o0 .. (zero past cin)
+    u4 wr[WP];
+    auto fetch = [&](int t) {
+#pragma unroll
+        for (int s = 0; s < WP; ++s) {
+            const int e = tid + 256 * s, o = e / G, g = e % G;
+            wr[s] = u4{0, 0, 0, 0};
+            if (e < CT * G && o0 + o < cin)
+                wr[s] = *reinterpret_cast<const u4 *>(
+                    wb + (static_cast<long>(t) * cin + o0 + o) * COUT + 8 * g);
+        }
+    };
+    auto stash = [&]() {
+#pragma unroll
+        for (int s = 0; s < WP; ++s) {
+            const int e = tid + 256 * s;
+            if (e < CT * G) *reinterpret_cast<u4 *>(Ws + e / G * ROW + 8 * (e % G)) = wr[s];
+        }
+    };
+    fetch(0);
+    for (int e = tid; e < NQ * G; e += 256) {
+        const int q = e / G, g = e % G;
+        const long gp = q0 + q;
+        u4 v = {0, 0, 0, 0};
+        if (gp >= 0 && gp < NP) v = *reinterpret_cast<const u4 *>(dZ + gp * COUT + 8 * g);
+        *reinterpret_cast<u4 *>(Zs + q * ROW + 8 * g) = v;
+    }
+    stash();
+    int lq[MT];
+    unsigned tapok[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int lp = wave * 32 * MT + m * 32 + (lane & 31);
+        const long pa = p0 + lp;
+        const int wa = static_cast<int>(pa % W), ha = static_cast<int>((pa / W) % H);
+        unsigned ok = 0;
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const int hh = ha - (t / 3 - 1), ww = wa - (t % 3 - 1);
+            if (pa < NP && hh >= 0 && hh < H && ww >= 0 && ww < W) ok |= 1u << t;
+        }
+        lq[m] = lp + W + 1;
+        tapok[m] = ok;
+    }
+    float16v sum[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sum[m][n][i] = 0.f;
+    __syncthreads();
+#pragma unroll 1
+    for (int t = 0; t < 9; ++t) {
+        if (t < 8) fetch(t + 1);
+        const int sh = (t / 3 - 1) * W + (t % 3 - 1);
+        float16v acc[MT][NT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.f;
+#pragma unroll 4
+        for (int kk = 0; kk < COUT; kk += 16) {
+            const int kb = kk + (lane >> 5) * 8;
+            bf16x8 b[NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                b[n] = *reinterpret_cast<const bf16x8 *>(Ws + (n * 32 + (lane & 31)) * ROW + kb);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                bf16x8 a = {};
+                if (tapok[m] >> t & 1u)
+                    a = *reinterpret_cast<const bf16x8 *>(Zs + (lq[m] - sh) * ROW + kb);
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[n], acc[m][n], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sum[m][n][i] += acc[m][n][i];
+        __syncthreads();
+        if (t < 8) {
+            stash();
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int o = o0 + n * 32 + (lane & 31);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const long p = p0 + wave * 32 * MT + m * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+                if (p < NP && o < cin) dX[p * cin + o] = sum[m][n][i];
+            }
+    }
+}
+
+// Gradient of the weights: dW[t, ci, co] = sum_p X[p + shift(t), ci] dZ[p, co].
+// Workgroup: 32 input channels x 32 NC output channels x all 9 taps over a
+// range of row groups; its wavefronts take NC channel blocks x 4 / NC shares
+// of the taps.  Per group of nr image rows LDS holds the input rows -1 ..
+// nr, a zero column each side and one zero row (for the taps outside the
+// image), and the dZ pixels, both as they lie in memory: 16 channel pairs of
+// 4 bytes per pixel and 8 bytes of padding, so a lane's pair of one pixel is one
+// 4-byte read, the four pixel groups of a wavefront fall on different banks,
+// and a tap is a constant offset from the pixel's address.  Eight pixels of a
+// pair are turned into two operands (the even and the odd channel of 8
+// pixels) by byte permutes: 4 MFMAs 16x16x32 per tap and 8 reads.  Partial
+// sums go to a workspace, one slice per blockIdx.x, and are added in order
+// by wgrad_reduce_kernel: no atomics, the same bits every run.
+constexpr int kWgRow = 36;                     // bf16 per staged pixel
+// bytes of the staged input rows, a multiple of 16
+__host__ __device__ inline size_t dw_x_bytes(int nr, int w)
+{
+    return (static_cast<size_t>(nr + 3) * (w + 2) * kWgRow * sizeof(bf16) + 15) / 16 * 16;
+}
+
+template <int NC>
+__global__ void __launch_bounds__(256) conv3x3_dw_kernel(int rows, int H, int W, int nr, int ks,
+                                                         int cin, int cout,
+                                                         const bf16 *__restrict__ X,
+                                                         const bf16 *__restrict__ dZ,
+                                                         float *__restrict__ ws)
+{
+    constexpr int KW = 4 / NC, TM = (8 + KW) / KW;
+    extern __shared__ __attribute__((aligned(16))) unsigned char conv_smem[];
+    const int W2 = W + 2, np = 32 * ks;        // padded row, pixels of a group
+    bf16 *Xs = reinterpret_cast<bf16 *>(conv_smem);
+    bf16 *Zs = Xs + dw_x_bytes(nr, W) / sizeof(bf16);   // [NC][np]
+    uint16_t *at = reinterpret_cast<uint16_t *>(Zs + NC * np * kWgRow);   // [3][np]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nc = wave % NC, kw = __builtin_amdgcn_readfirstlane(wave / NC);
+    const int c0 = blockIdx.y * 32, o0 = blockIdx.z * 32 * NC;
+    const int m4 = (lane & 15) * 4, g = lane >> 4;
+    // the zero borders, written once
+    for (int e = tid; e < (nr + 3) * W2 * (kWgRow / 4); e += 256) {
+        const int q = e / (kWgRow / 4), col = q % W2;
+        if (col == 0 || col == W + 1 || q / W2 == nr + 2)
+            *reinterpret_cast<short4v *>(Xs + q * kWgRow + 4 * (e % (kWgRow / 4))) = short4v{0, 0, 0, 0};
+    }
+    f32x4 acc[TM][2][2];
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][e >> 1][e & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const __amdgpu_buffer_rsrc_t xr =
+        buf_rsrc_uniform(X, static_cast<size_t>(rows) * W * cin * sizeof(bf16));
+    const __amdgpu_buffer_rsrc_t zr =
+        buf_rsrc_uniform(dZ, static_cast<size_t>(rows) * W * cout * sizeof(bf16));
+    const int groups = (rows + nr - 1) / nr;
+    for (int grp = blockIdx.x; grp < groups; grp += gridDim.x) {
+        const int r0 = grp * nr;
+        __syncthreads();
+        // input rows r0 - 1 .. r0 + nr (rows of all images are contiguous; past
+        // either end the buffer reads zero), 8 or (cin 4) 4 channels a piece,
+        // the loads of NI pieces in flight together
+        constexpr int NI = 6;
+        if (cin >= 8) {
+            const int n = (nr + 2) * W, dq = 64 / W, dr = 64 % W, cg = (tid & 3) * 8;
+            int q = tid >> 2, lr = q / W, col = q % W;
+            while (q < n) {
+                u32x4 v[NI];
+                int at_[NI];
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    const unsigned off = static_cast<unsigned>((((r0 - 1) * W + q) * cin + c0 + cg) * 2);
+                    v[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, q < n && c0 + cg < cin ? off : kBufOff, 0, 0);
+                    at_[i] = q < n ? q + 2 * lr + 1 : -1;
+                    q += 64;
+                    lr += dq;
+                    col += dr;
+                    if (col >= W) {
+                        col -= W;
+                        ++lr;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    if (at_[i] >= 0) {
+                        u32x2 *d = reinterpret_cast<u32x2 *>(Xs + at_[i] * kWgRow + cg);
+                        d[0] = u32x2{v[i][0], v[i][1]};
+                        d[1] = u32x2{v[i][2], v[i][3]};
+                    }
+            }
+        } else {
+            for (int q = tid; q < (nr + 2) * W; q += 256) {
+                const unsigned off = static_cast<unsigned>(((r0 - 1) * W + q) * cin * 2);
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(xr, off, 0, 0);
+                bf16 *d = Xs + (q + 2 * (q / W) + 1) * kWgRow;
+#pragma unroll
+                for (int c = 0; c < 32; c += 4) *reinterpret_cast<u32x2 *>(d + c) = c ? u32x2{0, 0} : v;
+            }
+        }
+        {
+            const int n = np * NC * 4;
+            for (int e0 = tid; e0 < n; e0 += 256 * NI) {
+                u32x4 v[NI];
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    const int e = e0 + 256 * i, p = e / (4 * NC), c = e % (4 * NC) * 8;
+                    const unsigned off = static_cast<unsigned>(((r0 * W + p) * cout + o0 + c) * 2);
+                    v[i] = __builtin_amdgcn_raw_buffer_load_b128(zr, p < nr * W ? off : kBufOff, 0, 0);
+                }
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    const int e = e0 + 256 * i, p = e / (4 * NC), c = e % (4 * NC) * 8;
+                    if (e < n) {
+                        u32x2 *d = reinterpret_cast<u32x2 *>(Zs + (c / 32 * np + p) * kWgRow + c % 32);
+                        d[0] = u32x2{v[i][0], v[i][1]};
+                        d[1] = u32x2{v[i][2], v[i][3]};
+                    }
+                }
+            }
+        }
+        // staged row of each pixel for the three tap rows, in units of 8 bytes
+        for (int p = tid; p < np; p += 256) {
+            const int lr = p / W, col = p % W, h = (r0 + lr) % H;
+            const bool in = p < nr * W;
+#pragma unroll
+            for (int dh = -1; dh <= 1; ++dh) {
+                const int row = in && h + dh >= 0 && h + dh < H ? lr + 1 + dh : nr + 2;
+                at[(dh + 1) * np + p] =
+                    static_cast<uint16_t>((row * W2 + (in ? col : 0) + 1) * (kWgRow / 4));
+            }
+        }
+        __syncthreads();
+        for (int k = 0; k < ks; ++k) {
+            auto pairs = [&](const unsigned (&w)[8], bf16x8 &even, bf16x8 &odd) {
+                unsigned ev[4], od[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    ev[i] = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x05040100u);
+                    od[i] = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x07060302u);
+                }
+                __builtin_memcpy(&even, ev, 16);
+                __builtin_memcpy(&odd, od, 16);
+            };
+            bf16x8 b[2];
+            {
+                unsigned w[8];
+                const unsigned char *z = reinterpret_cast<const unsigned char *>(
+                                             Zs + (nc * np + 32 * k + 8 * g) * kWgRow) + m4;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    w[j] = *reinterpret_cast<const unsigned *>(z + j * kWgRow * 2);
+                pairs(w, b[0], b[1]);
+            }
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                const int t = kw + KW * i;
+                if (t < 9) {
+                    uint16_t a8[8];
+                    __builtin_memcpy(a8, __builtin_assume_aligned(at + t / 3 * np + 32 * k + 8 * g, 16), 16);
+                    const unsigned char *x = conv_smem + m4 + (t % 3 - 1) * kWgRow * 2;
+                    unsigned w[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) w[j] = *reinterpret_cast<const unsigned *>(x + 8 * a8[j]);
+                    bf16x8 a[2];
+                    pairs(w, a[0], a[1]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i][e >> 1][e & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            a[e >> 1], b[e & 1], acc[i][e >> 1][e & 1], 0, 0, 0);
+                }
+            }
+        }
+    }
+    float *out = ws + static_cast<size_t>(blockIdx.x) * 9 * cin * cout;
+#pragma unroll
+    for (int q = 0; q < TM; ++q)
+#pragma unroll
+        for (int ea = 0; ea < 2; ++ea)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = kw + KW * q, c = c0 + 2 * (4 * g + i) + ea;
+                if (t < 9 && c < cin)
+                    *reinterpret_cast<float2 *>(
+                        out + (static_cast<size_t>(t) * cin + c) * cout + o0 + 32 * nc + (lane & 15) * 2) =
+                        float2{acc[q][ea][0][i], acc[q][ea][1][i]};
+            }
+}
+
+// g[e] = sum over the slices of ws, the bias partials bs likewise: 64 sums per
+// workgroup, four shares of the slices each, added in order
+__global__ void __launch_bounds__(256) wgrad_reduce_kernel(int n, int slices,
+                                                           const float *__restrict__ ws,
+                                                           float *__restrict__ g, int cout, int bslices,
+                                                           const float *__restrict__ bs,
+                                                           float *__restrict__ gb)
+{
+    __shared__ float part[256];
+    const int e = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
+    const bool w = e < n;
+    const float *src = w ? ws + e : bs + (e - n);
+    const int m = w ? slices : bslices, per = (m + 3) / 4, stride = w ? n : cout;
+    float s = 0.f;
+    if (e < n + cout) {
+        const int m1 = min(m, (q + 1) * per);
+#pragma unroll 8
+        for (int k = q * per; k < m1; ++k) s += src[static_cast<size_t>(k) * stride];
+    }
+    part[threadIdx.x] = s;
+    __syncthreads();
+    if (q == 0 && e < n + cout)
+        (w ? g[e] : gb[e - n]) = ((s + part[threadIdx.x + 64]) + part[threadIdx.x + 128]) + part[threadIdx.x + 192];
+}
+
+// dZ = dY * (y > 0) as bf16, and the block's sums of dZ per channel
+// (bs[block][Cc]): four channels per thread, Cc / 4 threads a pixel; Cc a
+// multiple of 4 that divides 1024
+__global__ void __launch_bounds__(256) relu_back_bias_kernel(long P, int Cc, long per,
+                                                             const float *__restrict__ dY,
+                                                             const bf16 *__restrict__ y,
+                                                             bf16 *__restrict__ dZ,
+                                                             float *__restrict__ bs)
+{
+    __shared__ float red[256][4];
+    const int cg = Cc / 4, c = (threadIdx.x % cg) * 4, px = threadIdx.x / cg, step = 256 / cg;
+    const long p1 = min(P, (blockIdx.x + 1) * per);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (long p = blockIdx.x * per + px; p < p1; p += step) {
+        const float4 d = *reinterpret_cast<const float4 *>(dY + p * Cc + c);
+        const short4v a = *reinterpret_cast<const short4v *>(y + p * Cc + c);
+        const float v[4] = {d.x, d.y, d.z, d.w};
+        short4v z;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bf16 b = f2bf(bf2f(static_cast<bf16>(a[q])) > 0.f ? v[q] : 0.f);
+            z[q] = static_cast<short>(b);
+            s[q] += bf2f(b);
+        }
+        *reinterpret_cast<short4v *>(dZ + p * Cc + c) = z;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[threadIdx.x][q] = s[q];
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < Cc) {
+        float t = 0.f;
+        for (int q = 0; q < step; ++q) t += red[q * cg + threadIdx.x / 4][threadIdx.x % 4];
+        bs[static_cast<size_t>(blockIdx.x) * Cc + threadIdx.x] = t;
+    }
+}
+
+// Backward of the 1x1 output layer (cin inputs of 32, two outputs): dX = dZ W^T,
+// and the block's sums of X^T dZ and dZ.  One input channel and pixel per thread.
+__global__ void __launch_bounds__(256) out_back_kernel(long P, long per, const float *__restrict__ dY,
+                                                       const bf16 *__restrict__ X,
+                                                       const bf16 *__restrict__ w,
+                                                       float *__restrict__ dX,
+                                                       float *__restrict__ ws, float *__restrict__ bs)
+{
+    __shared__ float red[256][4];
+    const int c = threadIdx.x & 31, px = threadIdx.x >> 5;
+    const float w0 = bf2f(w[2 * c]), w1 = bf2f(w[2 * c + 1]);
+    const long p1 = min(P, (blockIdx.x + 1) * per);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (long p = blockIdx.x * per + px; p < p1; p += 8) {
+        const float2 d = *reinterpret_cast<const float2 *>(dY + 2 * p);
+        const float z0 = bf2f(f2bf(d.x)), z1 = bf2f(f2bf(d.y)), x = bf2f(X[32 * p + c]);
+        dX[32 * p + c] = __builtin_fmaf(z1, w1, z0 * w0);
+        s[0] += x * z0;
+        s[1] += x * z1;
+        s[2] += z0;
+        s[3] += z1;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[threadIdx.x][q] = s[q];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        float t = 0.f;
+        for (int q = 0; q < 8; ++q) t += red[32 * q + threadIdx.x / 2][threadIdx.x % 2];
+        ws[blockIdx.x * 64 + threadIdx.x] = t;
+    } else if (threadIdx.x < 66) {
+        float t = 0.f;
+        for (int q = 0; q < 8; ++q) t += red[32 * q][2 + threadIdx.x - 64];
+        bs[blockIdx.x * 2 + threadIdx.x - 64] = t;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // element-wise and layout kernels
 // ---------------------------------------------------------------------------
 static inline unsigned nb(long n) { return static_cast<unsigned>((n + 255) / 256); }
@@ -697,6 +1116,109 @@ void conv3x3(int n, int h, int w, int cin, int cout, const bf16 *x, const bf16 *
         hipLaunchKernelGGL(conv3x3_kernel<32>, grid, dim3(256), 0, st, np, h, w, cin, cinp, cout, x,
                            wp, bias, y, relu);
     }
+}
+
+
+// ---- backward launchers ------------------------------------------------------
+constexpr size_t kBwdLds = 160 * 1024;
+// tiles of 32 input channels per workgroup (and 3 - nt pixel tiles a wavefront)
+static int dx_nt(int cin, int cout) { return cin % 64 == 0 && cout != 32 ? 2 : 1; }
+static size_t dx_lds(int px, int w, int ct, int cout)
+{
+    return static_cast<size_t>(px + 2 * w + 2 + ct) * (cout + 8) * sizeof(bf16);
+}
+// rows per group of conv3x3_dw_kernel: about 256 / NC pixels, which keeps two
+// workgroups' tiles on a CU
+static int dw_rows(int w, int nc) { return std::max(1, ((nc == 4 ? 128 : nc == 2 ? 192 : 256) + w / 2) / w); }
+static size_t dw_lds(int w, int nc)
+{
+    const int nr = dw_rows(w, nc), np = (nr * w + 31) / 32 * 32;
+    return dw_x_bytes(nr, w) + static_cast<size_t>(nc) * np * kWgRow * sizeof(bf16) +
+           3 * np * sizeof(uint16_t);
+}
+static int dw_chunks(int cout) { return cout % 128 == 0 ? 4 : cout % 64 == 0 ? 2 : 1; }
+// the direct backward kernels take a layer whose tiles fit (widths up to about
+// 500) and whose staged rows fit 16-bit offsets
+bool conv3x3_back_fits(int w, int cin, int cout)
+{
+    const int nc = dw_chunks(cout);
+    const bool co = cout == 32 || cout == 64 || cout == 128 || cout == 256;
+    const int nt = dx_nt(cin, cout);
+    return co && cin % 4 == 0 && dw_lds(w, nc) <= kBwdLds &&
+           dx_lds(128 * (3 - nt), w, 32 * nt, cout) <= kBwdLds &&
+           static_cast<long>(dw_rows(w, nc) + 3) * (w + 2) * (kWgRow / 4) < 65536;
+}
+// slices of the weight gradient's workspace: enough workgroups for the chip on
+// the wide levels, fewer where a slice is large (its write and read grow with it)
+int conv3x3_dw_slices(int n, int h, int w, int cin, int cout)
+{
+    const int nc = dw_chunks(cout), rows = n * h, nr = dw_rows(w, nc);
+    const int blocks = (cin + 31) / 32 * (cout / (32 * nc));
+    return std::max(1, std::min((rows + nr - 1) / nr, (nc == 1 ? 512 : 256) / blocks));
+}
+int relu_back_slices(long P) { return static_cast<int>(std::max(1L, std::min(512L, P / 64))); }
+
+void conv3x3_dw(int n, int h, int w, int cin, int cout, const bf16 *x, const bf16 *dz, float *ws,
+                hipStream_t st)
+{
+    const int nc = dw_chunks(cout), nr = dw_rows(w, nc), ks = (nr * w + 31) / 32;
+    const dim3 grid(conv3x3_dw_slices(n, h, w, cin, cout), (cin + 31) / 32, cout / (32 * nc));
+    const size_t lds = dw_lds(w, nc);
+    if (nc == 4)
+        hipLaunchKernelGGL(conv3x3_dw_kernel<4>, grid, dim3(256), lds, st, n * h, h, w, nr, ks, cin, cout, x, dz, ws);
+    else if (nc == 2)
+        hipLaunchKernelGGL(conv3x3_dw_kernel<2>, grid, dim3(256), lds, st, n * h, h, w, nr, ks, cin, cout, x, dz, ws);
+    else
+        hipLaunchKernelGGL(conv3x3_dw_kernel<1>, grid, dim3(256), lds, st, n * h, h, w, nr, ks, cin, cout, x, dz, ws);
+}
+
+#define TBL_DX_SHAPES(X) X(2, 1, 32) X(2, 1, 64) X(1, 2, 64) X(1, 2, 128) X(1, 2, 256) X(2, 1, 128) X(2, 1, 256)
+void conv3x3_dx(int n, int h, int w, int cin, int cout, const bf16 *dz, const bf16 *wb, float *dx,
+                hipStream_t st)
+{
+    const long np = static_cast<long>(n) * h * w;
+    const int nt = dx_nt(cin, cout), px = 128 * (3 - nt);
+    const dim3 grid(static_cast<unsigned>((np + px - 1) / px), (cin + 32 * nt - 1) / (32 * nt));
+#define X(MT, NT, CO)                                                                            \
+    if (nt == NT && cout == CO) {                                                                \
+        hipLaunchKernelGGL((conv3x3_dx_kernel<MT, NT, CO>), grid, dim3(256),                     \
+                           dx_lds(px, w, 32 * NT, CO), st, np, h, w, cin, dz, wb, dx);           \
+        return;                                                                                  \
+    }
+    TBL_DX_SHAPES(X)
+#undef X
+}
+void wgrad_reduce(int n, int slices, const float *ws, float *g, int cout, int bslices, const float *bs,
+                  float *gb, hipStream_t st)
+{
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((n + cout + 63) / 64), dim3(256), 0, st, n, slices, ws, g, cout,
+                       bslices, bs, gb);
+}
+void relu_back_bias(long P, int c, const float *dy, const bf16 *y, bf16 *dz, float *bs, hipStream_t st)
+{
+    const int s = relu_back_slices(P);
+    hipLaunchKernelGGL(relu_back_bias_kernel, dim3(s), dim3(256), 0, st, P, c, (P + s - 1) / s, dy, y, dz, bs);
+}
+void out_back(long P, const float *dy, const bf16 *x, const bf16 *w, float *dx, float *ws, float *bs,
+              hipStream_t st)
+{
+    const int s = relu_back_slices(P);
+    hipLaunchKernelGGL(out_back_kernel, dim3(s), dim3(256), 0, st, P, (P + s - 1) / s, dy, x, w, dx, ws, bs);
+}
+int nn_kernel_attributes()
+{
+    hipError_t e = hipSuccess;
+    auto allow = [&](const void *f) {
+        const hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kBwdLds);
+        if (r != hipSuccess) e = r;
+    };
+#define X(MT, NT, CO) allow(reinterpret_cast<const void *>(&conv3x3_dx_kernel<MT, NT, CO>));
+    TBL_DX_SHAPES(X)
+#undef X
+    allow(reinterpret_cast<const void *>(&conv3x3_dw_kernel<1>));
+    allow(reinterpret_cast<const void *>(&conv3x3_dw_kernel<2>));
+    allow(reinterpret_cast<const void *>(&conv3x3_dw_kernel<4>));
+    return e == hipSuccess ? TBL_OK : TBL_ERR_HIP;
 }
 
 }  // namespace nn

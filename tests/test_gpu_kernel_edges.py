@@ -123,3 +123,35 @@ def test_network_gradients_at_image_shapes(torch_mod, n, H, W):
     assert np.linalg.norm(gx.cpu().numpy() - rdx) <= 1e-5 * np.linalg.norm(rdx)
     if W < 500:
         assert np.array_equal(g, again)           # no atomics in the direct forms
+
+
+@pytest.mark.parametrize("nmodes, kphys", [(1, 4), (2, 4), (3, 8), (4, 8), (5, 16), (16, 32), (20, 64), (33, 128),
+                                           (64, 128), (65, 256), (100, 256), (40, 512), (30, 1024)])
+def test_nonlinear_terms_at_every_size(torch_mod, nmodes, kphys):
+    """Both forms of the nonlinear terms against the oracle (1e-13, as the
+    tests of their usual sizes), the mode counts at and below kphys / 2, a plane
+    that is no multiple of a group of points; fields of scales 1 to 1e-6."""
+    torch = torch_mod
+    g = wl.Grid(33, 17, nmodes, 2, 0.02, 1e-3, 1.02, 0.0, 0.3)
+    rng = np.random.default_rng(nmodes)
+    names = ("ux", "uy", "uz", "wx", "wy", "wz")
+    scale = dict(zip(names, (1.0, 1e-3, 0.1, 1e-2, 10.0, 1e-6)))
+    F = {k: scale[k] * (rng.normal(size=(nmodes, 17, 33)) + 1j * rng.normal(size=(nmodes, 17, 33))) for k in names}
+    base = {k: rng.normal(size=(17, 33)) for k in ("uxb", "uyb", "wzb", "varg", "dvargdx")}
+    p = oracle.make_params(g.nx, g.ny, g.nmodes, g.levels, g.dx, g.dy0, g.stf, g.alpha, g.beta)
+    zero = {k: np.zeros((17, 33)) for k in base}
+    with context(g) as ctx:
+        d = {k: torch.from_numpy(F[k]).to("cuda") for k in names}
+        for b in (base, zero):
+            db = {k: torch.from_numpy(b[k]).to("cuda") for k in b}
+            out = [torch.zeros_like(d["ux"]) for _ in range(4)]
+            ctx.terms_dev(kphys, {k: v.data_ptr() for k, v in db.items()}, *[d[k].data_ptr() for k in names],
+                          *[o.data_ptr() for o in out])
+            ctx.synchronize()
+            for o, ref in zip(out, oracle.terms(p, kphys, b, F)):
+                assert rel(o.cpu().numpy(), ref) < 1e-13
+        out = [torch.zeros_like(d["ux"]) for _ in range(3)]
+        ctx.terms_fi_dev(kphys, None, *[d[k].data_ptr() for k in names], *[o.data_ptr() for o in out])
+        ctx.synchronize()
+    for o, ref in zip(out, oracle.terms_fi(p, kphys, None, F)):
+        assert rel(o.cpu().numpy(), ref) < 1e-13

@@ -5,9 +5,6 @@
 
 namespace tbl {
 
-// points per workgroup of the nonlinear-terms kernel
-constexpr int kNlPts = 4;
-
 // base flow and curvature (COMMON /blas/, /vc/), real (nx, ny) device arrays
 struct BaseArgs {
     const double *uxb, *uyb, *wzb, *varg, *dvargdx;
@@ -40,7 +37,7 @@ struct RkArgs {
     int stage, nx, ny, K;
 };
 
-size_t nlterms_lds(int K, int N);
+bool nlterms_fits(int K, int N);   // kphys values the nonlinear terms accept
 int terms(const RhsArgs &r, int kphys, hipStream_t st);
 int drv_combine(const DrvArgs &r, hipStream_t st);
 int rk_update(const RkArgs &r, hipStream_t st);

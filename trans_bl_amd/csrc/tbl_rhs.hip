@@ -9,12 +9,9 @@
 // User layout (complex (nx, ny, K), x fastest); base-flow arrays real
 // (nx, ny).  All kernels but the nonlinear one are point-wise and
 // HBM-bound.  The nonlinear terms transform every (x, y) point's K modes to
-// kphys points in z, multiply there and transform back: a workgroup takes
-// kNlPts points, stages their 6 K modes in LDS, synthesises each physical
-// point's six values as a direct real DFT from a twiddle table in LDS,
-// forms the four products, and analyses them back mode by mode -- the same
-// transform pair as the reference's packed real FFT (mode 0 real, the
-// odd-even mode in mode 0's imaginary part), to rounding.
+// kphys points in z, multiply there and transform back, all in LDS
+// (nlterms_kernel) -- the transform pair of the reference's packed real FFT
+// (mode 0 real, the odd-even mode in mode 0's imaginary part), to rounding.
 #include "tbl_rhs.h"
 
 namespace tbl {
@@ -69,107 +66,230 @@ __global__ void lterms_kernel(RhsArgs r)
               r.wz[e], r.a[e], r.bb[e], r.c[e], r.d[e]);
 }
 
-// nlterms_gv (FI: nlterms_fi, the first three products, no base-flow
-// terms): kNlPts points per workgroup of 256 threads; LDS holds the six
-// inputs' modes [f][m][p], the four products [q][n][p] and the twiddles
-template <bool FI>
-__global__ void __launch_bounds__(256) nlterms_kernel(RhsArgs r, int N)
+// ---- nlterms_gv / nlterms_fi ------------------------------------------------------
+// DFT of R values in registers, exponent -2 pi i k q / R
+template <int R>
+__device__ __forceinline__ void dft(cxd (&x)[R])
 {
-    constexpr int NQ = FI ? 3 : 4;
-    extern __shared__ double sm[];
-    const int K = r.K, P = kNlPts;
-    const size_t plane = static_cast<size_t>(r.nx) * r.ny;
-    const size_t p0 = static_cast<size_t>(blockIdx.x) * P;
-    const int np = static_cast<int>(plane - p0 < static_cast<size_t>(P) ? plane - p0 : P);
-    cxd *M = reinterpret_cast<cxd *>(sm);                  // [6][K][P]
-    double *Q = sm + 2 * 6 * K * P;                        // [4][N][P]
-    double *cs = Q + 4 * N * P, *sn = cs + N;              // cos, sin (2 pi t / N)
-    const cxd *in[6] = {r.ux, r.uy, r.uz, r.wx, r.wy, r.wz};
-    for (int t = threadIdx.x; t < N; t += blockDim.x) {
-        cs[t] = r.tw[t];
-        sn[t] = r.tw[N + t];
+    if constexpr (R == 2) {
+        const cxd a = x[0], b = x[1];
+        x[0] = a + b;
+        x[1] = a - b;
+    } else if constexpr (R == 4) {
+        const cxd a = x[0] + x[2], b = x[0] - x[2], c = x[1] + x[3], d = x[1] - x[3];
+        x[0] = a + c;
+        x[2] = a - c;
+        x[1] = {b.re + d.im, b.im - d.re};
+        x[3] = {b.re - d.im, b.im + d.re};
+    } else {
+        cxd e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
+        dft<4>(e);
+        dft<4>(o);
+        const double h = 0.70710678118654752440;
+        const cxd t[4] = {o[0], {h * (o[1].re + o[1].im), h * (o[1].im - o[1].re)},
+                          {o[2].im, -o[2].re}, {h * (o[3].im - o[3].re), -h * (o[3].re + o[3].im)}};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            x[q] = e[q] + t[q];
+            x[q + 4] = e[q] - t[q];
+        }
     }
-    for (int t = threadIdx.x; t < 6 * K * P; t += blockDim.x) {
-        const int p = t % P, m = (t / P) % K, f = t / (P * K);
-        M[t] = p < np ? in[f][static_cast<size_t>(m) * plane + p0 + p] : cxd{0.0, 0.0};
+}
+__device__ __forceinline__ cxd conj_of(cxd a) { return {a.re, -a.im}; }
+
+// LDS slot of element n of one point's sequence: a skipped slot every 8 keeps
+// the butterflies' strided reads on all banks
+__host__ __device__ constexpr int nl_slot(int n) { return n + (n >> 3); }
+// points of a workgroup and sequence stride (complex): N * points = 1024, so 256
+// threads hold one pair of modes each
+template <int N>
+struct NlShape {
+    static constexpr int M = N / 2, P = 1024 / N, SEQ = (nl_slot(M - 1) + 1) * P;
+    static constexpr int FR = M >= 4 ? 4 : 2;           // radix of the innermost pass
+};
+// radix of the pass on sub-length L: 8 while that leaves 4s
+constexpr int nl_radix(int L) { return L % 64 == 32 || L >= 128 ? 8 : L == 8 ? 2 : 4; }
+
+// In-place passes of NS sequences: decimation in frequency from sub-length L
+// down to FR (natural order in, digit-reversed out), and its transpose back
+template <int N, int NS, int L, bool UP>
+__device__ __forceinline__ void nl_pass(cxd *x, const cxd *tw)
+{
+    using S = NlShape<N>;
+    constexpr int R = nl_radix(L), J = L / R, B = S::M / R * S::P;   // butterflies a sequence
+    for (int e = threadIdx.x; e < NS * B; e += 256) {
+        const int p = e % S::P, b = e / S::P % (S::M / R), f = e / B;
+        const int j = b % J, base = b / J * L + j;
+        cxd *s = x + f * S::SEQ + p;
+        cxd v[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            v[q] = s[nl_slot(base + q * J) * S::P];
+            if (UP && q) v[q] = cmul(v[q], tw[j * q * (N / L)]);
+        }
+        dft<R>(v);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (!UP && q) v[q] = cmul(v[q], tw[j * q * (N / L)]);
+            s[nl_slot(base + q * J) * S::P] = v[q];
+        }
     }
     __syncthreads();
-    // synthesis: v_n = Re c_0 + (Im c_0 / 2)(-1)^n + sum_m Re(c_m e^{-2 pi i m n / N})
-    for (int t = threadIdx.x; t < N * P; t += blockDim.x) {
-        const int p = t % P, n = t / P;
-        double v[6];
-        const double alt = (n & 1) ? -0.5 : 0.5;
+}
+template <int N, int NS, int L>
+__device__ __forceinline__ void nl_down(cxd *x, const cxd *tw)
+{
+    if constexpr (L > NlShape<N>::FR) {
+        nl_pass<N, NS, L, false>(x, tw);
+        nl_down<N, NS, L / nl_radix(L)>(x, tw);
+    }
+}
+template <int N, int NS, int L>
+__device__ __forceinline__ void nl_up(cxd *x, const cxd *tw)
+{
+    if constexpr (L > NlShape<N>::FR) {
+        nl_up<N, NS, L / nl_radix(L)>(x, tw);
+        nl_pass<N, NS, L, true>(x, tw);
+    }
+}
+
+// nlterms_gv (FI: nlterms_fi, the first three products, no base-flow terms).
+// Each field is a real sequence of N values in z: its even and odd values are
+// one complex sequence of M = N / 2 (no field is mixed with another, so a
+// small one keeps its own rounding), transformed in place in LDS.  The
+// inverse ends in digit-reversed order, where the products need no order;
+// its innermost pass, the products and the first pass back are one step in
+// registers.  A thread keeps the modes m and M - m of a point from the load to
+// the base-flow terms.  As a direct DFT (O(K N) per point, 65 GFLOP at
+// 1025x193x64 with N = 128) this kernel was bound by FP64 arithmetic: 3466 us;
+// as FFTs by its LDS passes and memory (10 fields of 203 MB): 619 us.
+template <int N, bool FI>
+__global__ void __launch_bounds__(256) nlterms_kernel(RhsArgs r)
+{
+    using S = NlShape<N>;
+    constexpr int M = S::M, P = S::P, NQ = FI ? 3 : 4, FR = S::FR;
+    extern __shared__ double sm[];
+    cxd *X = reinterpret_cast<cxd *>(sm), *tw = X + 6 * S::SEQ;
+    const int K = r.K, t = threadIdx.x;
+    const size_t plane = static_cast<size_t>(r.nx) * r.ny;
+    // neighbouring groups of points share cache lines: in a row on one XCD
+    const int groups = static_cast<int>((plane + P - 1) / P), per = (groups + 7) / 8;
+    const int grp = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    if (grp >= groups) return;
+    const size_t p0 = static_cast<size_t>(grp) * P;
+    // this thread's point and modes (item 0: modes 0 and M / 2)
+    const int p = t % P, m1 = t / P, m2 = m1 ? M - m1 : M / 2;
+    const bool live = p0 + p < plane;
+    const size_t at = live ? p0 + p : plane - 1;
+    const cxd *in[6] = {r.ux, r.uy, r.uz, r.wx, r.wy, r.wz};
+    cxd c1[6], c2[6];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        c1[f] = m1 < K ? in[f][m1 * plane + at] : cxd{0.0, 0.0};
+        c2[f] = m2 < K ? in[f][m2 * plane + at] : cxd{0.0, 0.0};
+    }
+    for (int e = t; e < N; e += 256) tw[e] = {r.tw[e], -r.tw[N + e]};
+    __syncthreads();
+    // synthesis: v_n = Re c_0 + (Im c_0 / 2)(-1)^n + sum_m Re(c_m e^{-2 pi i m n / N});
+    // with A_m = c_m / 2, A_{N-m} its conjugate, the even values' spectrum is A_m +
+    // A_{m+M}, the odd ones' (A_m - A_{m+M}) e^{-2 pi i m / N}
+    const cxd w1 = tw[m1], w2 = tw[m2];
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+        cxd z1, z2;
+        if (m1) {
+            const cxd a = 0.5 * c1[f], b = 0.5 * c2[f];
+            const cxd o1 = cmul(a - conj_of(b), w1), o2 = cmul(b - conj_of(a), w2);
+            z1 = a + conj_of(b) + cxd{-o1.im, o1.re};
+            z2 = b + conj_of(a) + cxd{-o2.im, o2.re};
+        } else {
+            const double a = c1[f].re, h = 0.5 * c1[f].im;
+            z1 = {a + h, a - h};
+            // m = M / 2 pairs with itself: Re c + i (i Im c)(-i) = c's conjugate pair
+            const cxd b = 0.5 * c2[f], o2 = cmul(b - conj_of(b), w2);
+            z2 = b + conj_of(b) + cxd{-o2.im, o2.re};
+        }
+        X[f * S::SEQ + nl_slot(m1) * P + p] = z1;
+        if (M > 1) X[f * S::SEQ + nl_slot(m2) * P + p] = z2;
+    }
+    __syncthreads();
+    nl_down<N, 6, M>(X, tw);
+    for (int e = t; e < M / FR * P; e += 256) {
+        cxd *s = X + nl_slot(e / P * FR) * P + e % P;       // FR divides 8: no skip inside
+        cxd v[6][FR];
 #pragma unroll
         for (int f = 0; f < 6; ++f) {
-            const cxd c0 = M[(f * K) * P + p];
-            v[f] = c0.re + alt * c0.im;
-        }
-        int idx = 0;
-        for (int m = 1; m < K; ++m) {
-            idx += n;
-            if (idx >= N) idx -= N;
-            const double cm = cs[idx], sm_ = sn[idx];
 #pragma unroll
-            for (int f = 0; f < 6; ++f) {
-                const cxd c = M[(f * K + m) * P + p];
-                v[f] += c.re * cm + c.im * sm_;
-            }
+            for (int q = 0; q < FR; ++q) v[f][q] = s[f * S::SEQ + q * P];
+            dft<FR>(v[f]);
         }
         // ux uy uz wx wy wz -> a = uy wx - ux wy, b = ux wz - uz wx,
-        // c = uz wy - uy wz, d = ux ux (nlterms_par.f:152-159)
-        Q[(0 * N + n) * P + p] = v[1] * v[3] - v[0] * v[4];
-        Q[(1 * N + n) * P + p] = v[0] * v[5] - v[2] * v[3];
-        Q[(2 * N + n) * P + p] = v[2] * v[4] - v[1] * v[5];
-        if (!FI) Q[(3 * N + n) * P + p] = v[0] * v[0];
+        // c = uz wy - uy wz, d = ux ux (nlterms_par.f:152-159), conjugated: the
+        // analysis has the opposite sign in the exponent
+        cxd y[4][FR];
+#pragma unroll
+        for (int q = 0; q < FR; ++q) {
+            const cxd ux = v[0][q], uy = v[1][q], uz = v[2][q], wx = v[3][q], wy = v[4][q], wz = v[5][q];
+            y[0][q] = {uy.re * wx.re - ux.re * wy.re, -(uy.im * wx.im - ux.im * wy.im)};
+            y[1][q] = {ux.re * wz.re - uz.re * wx.re, -(ux.im * wz.im - uz.im * wx.im)};
+            y[2][q] = {uz.re * wy.re - uy.re * wz.re, -(uz.im * wy.im - uy.im * wz.im)};
+            y[3][q] = {ux.re * ux.re, -(ux.im * ux.im)};
+        }
+#pragma unroll
+        for (int f = 0; f < NQ; ++f) {
+            dft<FR>(y[f]);
+#pragma unroll
+            for (int q = 0; q < FR; ++q) s[f * S::SEQ + q * P] = y[f][q];
+        }
     }
     __syncthreads();
-    // analysis: c_0 = (1/N) sum v_n (real), c_m = (2/N) sum v_n e^{+2 pi i m n / N};
-    // entries below 1e-14 flushed (nlterms_par.f:418-423); then the
-    // base-flow terms added (nlterms_par.f:167-177)
+    nl_up<N, NQ, M>(X, tw);
+    if (!live) return;
+    // analysis: c_0 = (1/N) sum v_n (real), c_m = (2/N) sum v_n e^{+2 pi i m n / N}
+    // from the even and odd values' transforms; entries below 1e-14 flushed
+    // (nlterms_par.f:418-423); then the base-flow terms (nlterms_par.f:167-177)
     cxd *out[4] = {r.a, r.bb, r.c, r.d};
-    for (int t = threadIdx.x; t < K * P; t += blockDim.x) {
-        const int p = t % P, m = t / P;
-        if (p >= np) continue;
-        double re[4] = {0, 0, 0, 0}, im[4] = {0, 0, 0, 0};
-        int idx = 0;
-        for (int n = 0; n < N; ++n) {
-            const double cm = cs[idx], sm_ = sn[idx];
+    cxd n1[4], n2[4];
+    const double sc = 2.0 / static_cast<double>(N);
+    auto flush = [](cxd z) -> cxd {
+        return {fabs(z.re) < 1e-14 ? 0.0 : z.re, fabs(z.im) < 1e-14 ? 0.0 : z.im};
+    };
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                const double v = Q[(q * N + n) * P + p];
-                re[q] += v * cm;
-                im[q] += v * sm_;
-            }
-            idx += m;
-            if (idx >= N) idx -= N;
+    for (int f = 0; f < NQ; ++f) {
+        const cxd u = conj_of(X[f * S::SEQ + nl_slot(m1) * P + p]);
+        const cxd v = M > 1 ? conj_of(X[f * S::SEQ + nl_slot(m2) * P + p]) : cxd{0.0, 0.0};
+        if (m1) {
+            const cxd e = 0.5 * (u + conj_of(v)), d = 0.5 * (u - conj_of(v));
+            const cxd o = cmul(cxd{d.im, -d.re}, conj_of(w1));
+            n1[f] = flush(sc * (e + o));
+            n2[f] = flush(sc * conj_of(e - o));
+        } else {
+            n1[f] = flush(cxd{0.5 * sc * (u.re + u.im), 0.0});
+            n2[f] = flush(sc * v);
         }
-        const double sc = (m == 0 ? 1.0 : 2.0) / static_cast<double>(N);
-        const size_t e2 = p0 + p;
+    }
+    const size_t e2 = p0 + p;
+    auto put = [&](int m, const cxd (&c)[6], const cxd (&nl)[4]) {
+        if (m >= K) return;
         const size_t e = static_cast<size_t>(m) * plane + e2;
-        cxd nl[4];
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            double x = re[q] * sc, y = m == 0 ? 0.0 : im[q] * sc;
-            if (fabs(x) < 1e-14) x = 0.0;
-            if (fabs(y) < 1e-14) y = 0.0;
-            nl[q] = {x, y};
-        }
         if (FI) {
             out[0][e] = nl[0];
             out[1][e] = nl[1];
             out[2][e] = nl[2];
-            continue;
+            return;
         }
         cxd la, lb, lc, ld;
-        lin_terms(r.b.uxb[e2], r.b.uyb[e2], r.b.wzb[e2], M[(0 * K + m) * P + p],
-                  M[(1 * K + m) * P + p], M[(3 * K + m) * P + p], M[(4 * K + m) * P + p],
-                  M[(5 * K + m) * P + p], la, lb, lc, ld);
+        lin_terms(r.b.uxb[e2], r.b.uyb[e2], r.b.wzb[e2], c[0], c[1], c[3], c[4], c[5], la, lb, lc, ld);
         out[0][e] = la + nl[0];
         out[1][e] = lb + nl[1];
         out[2][e] = lc + nl[2];
         out[3][e] = ld + nl[3];
-    }
+    };
+    put(m1, c1, n1);
+    if (M > 1) put(m2, c2, n2);
 }
+
+#define TBL_NL_SIZES(X) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
 
 // drv_gv's combination (main_par.f:1380-1397), rows 2..ny
 __global__ void drv_combine_kernel(DrvArgs r)
@@ -235,9 +355,11 @@ __global__ void pert_kernel(cxd *uy, cxd *d2, const cxd *pu, const cxd *pd, int 
 
 }  // namespace
 
-size_t nlterms_lds(int K, int N)
+bool nlterms_fits(int K, int N)
 {
-    return sizeof(double) * (2 * 6 * static_cast<size_t>(K) * kNlPts + 4 * static_cast<size_t>(N) * kNlPts + 2 * N);
+    // the modes and values of 4 points and the twiddles within 160 KB of LDS
+    return sizeof(double) * (2 * 6 * 4 * static_cast<size_t>(K) + (4 * 4 + 2) * static_cast<size_t>(N)) <=
+           160 * 1024;
 }
 
 int terms(const RhsArgs &r, int kphys, hipStream_t st)
@@ -247,13 +369,20 @@ int terms(const RhsArgs &r, int kphys, hipStream_t st)
         hipLaunchKernelGGL(lterms_kernel, grid, dim3(256), 0, st, r);
     } else {
         const size_t plane = static_cast<size_t>(r.nx) * r.ny;
-        dim3 grid(static_cast<unsigned>((plane + kNlPts - 1) / kNlPts));
-        if (r.fi)
-            hipLaunchKernelGGL(nlterms_kernel<true>, grid, dim3(256), nlterms_lds(r.K, kphys), st,
-                               r, kphys);
-        else
-            hipLaunchKernelGGL(nlterms_kernel<false>, grid, dim3(256), nlterms_lds(r.K, kphys), st,
-                               r, kphys);
+#define X(N)                                                                                  \
+    if (kphys == N) {                                                                         \
+        const size_t groups = (plane + NlShape<N>::P - 1) / NlShape<N>::P;                    \
+        const dim3 grid(static_cast<unsigned>((groups + 7) / 8 * 8));                         \
+        const size_t lds = sizeof(cxd) * (6 * NlShape<N>::SEQ + N);                           \
+        if (r.fi)                                                                             \
+            hipLaunchKernelGGL((nlterms_kernel<N, true>), grid, dim3(256), lds, st, r);       \
+        else                                                                                  \
+            hipLaunchKernelGGL((nlterms_kernel<N, false>), grid, dim3(256), lds, st, r);      \
+        return TBL_OK;                                                                        \
+    }
+        TBL_NL_SIZES(X)
+#undef X
+        return TBL_ERR_ARG;
     }
     return TBL_OK;
 }
@@ -285,10 +414,13 @@ int pert_rows(cx<double> *uy, cx<double> *d2, const cx<double> *pu, const cx<dou
 
 int rhs_kernel_attributes()
 {
-    TBL_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&nlterms_kernel<false>),
+#define X(N)                                                                                       \
+    TBL_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&nlterms_kernel<N, false>),         \
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));          \
+    TBL_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&nlterms_kernel<N, true>),          \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    TBL_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&nlterms_kernel<true>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    TBL_NL_SIZES(X)
+#undef X
     return TBL_OK;
 }
 

@@ -155,3 +155,41 @@ def test_nonlinear_terms_at_every_size(torch_mod, nmodes, kphys):
         ctx.synchronize()
     for o, ref in zip(out, oracle.terms_fi(p, kphys, None, F)):
         assert rel(o.cpu().numpy(), ref) < 1e-13
+
+
+RHS_GRIDS = [g for g in DERIV_GRIDS if g[0] >= 65 or g[1] > 400]
+
+
+@pytest.mark.parametrize("form", ["linear", "nonlinear", "flat plate", "in place"])
+@pytest.mark.parametrize("nx, ny", RHS_GRIDS)
+def test_right_hand_side_at_every_shape(torch_mod, nx, ny, form):
+    """The right-hand side against the oracle on random values (1e-12 of the
+    largest value, as the parity tests); in place: dvx over wx, dvz over wz,
+    which the kernels that need their inputs twice must not take.  Row 1 keeps
+    the caller's values."""
+    torch = torch_mod
+    g = wl.Grid(nx, ny, 3, 2, 0.02, 1e-3, 1.004, 0.0, 0.3)
+    rng = np.random.default_rng(nx + ny)
+    names = ("ux", "uy", "uz", "wx", "wy", "wz")
+    F = {k: rng.normal(size=(3, ny, nx)) + 1j * rng.normal(size=(3, ny, nx)) for k in names}
+    base = {k: rng.normal(size=(ny, nx)) for k in ("uxb", "uyb", "wzb", "varg", "dvargdx")}
+    kphys = 8 if form == "nonlinear" else 0
+    Re = 1e4
+    p = oracle.make_params(g.nx, g.ny, g.nmodes, g.levels, g.dx, g.dy0, g.stf, g.alpha, g.beta)
+    ref = oracle.drv_fi(p, Re, 0, base, F) if form == "flat plate" else oracle.drv_gv(p, Re, kphys, base, F)
+    with context(g) as ctx:
+        d = {k: torch.from_numpy(F[k]).to("cuda") for k in names}
+        keep = {k: torch.from_numpy(base[k]).to("cuda") for k in base}
+        db = {k: keep[k].data_ptr() for k in base}
+        out = [torch.full_like(d["ux"], 7.0) for _ in range(3)]
+        first = [7.0] * 3
+        if form == "in place":
+            out[0], out[2] = d["wx"], d["wz"]
+            first = [F["wx"][:, 0], 7.0, F["wz"][:, 0]]
+        call = ctx.drv_fi_dev if form == "flat plate" else ctx.drv_gv_dev
+        call(Re, kphys, db, *[d[k].data_ptr() for k in names], *[o.data_ptr() for o in out])
+        ctx.synchronize()
+        got = [o.cpu().numpy() for o in out]
+    for q in range(3):
+        assert np.all(got[q][:, 0] == first[q])
+        assert rel(got[q][:, 1:], ref[q][:, 1:]) < 1e-12, "xyz"[q]

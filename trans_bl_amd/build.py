@@ -46,6 +46,7 @@ SOURCES = [
     "tbl_xline.hip",
     "tbl_loop.cpp",
     "tbl_rhs.hip",
+    "tbl_drv.hip",
     "tbl_rk4.cpp",
 ]
 

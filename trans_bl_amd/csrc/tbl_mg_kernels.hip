@@ -519,6 +519,7 @@ int set_kernel_attributes()
     if (rc == TBL_OK) rc = deriv_kernel_attributes();
     if (rc == TBL_OK) rc = xline_kernel_attributes();
     if (rc == TBL_OK) rc = rhs_kernel_attributes();
+    if (rc == TBL_OK) rc = drv_kernel_attributes();
     return rc;
 }
 

@@ -1,7 +1,7 @@
 // Argument blocks and launchers of the right-hand-side kernels (tbl_rhs.hip).
 #pragma once
 
-#include "tbl_common.h"
+#include "tbl_kernels.h"
 
 namespace tbl {
 
@@ -21,10 +21,11 @@ struct RhsArgs {
 
 struct DrvArgs {
     BaseArgs b;
-    const cx<double> *wx, *wy, *wz, *bb, *c, *d;
+    const cx<double> *ux, *uy, *wx, *wy, *wz, *a, *bb, *c, *d;
+    // drv_combine only
     const cx<double> *dadx, *dbdx, *dddx, *dady, *dcdy;
     const cx<double> *xx, *yx, *zx, *xy, *yy, *zy;    // d2w/dx2, d2w/dy2 of wx, wy, wz
-    cx<double> *dvx, *dvy, *dvz;
+    cx<double> *dv[3];
     double rre, fac_y, beta;
     int nx, ny, K;
     int fi;                    // drv_fi: no curvature terms (d, dddx, varg unused)
@@ -40,6 +41,12 @@ struct RkArgs {
 bool nlterms_fits(int K, int N);   // kphys values the nonlinear terms accept
 int terms(const RhsArgs &r, int kphys, hipStream_t st);
 int drv_combine(const DrvArgs &r, hipStream_t st);
+// the derivatives and the combination in six launches (tbl_drv.hip); lin: the
+// terms from the fields and the base flow (Goertler form), else a, bb, c, d;
+// dv may alias none of the inputs
+bool drv_fused_fits(const DerivArgs &A);
+int drv_fused(const DerivArgs &A, const DrvArgs &r, bool lin, hipStream_t st);
+int drv_kernel_attributes();
 int rk_update(const RkArgs &r, hipStream_t st);
 int pert_rows(cx<double> *uy, cx<double> *d2, const cx<double> *pu, const cx<double> *pd,
               int nx, int ny, int K, int i0, int i1, hipStream_t st);

@@ -304,17 +304,17 @@ __global__ void drv_combine_kernel(DrvArgs r)
     const double rre = r.rre, fy = r.fac_y;
     if (r.fi) {
         // drv_fi's combination (main_par.f:1317-1331): no curvature terms
-        r.dvx[e] = -r.dady[e] + mul_i(kb, r.bb[e]) + rre * (r.xx[e] + fy * r.xy[e] + k2 * r.wx[e]);
-        r.dvy[e] = -mul_i(kb, r.c[e]) + r.dadx[e] + rre * (r.yx[e] + fy * r.yy[e] + k2 * r.wy[e]);
-        r.dvz[e] = -r.dbdx[e] + r.dcdy[e] + rre * (r.zx[e] + fy * r.zy[e] + k2 * r.wz[e]);
+        r.dv[0][e] = -r.dady[e] + mul_i(kb, r.bb[e]) + rre * (r.xx[e] + fy * r.xy[e] + k2 * r.wx[e]);
+        r.dv[1][e] = -mul_i(kb, r.c[e]) + r.dadx[e] + rre * (r.yx[e] + fy * r.yy[e] + k2 * r.wy[e]);
+        r.dv[2][e] = -r.dbdx[e] + r.dcdy[e] + rre * (r.zx[e] + fy * r.zy[e] + k2 * r.wz[e]);
         return;
     }
     const double vg = r.b.varg[e2], dvg = r.b.dvargdx[e2];
     const cxd d = r.d[e];
-    r.dvx[e] = -r.dady[e] + mul_i(kb, r.bb[e]) - vg * mul_i(kb, d)
+    r.dv[0][e] = -r.dady[e] + mul_i(kb, r.bb[e]) - vg * mul_i(kb, d)
                + rre * (r.xx[e] + fy * r.xy[e] + k2 * r.wx[e]);
-    r.dvy[e] = -mul_i(kb, r.c[e]) + r.dadx[e] + rre * (r.yx[e] + fy * r.yy[e] + k2 * r.wy[e]);
-    r.dvz[e] = -r.dbdx[e] + r.dcdy[e] + vg * r.dddx[e] + dvg * d
+    r.dv[1][e] = -mul_i(kb, r.c[e]) + r.dadx[e] + rre * (r.yx[e] + fy * r.yy[e] + k2 * r.wy[e]);
+    r.dv[2][e] = -r.dbdx[e] + r.dcdy[e] + vg * r.dddx[e] + dvg * d
                + rre * (r.zx[e] + fy * r.zy[e] + k2 * r.wz[e]);
 }
 

@@ -1,11 +1,12 @@
 // Right-hand side (drv_gv with lterms_gv or nlterms_gv) and the RK4 time
 // step of the reference's Goertler case on the GPU: host side -- work
-// fields, the z-DFT twiddle table, the launch sequence of drv_gv (terms,
-// the eleven derivatives as seven derivative calls, the combination) and
+// fields, the z-DFT twiddle table, the launch sequence of drv_gv (nonlinear
+// terms, then the derivatives and their combination per component) and
 // of the four RK4 stages around tbl_loop_dev (main_par.f:266-349); and
 // drv_fi, the flat-plate form (main_par.f:1264-1336: lterms_fi /
 // nlterms_fi, ten derivatives, the combination without curvature terms).
 #include <cmath>
+#include <cstdint>
 #include <vector>
 
 #include "tbl_ctx.h"
@@ -88,6 +89,28 @@ int do_terms(tbl_ctx *c, int kphys, const tbl_base *b, const double *const *f,
     return TBL_OK;
 }
 
+// does an output share memory with an input or another output?
+bool dv_overlaps(const tbl_ctx *c, const tbl_base *b, const double *const *f, cx<double> *const *dv)
+{
+    const size_t nf = field(c) * sizeof(cx<double>);
+    const size_t nb = static_cast<size_t>(c->g.nx) * c->g.ny * sizeof(double);
+    auto apart = [](const void *p, size_t np, const void *q, size_t nq) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(p), y = reinterpret_cast<uintptr_t>(q);
+        return !p || x + np <= y || y + nq <= x;
+    };
+    const BaseArgs a = base_of(b);
+    const double *base[5] = {a.uxb, a.uyb, a.wzb, a.varg, a.dvargdx};
+    for (int q = 0; q < 3; ++q) {
+        for (int p = 0; p < 6; ++p)
+            if (!apart(f[p], nf, dv[q], nf)) return true;
+        for (int p = 0; p < 5; ++p)
+            if (!apart(base[p], nb, dv[q], nf)) return true;
+        for (int p = 0; p < q; ++p)
+            if (!apart(dv[p], nf, dv[q], nf)) return true;
+    }
+    return false;
+}
+
 // drv_gv (main_par.f:1339-1403), or with fi drv_fi (main_par.f:1264-1336):
 // f = ux, uy, uz, wx, wy, wz; dv = dvx, dvy, dvz
 int drv_gv(tbl_ctx *c, double Re, int kphys, const tbl_base *b, const double *const *f,
@@ -97,28 +120,49 @@ int drv_gv(tbl_ctx *c, double Re, int kphys, const tbl_base *b, const double *co
     const size_t n = field(c);
     cx<double> *w[15];
     for (int q = 0; q < 15; ++q) w[q] = c->d_rhs + q * n;
-    cx<double> *a = w[0], *bb = w[1], *cc = w[2], *d = w[3];
-    TRY(do_terms(c, kphys, b, f, w, fi));
-    auto D = [](cx<double> *p) { return reinterpret_cast<double *>(p); };
     const DerivArgs &A = c->dargs;
     hipStream_t st = c->stream;
-    // a: d/dx, d/dy; b, d (not in drv_fi): d/dx; c: d/dy; wx, wy, wz:
-    // d2/dx2, d2/dy2
-    TRY(derivs4(A, D(a), D(w[4]), nullptr, D(w[7]), nullptr, st));
-    TRY(derivs4(A, D(bb), D(w[5]), nullptr, nullptr, nullptr, st));
-    if (!fi) TRY(derivs4(A, D(d), D(w[6]), nullptr, nullptr, nullptr, st));
-    TRY(derivs4(A, D(cc), nullptr, nullptr, D(w[8]), nullptr, st));
-    TRY(derivs4(A, f[3], nullptr, D(w[9]), nullptr, D(w[12]), st));
-    TRY(derivs4(A, f[4], nullptr, D(w[10]), nullptr, D(w[13]), st));
-    TRY(derivs4(A, f[5], nullptr, D(w[11]), nullptr, D(w[14]), st));
     DrvArgs r{};
     r.b = base_of(b);
+    r.ux = C(f[0]);
+    r.uy = C(f[1]);
     r.wx = C(f[3]);
     r.wy = C(f[4]);
     r.wz = C(f[5]);
-    r.bb = bb;
-    r.c = cc;
-    r.d = d;
+    r.a = w[0];
+    r.bb = w[1];
+    r.c = w[2];
+    r.d = w[3];
+    for (int q = 0; q < 3; ++q) r.dv[q] = dv[q];
+    r.fi = fi ? 1 : 0;
+    r.rre = 1.0 / Re;
+    r.fac_y = c->g.fac_y;
+    r.beta = c->g.beta;
+    r.nx = c->g.nx;
+    r.ny = c->g.ny;
+    r.K = c->K;
+    if (drv_fused_fits(A) && !dv_overlaps(c, b, f, dv)) {
+        const bool lin = kphys == 0 && !fi;
+        if (!lin) TRY(do_terms(c, kphys, b, f, w, fi));
+        TRY(drv_fused(A, r, lin, st));
+        TBL_HIP(hipGetLastError());
+        return TBL_OK;
+    }
+    // every derivative in a field of its own: y-lines too long for the fused
+    // kernels, or an output in the place of an input
+    auto D = [](const cx<double> *p) {
+        return reinterpret_cast<double *>(const_cast<cx<double> *>(p));
+    };
+    TRY(do_terms(c, kphys, b, f, w, fi));
+    // a: d/dx, d/dy; b, d (not in drv_fi): d/dx; c: d/dy; wx, wy, wz:
+    // d2/dx2, d2/dy2
+    TRY(derivs4(A, D(r.a), D(w[4]), nullptr, D(w[7]), nullptr, st));
+    TRY(derivs4(A, D(r.bb), D(w[5]), nullptr, nullptr, nullptr, st));
+    if (!fi) TRY(derivs4(A, D(r.d), D(w[6]), nullptr, nullptr, nullptr, st));
+    TRY(derivs4(A, D(r.c), nullptr, nullptr, D(w[8]), nullptr, st));
+    TRY(derivs4(A, f[3], nullptr, D(w[9]), nullptr, D(w[12]), st));
+    TRY(derivs4(A, f[4], nullptr, D(w[10]), nullptr, D(w[13]), st));
+    TRY(derivs4(A, f[5], nullptr, D(w[11]), nullptr, D(w[14]), st));
     r.dadx = w[4];
     r.dbdx = w[5];
     r.dddx = w[6];
@@ -130,16 +174,6 @@ int drv_gv(tbl_ctx *c, double Re, int kphys, const tbl_base *b, const double *co
     r.xy = w[12];
     r.yy = w[13];
     r.zy = w[14];
-    r.dvx = dv[0];
-    r.dvy = dv[1];
-    r.dvz = dv[2];
-    r.fi = fi ? 1 : 0;
-    r.rre = 1.0 / Re;
-    r.fac_y = c->g.fac_y;
-    r.beta = c->g.beta;
-    r.nx = c->g.nx;
-    r.ny = c->g.ny;
-    r.K = c->K;
     TRY(drv_combine(r, st));
     TBL_HIP(hipGetLastError());
     return TBL_OK;

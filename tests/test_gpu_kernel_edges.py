@@ -77,6 +77,26 @@ def test_derivatives_at_every_shape(torch_mod, nx, ny):
         assert rel(v, oracle.deriv(p, kind, f)) < 1e-12, kind
 
 
+@pytest.mark.parametrize("nx, ny, nmodes", [(17, 9, 1), (129, 33, 4), (193, 65, 3), (321, 97, 5), (449, 113, 2), (577, 143, 1)],
+                         ids=lambda v: str(v))
+def test_derivatives_of_small_grids_in_one_launch(torch_mod, nx, ny, nmodes):
+    """All four derivatives in one launch against a launch per direction: the
+    same arithmetic, equal to the bit."""
+    torch = torch_mod
+    g = wl.Grid(nx, ny, nmodes, 2, 0.02, 1e-3, 1.004, 0.0, 0.3)
+    rng = np.random.default_rng(nx * ny)
+    f = rng.normal(size=(nmodes, ny, nx)) + 1j * rng.normal(size=(nmodes, ny, nx))
+    with context(g) as ctx:
+        fd = torch.from_numpy(f).to("cuda")
+        one, two = ([torch.zeros_like(fd) for _ in range(4)] for _ in range(2))
+        p = [o.data_ptr() for o in two]
+        ctx.derivs_dev(fd.data_ptr(), *[o.data_ptr() for o in one])
+        ctx.derivs_dev(fd.data_ptr(), p[0], p[1], 0, 0)
+        ctx.derivs_dev(fd.data_ptr(), 0, 0, p[2], p[3])
+        ctx.synchronize()
+        for a, b in zip(one, two):
+            assert torch.equal(a, b) and torch.any(a != 0)
+
 
 @pytest.mark.parametrize("n, H, W", [(2, 8, 8), (3, 8, 40), (1, 40, 56), (2, 32, 136), (1, 16, 264), (1, 8, 1024)],
                          ids=lambda v: str(v))

@@ -43,8 +43,7 @@ namespace tbl {
 // From 3 wavefronts per part the registers are held to 4 wavefronts a SIMD: two
 // workgroups a CU (2049x257x32: 276 -> 198 us; below that it only spilled).
 template <int R, int W, bool D1, bool D2>
-__global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
-    deriv_x_kernel(DerivArgs A, const C *__restrict__ f, C *__restrict__ o1, C *__restrict__ o2)
+__device__ __forceinline__ void deriv_x_line(const DerivArgs &A, int block, const C *f, C *o1, C *o2)
 {
     constexpr int NT = 128 * W, N = (R + 1) / 2, LP = 64 * R * W + 4;
     __shared__ double planes[2 * LP], maps[16 * W], tab[kXTab];
@@ -52,7 +51,7 @@ __global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int part = wv / W, w = wv % W;
     const int nx = A.nx;
-    const size_t line = static_cast<size_t>(blockIdx.x) * nx;
+    const size_t line = static_cast<size_t>(block) * nx;
     {
         const __amdgpu_buffer_rsrc_t fr = buf_rsrc(f + line, static_cast<size_t>(nx) * sizeof(C));
         C v[N];
@@ -96,6 +95,13 @@ __global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
     if constexpr (D2) out(b, o2);
 }
 
+template <int R, int W, bool D1, bool D2>
+__global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
+    deriv_x_kernel(DerivArgs A, const C *__restrict__ f, C *__restrict__ o1, C *__restrict__ o2)
+{
+    deriv_x_line<R, W, D1, D2>(A, static_cast<int>(blockIdx.x), f, o1, o2);
+}
+
 // y-lines: o1 = d/dy (fv: with the wall row forced, deryfv), o2 = d2/dy2 of f.
 // Workgroup: 8 columns x all rows of one mode, both parts, in LDS (column
 // stride LP, 4 past a multiple of 32 values: the 8 columns x 4 rows of half a
@@ -106,9 +112,8 @@ __global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
 // offset from the lane's first.  The stores do not stream: a row's 128 bytes
 // are rarely one cache line (with nt 8 of 9 sizes were up to 50 % slower).
 template <int G, int R, bool D1, bool D2>
-__global__ void __launch_bounds__(16 * G) deriv_y_kernel(DerivArgs A, const C *__restrict__ f,
-                                                         C *__restrict__ o1, int fv,
-                                                         C *__restrict__ o2)
+__device__ __forceinline__ void deriv_y_tile(const DerivArgs &A, int block, const C *f, C *o1, int fv,
+                                             C *o2)
 {
     constexpr int TX = kDerivYCols, NT = 2 * TX * G, N = (R + 1) / 2, M = G * R, LP = M + 4;
     constexpr int NTAB = 6 * M + 64;
@@ -121,7 +126,7 @@ __global__ void __launch_bounds__(16 * G) deriv_y_kernel(DerivArgs A, const C *_
     // at their boundary -- run on one XCD and share its L2
     const int tiles_x = (nx + TX - 1) / TX;
     const int B = tiles_x * A.K, per = (B + 7) / 8;
-    const int m = static_cast<int>(blockIdx.x % 8) * per + static_cast<int>(blockIdx.x / 8);
+    const int m = block % 8 * per + block / 8;
     if (m >= B) return;
     const int x0 = (m % tiles_x) * TX, k = m / tiles_x;
     const size_t plane = static_cast<size_t>(nx) * ny, mb = plane * k;
@@ -167,6 +172,29 @@ __global__ void __launch_bounds__(16 * G) deriv_y_kernel(DerivArgs A, const C *_
     if constexpr (D1) out(a, o1);
     if constexpr (D1 && D2) __syncthreads();
     if constexpr (D2) out(b, o2);
+}
+
+template <int G, int R, bool D1, bool D2>
+__global__ void __launch_bounds__(16 * G) deriv_y_kernel(DerivArgs A, const C *__restrict__ f,
+                                                         C *__restrict__ o1, int fv,
+                                                         C *__restrict__ o2)
+{
+    deriv_y_tile<G, R, D1, D2>(A, static_cast<int>(blockIdx.x), f, o1, fv, o2);
+}
+
+// all four derivatives of a small grid in one launch: the first ybs blocks (a
+// multiple of 8) are y-tiles, the others x-lines of one wavefront per part (the
+// blocks' other wavefronts leave before any barrier)
+template <int RX, int RY>
+__global__ void __launch_bounds__(256) deriv_both_kernel(DerivArgs A, int ybs, const C *__restrict__ f,
+                                                         C *__restrict__ dx, C *__restrict__ dxx,
+                                                         C *__restrict__ dy, C *__restrict__ dyy)
+{
+    const int block = static_cast<int>(blockIdx.x);
+    if (block < ybs)
+        deriv_y_tile<16, RY, true, true>(A, block, f, dy, 0, dyy);
+    else if (threadIdx.x < 128)
+        deriv_x_line<RX, 1, true, true>(A, block - ybs, f, dx, dxx);
 }
 
 // y-lines of more than 64 * 9 rows: one thread per column, the forward sweep
@@ -284,6 +312,12 @@ int deriv_y_rows(int ny, int *G, int *R)
     return *G * *R;
 }
 
+// bytes of LDS of a y workgroup: the tile's planes and the tables
+static size_t y_lds(int rows)
+{
+    return (static_cast<size_t>(2 * kDerivYCols) * (rows + 4) + 6 * rows + 64) * sizeof(double);
+}
+
 static int deriv_y(const DerivArgs &A, const C *f, C *o1, int fv, C *o2, hipStream_t st)
 {
     int G, R;
@@ -296,8 +330,7 @@ static int deriv_y(const DerivArgs &A, const C *f, C *o1, int fv, C *o2, hipStre
     }
     const int tiles = (A.nx + kDerivYCols - 1) / kDerivYCols * A.K;
     const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8));
-    const size_t lds =
-        (static_cast<size_t>(2 * kDerivYCols) * (rows + 4) + 6 * rows + 64) * sizeof(double);
+    const size_t lds = y_lds(rows);
 #define X(GG, RR)                                                                               \
     if (G == GG && R == RR) {                                                                   \
         const dim3 block(16 * GG);                                                              \
@@ -331,11 +364,46 @@ int deriv(const DerivArgs &A, int kind, const double *f, double *out, hipStream_
     }
 }
 
+// Small grids take all four derivatives in one launch: a launch costs 3-5 us of
+// latency whatever its size, and the two kinds of blocks share the chip's last
+// wave.  Two launches -> one, us: 65x33x2 7.4 -> 4.4, 129x33x4 8.3 -> 4.6,
+// 385x97x8 14.2 -> 10.7, 513x129x16 (3104 blocks) 29.4 -> 23.7, 513x129x32
+// (6208) 46.1 -> 41.0, 513x129x64 (12416) 77.2 -> 76.3; from there on nothing or
+// a loss (129x129x256, 37376: 103 -> 121), the larger kernel's registers and LDS
+// cost occupancy.  Longer lines' x-blocks would leave half of a y-block's
+// threads' registers idle: they keep their own launches.
+constexpr int kBothBlocks = 8192;
+static bool derivs_both(const DerivArgs &A, const C *f, C *dx, C *dxx, C *dy, C *dyy, hipStream_t st)
+{
+    int RX, W, G, RY;
+    const int rows = deriv_y_rows(A.ny, &G, &RY);
+    if (!x_shape(A.nx, &RX, &W) || W != 1 || G != 16) return false;
+    const long tiles = (A.nx + kDerivYCols - 1) / kDerivYCols * static_cast<long>(A.K);
+    const long ybs = (tiles + 7) / 8 * 8, blocks = ybs + static_cast<long>(A.ny) * A.K;
+    if (blocks > kBothBlocks) return false;
+    const size_t lds = y_lds(rows);
+#define XY(RRX, RRY)                                                                              \
+    if (RX == RRX && RY == RRY) {                                                                 \
+        hipLaunchKernelGGL((deriv_both_kernel<RRX, RRY>), dim3(static_cast<unsigned>(blocks)),    \
+                           dim3(256), lds, st, A, static_cast<int>(ybs), f, dx, dxx, dy, dyy);    \
+        return true;                                                                              \
+    }
+#define X(RRX) XY(RRX, 3) XY(RRX, 5) XY(RRX, 7) XY(RRX, 9)
+    X(2) X(3) X(5) X(7) X(9)
+#undef X
+#undef XY
+    return false;
+}
+
 int derivs4(const DerivArgs &A, const double *f, double *dx, double *dxx, double *dy, double *dyy,
             hipStream_t st)
 {
     const C *fi = reinterpret_cast<const C *>(f);
     int rc = TBL_OK;
+    if (dx && dxx && dy && dyy &&
+        derivs_both(A, fi, reinterpret_cast<C *>(dx), reinterpret_cast<C *>(dxx),
+                    reinterpret_cast<C *>(dy), reinterpret_cast<C *>(dyy), st))
+        return TBL_OK;
     if (dx || dxx)
         rc = deriv_x(A, fi, reinterpret_cast<C *>(dx), reinterpret_cast<C *>(dxx), st);
     if (rc == TBL_OK && (dy || dyy))

@@ -213,3 +213,28 @@ def test_right_hand_side_at_every_shape(torch_mod, nx, ny, form):
     for q in range(3):
         assert np.all(got[q][:, 0] == first[q])
         assert rel(got[q][:, 1:], ref[q][:, 1:]) < 1e-12, "xyz"[q]
+
+
+@pytest.mark.parametrize("g", [
+    wl.Grid(65, 33, 3, 4, 0.05, 2e-3, 1.03, 0.0, 0.9),      # strips of 2 columns, one row chunk
+    wl.Grid(89, 41, 2, 4, 0.05, 1e-3, 1.03, 0.1, 0.7),
+    wl.Grid(145, 117, 2, 3, 0.03, 3e-4, 1.015, 0.0, 0.3),   # 116 rows: two full chunks
+    wl.Grid(145, 121, 2, 3, 0.03, 3e-4, 1.015, 0.0, 0.3),   # two rows in the third
+    wl.Grid(609, 65, 40, 3, 0.02, 5e-4, 1.02, 0.0, 0.3)],   # strips of 32 and a rest
+    ids=lambda g: f"{g.nx}x{g.ny}x{g.nmodes}l{g.levels}")
+def test_fas_cycles_match_oracle(torch_mod, g):
+    """Two FP64 cycles, wall and boundary columns non-zero (they are injected
+    too), against the oracle in the same line order: iterates to 1e-10 (last-bit
+    differences of some 600 line solves, each of condition up to 1e4), the checks'
+    largest defects to 1e-5 (differences of values up to 1e6 times as large)."""
+    p = oracle.make_params(g.nx, g.ny, g.nmodes, g.levels, g.dx, g.dy0, g.stf, g.alpha, g.beta)
+    f = wl.wavepacket_rhs(g, tag="fas")
+    u = 0.01 * wl.wavepacket_rhs(g, tag="fas-start")
+    u[:, 0, :] = 0.003
+    u[:, :, 0] = 0.002
+    u[:, :, -1] = -0.001
+    with context(g) as ctx:
+        got, _, res = ctx.poi_uy(None, -f, u, 0.0, max_cycles=2)[:3]
+    ref, _, rres = oracle.poi_uy(p, np.zeros_like(f), -f, u, 0.0, max_cycles=2, order=1)
+    assert rel(got, ref) < 1e-10, rel(got, ref)
+    assert rel(res, rres) < 1e-5, rel(res, rres)

@@ -48,12 +48,19 @@ constexpr int kDefBlock = sizeof(T) == 4 ? 8 : 2;
 
 // columns per strip: longer strips load fewer halo columns; the mixed
 // defect (FP64 in, FP32 out) was measured fastest at 64 on nx = 1025, the
-// others at 32
+// others at 32.  Small levels take shorter strips, down to 2 columns, until
+// there are kDefWaves wavefronts (`waves` per strip): the march is a chain of
+// load latencies, one per block of columns (385x97x8 and its coarser levels,
+// FP64: 16.7 -> 4.7 us per launch of the plain form; the solve 5.03 -> 4.63 ms
+// with the one-pass form above).
+constexpr int kDefWaves = 1024;
 template <typename T, typename TO>
-__host__ __device__ inline int defect_strip(int nx)
+static int defect_strip(int nx, int waves)
 {
-    if (sizeof(T) == 8 && sizeof(TO) == 4 && nx >= 1024) return 64;
-    return nx >= 512 ? 32 : 16;
+    int strip = sizeof(T) == 8 && sizeof(TO) == 4 && nx >= 1024 ? 64 : nx >= 512 ? 32 : 16;
+    while (strip > 2 && static_cast<long>(waves) * ((nx - 2 + strip - 1) / strip) < kDefWaves)
+        strip /= 2;
+    return strip;
 }
 
 // The restricting form (RS): the defect's full-weighting restriction onto
@@ -61,11 +68,16 @@ __host__ __device__ inline int defect_strip(int nx)
 // wavefronts own kDefRowsRs rows with three halo rows each side, so the
 // defect is formed on one halo row each side as well and every even fine
 // row has its two neighbours' defects in the wavefront; each strip walks
-// one column past its end for the same reason in x.
+// one column past its end for the same reason in x.  The FP64 form (the FAS
+// cycle) injects v as well, into the coarser v and its copy, from the columns
+// the march holds: 2 passes over a level read and 3/4 of one written, against
+// 4.5 and 1.75 with the stored defect and restrict_kernel.  Plain FP64 solve of
+// 1025x193x64: 13.7 -> 12.6 ms.
 constexpr int kDefRowsRs = 58;
 template <typename T>
 struct CoarseOut {
     cx<T> *S;              // the coarser level's source (nullptr: plain defect)
+    cx<T> *V, *W;          // FP64: the coarser level's v and its copy
     int nx, ny, ld;
     size_t plane;
 };
@@ -82,6 +94,7 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
     // out: no reference counterpart); the FP64 defect rounds as written
     constexpr bool kFuse = sizeof(T) == 4 || sizeof(TO) == 4;
     constexpr int kRows = RS ? kDefRowsRs : kDefRows, kHalo = RS ? 3 : 2;
+    constexpr bool kInj = RS && sizeof(T) == 8;
     const int lane = threadIdx.x & 63;
     const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int k = blockIdx.y;
@@ -128,7 +141,7 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
     // the restricting form holds two more row sums: 4 columns per block keep
     // it at 96 registers, five wavefronts per SIMD (three at 8; measured
     // 7.26 -> 7.18 ms per 1025x193x64 mixed solve)
-    constexpr int B = RS ? 4 : kDefBlock<T>;
+    constexpr int B = RS && sizeof(T) == 4 ? 4 : kDefBlock<T>;
     // win[t] = column i0 - 2 + t of the current block (i0 .. i0+B-1 computed),
     // sq[t] = source column i0 + t; nb / ns: the next block's new columns
     cx<T> win[B + 4], sq[B], nb[B], ns[B];
@@ -139,6 +152,16 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
 #pragma unroll
     for (int t = 0; t < B; ++t) sq[t] = sload(ia + t);
     double amax = 0.0;
+    // restrict's injection of fine column i (even) to the coarser level, wall
+    // row and boundary columns included
+    const bool inj = kInj && (own || j == 0) && !(j & 1);
+    auto inject = [&](int i, cx<T> v) {
+        if (!inj) return;
+        const size_t o = static_cast<size_t>(k) * co.plane + static_cast<size_t>(i >> 1) * co.ld + (j >> 1);
+        co.V[o] = cx<TO>{static_cast<TO>(v.re), static_cast<TO>(v.im)};
+        co.W[o] = cx<TO>{static_cast<TO>(v.re), static_cast<TO>(v.im)};
+    };
+    if (kInj && ia == 1) inject(0, win[1]);
     for (int i0 = ia; i0 < ib; i0 += B) {
         if (i0 + B < ib) {
 #pragma unroll
@@ -213,12 +236,16 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
                 const cx<T> r = mac_f<kFuse>(si, lv, s_cur);   // s + si lv
                 rv = r;
                 if (!RS) out[o] = cx<TO>{static_cast<TO>(r.re), static_cast<TO>(r.im)};
-                if (!RS && resmax) {
+                if ((!RS || kInj) && resmax) {
                     // max of |r|^2; one square root per wavefront below
                     // (sqrt is monotone and correctly rounded: same maximum)
                     const double rr = static_cast<double>(r.re), ri = static_cast<double>(r.im);
                     amax = fmax(amax, rr * rr + ri * ri);
                 }
+            }
+            if constexpr (kInj) {
+                if (!(i & 1) && i < ib0) inject(i, w2);
+                if (i == nx - 2) inject(nx - 1, w3);
             }
             if constexpr (RS) {
                 // restrict_kernel's full weighting, separated: the row sum
@@ -565,9 +592,9 @@ template <typename T, typename TO>
 void defect(const LevelArgs<T> &L, const cx<T> *V, const cx<T> *S, cx<TO> *out, T si,
             const int *active, double *resmax, hipStream_t st)
 {
-    const int strip = defect_strip<T, TO>(L.nx);
-    const int nstrips = (L.nx - 2 + strip - 1) / strip;
     const int jchunks = (L.ny - 1 + kDefRows - 1) / kDefRows;
+    const int strip = defect_strip<T, TO>(L.nx, jchunks * L.K);
+    const int nstrips = (L.nx - 2 + strip - 1) / strip;
     const int blocks = (nstrips * jchunks + 3) / 4;
     hipLaunchKernelGGL((defect_march_kernel<T, TO>), dim3(blocks, L.K), dim3(256), 0, st, L, V, S,
                        out, si, active, resmax, strip, nstrips, jchunks, CoarseOut<TO>{});
@@ -575,16 +602,16 @@ void defect(const LevelArgs<T> &L, const cx<T> *V, const cx<T> *S, cx<TO> *out, 
 
 template <typename T>
 void defect_restrict(const LevelArgs<T> &L, const Level &Cl, const cx<T> *V, const cx<T> *S,
-                     cx<T> *Sc, const int *active, hipStream_t st)
+                     cx<T> *Vc, cx<T> *Wc, cx<T> *Sc, const int *active, double *resmax,
+                     hipStream_t st)
 {
-    const int strip = defect_strip<T, T>(L.nx);   // even: strips start on odd columns
-    const int nstrips = (L.nx - 2 + strip - 1) / strip;
     const int jchunks = (L.ny - 1 + kDefRowsRs - 1) / kDefRowsRs;
+    const int strip = defect_strip<T, T>(L.nx, jchunks * L.K);   // even: strips start on odd columns
+    const int nstrips = (L.nx - 2 + strip - 1) / strip;
     const int blocks = (nstrips * jchunks + 3) / 4;
-    const CoarseOut<T> co{Sc, Cl.nx, Cl.ny, Cl.ld, Cl.plane};
+    const CoarseOut<T> co{Sc, Vc, Wc, Cl.nx, Cl.ny, Cl.ld, Cl.plane};
     hipLaunchKernelGGL((defect_march_kernel<T, T, true>), dim3(blocks, L.K), dim3(256), 0, st, L,
-                       V, S, static_cast<cx<T> *>(nullptr), T(-1), active,
-                       static_cast<double *>(nullptr), strip, nstrips, jchunks, co);
+                       V, S, static_cast<cx<T> *>(nullptr), T(-1), active, resmax, strip, nstrips, jchunks, co);
 }
 
 template <typename T>
@@ -670,8 +697,12 @@ template void defect<double, float>(const LevelArgs<double> &, const cx<double> 
                                     hipStream_t);
 template void defect<float, float>(const LevelArgs<float> &, const cx<float> *, const cx<float> *,
                                    cx<float> *, float, const int *, double *, hipStream_t);
+template void defect_restrict<double>(const LevelArgs<double> &, const Level &, const cx<double> *,
+                                      const cx<double> *, cx<double> *, cx<double> *, cx<double> *,
+                                      const int *, double *, hipStream_t);
 template void defect_restrict<float>(const LevelArgs<float> &, const Level &, const cx<float> *,
-                                     const cx<float> *, cx<float> *, const int *, hipStream_t);
+                                     const cx<float> *, cx<float> *, cx<float> *, cx<float> *,
+                                     const int *, double *, hipStream_t);
 template void restrict_level<double>(const Level &, const Level &, int, const cx<double> *,
                                      const cx<double> *, cx<double> *, cx<double> *, cx<double> *,
                                      int, const int *, hipStream_t);

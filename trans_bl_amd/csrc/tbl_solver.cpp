@@ -451,14 +451,14 @@ int fas_cycle(tbl_ctx *c, const Sched &s, double tol)
     for (int l = 0; l < L - 1; ++l) {
         TRY(smooth_sweeps<double>(c->la_d[l], c->V[l], c->S[l], c->lu_d[l], s.nu1, rf_of(s.nu1),
                                   c->d_active, c->G64[l], c->H64[l], st));
-        defect<double, double>(c->la_d[l], c->V[l], c->S[l], c->R[l], -1.0, c->d_active,
-                               l == 0 ? c->d_resmax : nullptr, st);
+        // the defect's restriction and the injected v in one pass (modes that the
+        // check below stops leave their coarser levels unused)
+        defect_restrict<double>(c->la_d[l], c->lv[l + 1], c->V[l], c->S[l], c->V[l + 1], c->W[l + 1],
+                                c->S[l + 1], c->d_active, l == 0 ? c->d_resmax : nullptr, st);
         if (l == 0)
             hipLaunchKernelGGL(decide2_kernel, dim3((K + 255) / 256), dim3(256), 0, st, K,
                                c->d_resmax, tol, c->d_cycle, c->d_active, c->d_cycles,
                                c->d_lastres, c->d_nactive);
-        restrict_level<double>(c->lv[l], c->lv[l + 1], K, c->V[l], c->R[l], c->V[l + 1],
-                               c->W[l + 1], c->S[l + 1], 1, c->d_active, st);
         defect<double, double>(c->la_d[l + 1], c->V[l + 1], c->S[l + 1], c->S[l + 1], 1.0,
                                c->d_active, nullptr, st);
     }
@@ -513,8 +513,8 @@ int correction_vcycle(tbl_ctx *c, const Sched &s, std::vector<cx<float> *> &e, i
         // the coarser source is the restricted defect (one pass, no stored
         // defect); the coarser e starts from zero -- cleared here unless its
         // first sweep starts from zero by itself
-        defect_restrict<float>(c->la_f[l], c->lv[l + 1], e[l], c->S32[l], c->S32[l + 1],
-                               c->d_active, st);
+        defect_restrict<float>(c->la_f[l], c->lv[l + 1], e[l], c->S32[l], nullptr, nullptr,
+                               c->S32[l + 1], c->d_active, nullptr, st);
         if (!zero_start(l + 1))
             convert<float, float>(c->lv[l + 1].plane * K, e[l + 1], e[l + 1], 1, st);
     }

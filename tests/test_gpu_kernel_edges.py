@@ -145,6 +145,37 @@ def test_network_gradients_at_image_shapes(torch_mod, n, H, W):
         assert np.array_equal(g, again)           # no atomics in the direct forms
 
 
+@pytest.mark.parametrize("n, H, W", [(1, 8, 8), (37, 24, 152), (3, 40, 152), (1, 8, 160)], ids=lambda v: str(v))
+def test_network_forward_at_image_shapes(torch_mod, n, H, W):
+    """Outputs against the numpy network: a tile that one image does not fill,
+    two tiles per wavefront with a rest, the widest image of the staged form
+    and one past it.  Weights and inputs as in the gradients' test: every value
+    before a bf16 rounding is exact in both, so the outputs agree to the fp32
+    sum over 32 channels (1e-6)."""
+    torch = torch_mod
+    from oracle import unet_ref as U
+    from trans_bl_amd import guess
+    rng = np.random.default_rng(H * W + n)
+    x = rng.integers(0, 5, size=(n, H, W, 4)).astype(np.float32)
+    theta = []
+    for name, cin, cout, ks, lvl, relu in U.layers():
+        w = np.zeros((ks * ks, cin, cout))
+        o = np.arange(cout)
+        tap = np.where(o % 2 > 0, ks * ks // 2, rng.integers(0, ks * ks, cout))
+        w[tap, 3 * o % cin, o] = 1.0
+        if name == "OUT":
+            w[:] = 1.0                            # the gradient reaches every layer
+        theta += [w.ravel(), rng.integers(0, 2, cout)]
+    theta = np.concatenate(theta)
+    net = guess.Net(H, W, n, seed=7)
+    net.set_params(theta.astype(np.float32))
+    xd, yd = torch.from_numpy(x).cuda(), torch.zeros((n, H, W, 2), device="cuda")
+    torch.cuda.synchronize()
+    net.forward(xd.data_ptr(), yd.data_ptr(), n)
+    out = U.UNet(theta, bf16=True).forward(x)
+    assert np.any(out) and np.max(np.abs(yd.cpu().numpy() - out)) <= 1e-6 * np.max(np.abs(out))
+
+
 @pytest.mark.parametrize("nmodes, kphys", [(1, 4), (2, 4), (3, 8), (4, 8), (5, 16), (16, 32), (20, 64), (33, 128),
                                            (64, 128), (65, 256), (100, 256), (40, 512), (30, 1024)])
 def test_nonlinear_terms_at_every_size(torch_mod, nmodes, kphys):

@@ -223,148 +223,169 @@ __global__ void __launch_bounds__(256) conv3x3_kernel(long NP, int H, int W, int
 
 // Same convolution with the input staged in LDS, on gfx950's K=16 matrix
 // instruction (v_mfma_f32_32x32x16_bf16): a workgroup owns PX consecutive
-// flattened output pixels (4 wavefronts x MT 32-pixel tiles) and CT = 32*NT
+// flattened output pixels (4 wavefronts x MT 32-pixel tiles) and CT = 32
 // output channels.  Per 32-channel chunk it holds the packed weights and the
-// PX + 2W + 2 input pixels its 3x3 taps can reach in LDS (rows of CKQ bf16,
-// 16-byte aligned, so every A and B fragment is one 16-byte LDS read).  The
-// next chunk's global loads (NI 8-byte pieces of input and the weights per
-// thread) are issued before the current chunk's arithmetic and written to
-// LDS after it.
-constexpr int CKQ = CK + 8;     // LDS row of the K=16 kernel (80 bytes)
+// PX + 2W + 2 input pixels its 3x3 taps can reach in LDS.  The next chunk's
+// global loads (NI 16-byte pieces of input and the weights per thread) are
+// issued before the current chunk's arithmetic and written to LDS after it.
+// The weights are the first operand, the pixels the second: a lane's results
+// are 4 consecutive channels of one pixel, 8-byte stores.
+//
+// What bounds it: LDS reads (3 fragments of 1 KB for 2 MFMAs with MT = 2, 128 B
+// a clock) and the loads' latency, one per chunk: three workgroups a CU cover
+// more of it than twice the channels each (a quarter slower) or a loop over
+// tiles with the next one's loads ahead (the registers).  So rows are
+// 64 bytes with their pieces permuted against bank conflicts (not padded to
+// 80), offsets are 32-bit and formed once, and a tap outside the image reads a
+// row of zeros instead of branching.  Four input channels (CIN4: the first
+// layer) take one 8-byte piece a pixel and the first half of a chunk's K; the
+// other half would add zeros.  64 images of
+// 32x136, the 14 layers together: 448 -> 243 us (with padded rows, branches,
+// 64-bit divisions and 2-byte stores: 2.1 to 1.2 times each).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-template <int MT, int NT, int NI>
-__global__ void __launch_bounds__(256) conv3x3s_kernel(long NP, int H, int W, int cin, int cinp,
+// byte offset of piece p (8 channels) of row r in LDS.  A 16-byte LDS access
+// takes 16 lanes at a time, 0-3, 12-15, 20-27 (and 4-11, 16-19, 28-31, and so in
+// the upper half): a piece of these rows after any first row, and the pieces of
+// 4 rows, lie in 16 different columns of the 256 bytes.
+__device__ __forceinline__ unsigned conv_slot(unsigned r, unsigned p)
+{
+    return r * 64 + ((p ^ (r >> 2 & 3)) << 4);
+}
+
+template <int MT, int NI, bool CIN4>
+__global__ void __launch_bounds__(256, 3) conv3x3s_kernel(int NP, int H, int W, int cin, int cinp,
                                                        int cout, const bf16 *__restrict__ X,
                                                        const bf16 *__restrict__ wp,
                                                        const float *__restrict__ bias,
                                                        bf16 *__restrict__ Y, int relu)
 {
-    constexpr int CT = 32 * NT, PX = 4 * 32 * MT, WPT = 9 * CT * (CK / 4) / 256;
-    static_assert(9 * CT * (CK / 4) % 256 == 0, "weight pieces per thread");
-    __shared__ __attribute__((aligned(16))) bf16 Ws[9][CT][CKQ];
+    constexpr int CT = 32, PX = 128 * MT, WPT = (9 * CT * 4 + 255) / 256;
     extern __shared__ __attribute__((aligned(16))) unsigned char conv_smem[];
-    bf16 (*Xs)[CKQ] = reinterpret_cast<bf16 (*)[CKQ]>(conv_smem);
-    const int NQ = PX + 2 * W + 2;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const long p0 = static_cast<long>(blockIdx.x) * PX;
-    const long q0 = p0 - W - 1;                   // global pixel of Xs[0]
+    unsigned char *Ws = conv_smem, *Xs = Ws + 9 * CT * 64;
+    const int NQ = PX + 2 * W + 2;                // staged pixels; row NQ: zeros
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
+    const int p0 = static_cast<int>(blockIdx.x) * PX;
+    const int q0 = p0 - W - 1;                    // pixel of Xs row 0
     const int o0 = blockIdx.y * CT;
-    // this lane's A-operand pixels (row of each 32x16 fragment) and tap masks
-    int lq[MT];
-    unsigned tapok[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int lp = wave * 32 * MT + m * 32 + (lane & 31);
-        const long pa = p0 + lp;
-        const int wa = static_cast<int>(pa % W), ha = static_cast<int>((pa / W) % H);
-        unsigned ok = 0;
-#pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            const int hh = ha + t / 3 - 1, ww = wa + t % 3 - 1;
-            if (pa < NP && hh >= 0 && hh < H && ww >= 0 && ww < W) ok |= 1u << t;
-        }
-        lq[m] = lp + W + 1;
-        tapok[m] = ok;
-    }
-    float16v acc[MT][NT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.f;
     // buffer resources: the weights, and the activations from the tile's
-    // first reachable pixel; pieces outside the image or past cin read zero
-    const long qb = q0 > 0 ? q0 : 0;
+    // first reachable pixel; pieces outside the batch read zero
+    const int qb = q0 > 0 ? q0 : 0;
     const __amdgpu_buffer_rsrc_t wres =
         buf_rsrc_uniform(wp, static_cast<size_t>(9) * cout * cinp * sizeof(bf16));
-    const __amdgpu_buffer_rsrc_t xres =
-        buf_rsrc_uniform(X + qb * cin, static_cast<size_t>(NP - qb) * cin * sizeof(bf16));
-    short4v wr[WPT], xr[NI];
+    const __amdgpu_buffer_rsrc_t xres = buf_rsrc_uniform(
+        X + static_cast<size_t>(qb) * cin,
+        static_cast<size_t>(min(NP - qb, NQ)) * cin * sizeof(bf16));
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    // this thread's first pieces; the others follow at uniform distances (64 rows
+    // of weights, or 64 pixels, 256 with CIN4), past the last one past the range;
+    // before the batch (the first tile) the offset wraps past it
+    const unsigned wo = static_cast<unsigned>(((tid / 4 / CT * cout + o0 + tid / 4 % CT) * cinp + 8 * (tid % 4)) * 2);
+    const unsigned wd = static_cast<unsigned>((64 / CT) * cout * cinp * 2);
+    const unsigned xo = static_cast<unsigned>(
+        (q0 - qb) * cin * 2 + (CIN4 ? tid * cin * 2 : (tid / 4 * cin + 8 * (tid % 4)) * 2));
+    const unsigned xd = static_cast<unsigned>((CIN4 ? 256 : 64) * cin * 2);
+    u4 wr[WPT], xr[NI];
     auto fetch = [&](int c0) {
 #pragma unroll
-        for (int s = 0; s < WPT; ++s) {
-            const int e = tid + 256 * s;
-            const int q = e % (CK / 4), o = (e / (CK / 4)) % CT, t = e / ((CK / 4) * CT);
-            const unsigned off = static_cast<unsigned>(((t * cout + o0 + o) * cinp + c0 + 4 * q) * 2);
-            wr[s] = __builtin_bit_cast(short4v, __builtin_amdgcn_raw_buffer_load_b64(wres, off, 0, 0));
-        }
+        for (int s = 0; s < WPT; ++s)
+            wr[s] = __builtin_amdgcn_raw_buffer_load_b128(wres, wo + (s * wd + 2 * c0), 0, 0);
 #pragma unroll
         for (int s = 0; s < NI; ++s) {
-            const int e = tid + 256 * s;
-            const int q = e / (CK / 4), g = e % (CK / 4);
-            const long gp = q0 + q;
-            // cin is a multiple of 4: a 4-channel group is all in range or none
-            const bool ok = q < NQ && gp >= 0 && c0 + 4 * g < cin;
-            const unsigned off =
-                ok ? static_cast<unsigned>(((gp - qb) * cin + c0 + 4 * g) * 2) : kBufOff;
-            xr[s] = __builtin_bit_cast(short4v, __builtin_amdgcn_raw_buffer_load_b64(xres, off, 0, 0));
+            if constexpr (CIN4) {
+                const u2 v = __builtin_amdgcn_raw_buffer_load_b64(xres, xo + s * xd, 0, 0);
+                xr[s] = u4{v.x, v.y, 0, 0};
+            } else {
+                xr[s] = __builtin_amdgcn_raw_buffer_load_b128(xres, xo + (s * xd + 2 * c0), 0, 0);
+            }
         }
     };
     auto stash = [&]() {
 #pragma unroll
         for (int s = 0; s < WPT; ++s) {
             const int e = tid + 256 * s;
-            const int q = e % (CK / 4), o = (e / (CK / 4)) % CT, t = e / ((CK / 4) * CT);
-            *reinterpret_cast<short4v *>(&Ws[t][o][4 * q]) = wr[s];
+            if (256 * (s + 1) <= 9 * CT * 4 || e < 9 * CT * 4)
+                *reinterpret_cast<u4 *>(Ws + conv_slot(e / 4, e % 4)) = wr[s];
         }
 #pragma unroll
         for (int s = 0; s < NI; ++s) {
-            const int e = tid + 256 * s;
-            const int q = e / (CK / 4), g = e % (CK / 4);
-            if (q < NQ) *reinterpret_cast<short4v *>(&Xs[q][4 * g]) = xr[s];
+            const int e = tid + 256 * s, q = CIN4 ? e : e / 4, g = CIN4 ? 0 : e % 4;
+            if (q < NQ) *reinterpret_cast<u4 *>(Xs + conv_slot(q, g)) = xr[s];
         }
     };
     fetch(0);
+    if (tid < 4) *reinterpret_cast<u4 *>(Xs + NQ * 64 + 16 * tid) = u4{0, 0, 0, 0};
+    // this lane's pixels: offsets of their fragments per tap (K 8 half .. + 7)
+    unsigned xa[MT][9];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int lp = wave * 32 * MT + m * 32 + (lane & 31);
+        const unsigned pa = static_cast<unsigned>(p0 + lp), row = pa / static_cast<unsigned>(W);
+        const int wa = static_cast<int>(pa - row * W), ha = static_cast<int>(row % static_cast<unsigned>(H));
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const int hh = ha + t / 3 - 1, ww = wa + t % 3 - 1;
+            const bool ok = (static_cast<unsigned>(hh) < static_cast<unsigned>(H)) &
+                            (static_cast<unsigned>(ww) < static_cast<unsigned>(W)) &
+                            (!CIN4 || half == 0);
+            const unsigned r = static_cast<unsigned>(lp + W + 1 + (t / 3 - 1) * W + t % 3 - 1);
+            xa[m][t] = ok ? conv_slot(r, half) : static_cast<unsigned>(NQ * 64);
+        }
+    }
+    const unsigned wa0 = conv_slot(lane & 31, half);   // + 64 bytes per further row
+    float16v acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[m][i] = 0.f;
     stash();
     __syncthreads();
     for (int c0 = 0; c0 < cinp; c0 += CK) {
         const bool more = c0 + CK < cinp;
         if (more) fetch(c0 + CK);
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            const int sh = (t / 3 - 1) * W + (t % 3 - 1);
+        for (int t = 0; t < 9; ++t)
 #pragma unroll
-            for (int kk = 0; kk < CK; kk += 16) {
-                const int kb = kk + (lane >> 5) * 8;
-                bf16x8 b[NT];
-#pragma unroll
-                for (int n = 0; n < NT; ++n)
-                    b[n] = *reinterpret_cast<const bf16x8 *>(&Ws[t][n * 32 + (lane & 31)][kb]);
+            for (int kk = 0; kk < (CIN4 ? 1 : 2); ++kk) {     // pieces half + 2 kk
+                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(Ws + t * CT * 64 + (wa0 ^ (32 * kk)));
 #pragma unroll
                 for (int m = 0; m < MT; ++m) {
-                    bf16x8 a = {};
-                    if (tapok[m] >> t & 1u) a = *reinterpret_cast<const bf16x8 *>(&Xs[lq[m] + sh][kb]);
-#pragma unroll
-                    for (int n = 0; n < NT; ++n)
-                        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[n], acc[m][n], 0, 0, 0);
+                    const bf16x8 a = *reinterpret_cast<const bf16x8 *>(Xs + (xa[m][t] ^ (32 * kk)));
+                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, acc[m], 0, 0, 0);
                 }
             }
-        }
         __syncthreads();
         if (more) {
             stash();
             __syncthreads();
         }
     }
-    // D layout: lane holds output channel (lane & 31); register i holds pixel
-    // 8*(i/4) + 4*(lane/32) + (i%4) of the 32-pixel tile
+    // D layout: lane holds pixel (lane & 31); register i output channel
+    // 8*(i/4) + 4*half + (i%4) of the 32
+    const int o = o0 + 4 * half;
+    f32x4 bo[4];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        const int o = o0 + n * 32 + (lane & 31);
-        const float bo = bias[o];
+    for (int g = 0; g < 4; ++g) bo[g] = *reinterpret_cast<const f32x4 *>(bias + o + 8 * g);
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m) {
+        const int p = p0 + wave * 32 * MT + m * 32 + (lane & 31);
+        if (p >= NP) continue;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const long p = p0 + wave * 32 * MT + m * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-                if (p < NP) {
-                    float v = acc[m][n][i] + bo;
-                    if (relu) v = fmaxf(v, 0.f);
-                    Y[p * cout + o] = f2bf(v);
-                }
+        for (int g = 0; g < 4; ++g) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] = acc[m][4 * g + i] + bo[g][i];
+                if (relu) v[i] = fmaxf(v[i], 0.f);
             }
+            u2 y;
+            y.x = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{v[0], v[1]}), bf16x2));
+            y.y = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{v[2], v[3]}), bf16x2));
+            *reinterpret_cast<u2 *>(Y + static_cast<size_t>(p) * cout + o + 8 * g) = y;
+        }
     }
 }
 
@@ -1065,17 +1086,18 @@ void zero(long n, float *a, hipStream_t st)
     if (n > 0) hipLaunchKernelGGL(zero_kernel, dim3(nb(n)), dim3(256), 0, st, n, a);
 }
 int conv3x3_cinp(int cin) { return (cin + CK - 1) / CK * CK; }
-// conv3x3s_kernel: dynamic LDS of the input stage for PX pixels of width w
-// (the weight stage, at most 9 * 64 * CKQ bf16 = 46 KB, is static), and the
-// 8-byte input pieces per thread it holds in registers
-static size_t conv3x3s_lds(int px, int w) { return static_cast<size_t>(px + 2 * w + 2) * CKQ * sizeof(bf16); }
-constexpr size_t kConvStagedLds = 64 * 1024;
-// input pieces per thread of the two tilings (reach of widths up to 143)
-constexpr int kConvPieces128 = 13, kConvPieces256 = 17;
-static bool conv3x3s_fits(int px, int w, int pieces)
+// conv3x3s_kernel's forms: tiles per wavefront and 16-byte input pieces per
+// thread, which bound the width: 128 MT + 2W + 2 <= 64 NI (159).  Two tiles
+// read 3 fragments for 2 MFMAs instead of 2 for 1 and stage fewer neighbours,
+// but pay with fewer workgroups: not below two a CU (128 channels of 64 images of
+// 8x34, 272 workgroups against 544: 14.2 against 13.0 us; 64 channels of 16x68,
+// 544 against 1088: 13.7 against 15.2).
+#define TBL_CONV_FORMS(X) X(2, 9) X(1, 7)
+static bool conv3x3s_fits(int mt, int w, int ni) { return 128 * mt + 2 * w + 2 <= 64 * ni; }
+static size_t conv3x3s_lds(int mt, int w) { return 64 * (static_cast<size_t>(9) * 32 + 128 * mt + 2 * w + 3); }
+static int conv3x3s_tiles(long np, int w, int cout)
 {
-    return conv3x3s_lds(px, w) <= kConvStagedLds &&
-           static_cast<long>(px + 2 * w + 2) * (CK / 4) <= 256L * pieces;
+    return conv3x3s_fits(2, w, 9) && (np + 255) / 256 * (cout / 32) >= 512 ? 2 : 1;
 }
 void pack_conv3x3(int cin, int cout, const bf16 *w, bf16 *wp, hipStream_t st)
 {
@@ -1088,24 +1110,36 @@ void conv3x3(int n, int h, int w, int cin, int cout, const bf16 *x, const bf16 *
 {
     const int cinp = conv3x3_cinp(cin);
     const long np = static_cast<long>(n) * h * w;
-    // dynamic LDS above the default limit is opted into once per process
-    static const bool staged_ok =
-        hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3x3s_kernel<1, 2, kConvPieces128>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kConvStagedLds) == hipSuccess &&
-        hipFuncSetAttribute(reinterpret_cast<const void *>(&conv3x3s_kernel<2, 1, kConvPieces256>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kConvStagedLds) == hipSuccess;
-    // LDS-staged form when the reach of a tile fits beside the weights
-    if (staged_ok && cout % 64 == 0 && conv3x3s_fits(128, w, kConvPieces128)) {
-        dim3 grid(static_cast<unsigned>((np + 127) / 128), cout / 64);
-        hipLaunchKernelGGL((conv3x3s_kernel<1, 2, kConvPieces128>), grid, dim3(256),
-                           conv3x3s_lds(128, w), st, np, h, w, cin, cinp, cout, x, wp, bias, y, relu);
-        return;
+    // the staged form: whole chunks of channels or the first layer's four, 32-bit
+    // pixel and byte counts of a tile, and a reach that its pieces hold
+    if (cout % 32 == 0 && (cin % CK == 0 || cin == 4) && np < (1L << 31) - 512 &&
+        conv3x3s_fits(1, w, 7) && static_cast<long>(cout) * cinp * 18 < (1L << 31)) {
+        static const bool staged_ok = [] {
+            bool ok = true;
+#define X(MT, NI)                                                                              \
+    for (const void *f : {reinterpret_cast<const void *>(&conv3x3s_kernel<MT, NI, false>),     \
+                          reinterpret_cast<const void *>(&conv3x3s_kernel<MT, NI, true>)})     \
+        ok = ok && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
+            TBL_CONV_FORMS(X)
+#undef X
+            return ok;
+        }();
+        const int mt = conv3x3s_tiles(np, w, cout);
+#define X(MT, NI)                                                                              \
+    if (staged_ok && mt == MT) {                                                               \
+        const dim3 grid(static_cast<unsigned>((np + 128 * MT - 1) / (128 * MT)), cout / 32);   \
+        if (cin == 4)                                                                          \
+            hipLaunchKernelGGL((conv3x3s_kernel<MT, NI, true>), grid, dim3(256),               \
+                               conv3x3s_lds(MT, w), st, static_cast<int>(np), h, w, cin, cinp, \
+                               cout, x, wp, bias, y, relu);                                    \
+        else                                                                                   \
+            hipLaunchKernelGGL((conv3x3s_kernel<MT, NI, false>), grid, dim3(256),              \
+                               conv3x3s_lds(MT, w), st, static_cast<int>(np), h, w, cin, cinp, \
+                               cout, x, wp, bias, y, relu);                                    \
+        return;                                                                                \
     }
-    if (staged_ok && cout % 32 == 0 && conv3x3s_fits(256, w, kConvPieces256)) {
-        dim3 grid(static_cast<unsigned>((np + 255) / 256), cout / 32);
-        hipLaunchKernelGGL((conv3x3s_kernel<2, 1, kConvPieces256>), grid, dim3(256),
-                           conv3x3s_lds(256, w), st, np, h, w, cin, cinp, cout, x, wp, bias, y, relu);
-        return;
+        TBL_CONV_FORMS(X)
+#undef X
     }
     if (cout % 64 == 0) {
         dim3 grid(static_cast<unsigned>((np + 63) / 64), cout / 64);

@@ -69,7 +69,6 @@ struct tbl_net {
     bf16 *act[NCONV] = {nullptr};
     bf16 *pool_out[3] = {nullptr};
     bf16 *cat[3] = {nullptr};
-    float *z = nullptr;          // fp32 output of the current GEMM (max P*cout)
     float *out = nullptr;        // fp32 network output (P0 x 2)
     bf16 *col = nullptr;         // im2col scratch
     float *dcol = nullptr;       // dcol scratch
@@ -154,7 +153,6 @@ int net_alloc(tbl_net *n)
         A_(n->cat[l], N * n->hw(l) * cc[l]);
         A_(n->d_cat[l], N * n->hw(l) * cc[l]);
     }
-    A_(n->z, maxz);
     A_(n->out, N * n->hw(0) * 2);
     A_(n->d_out, N * n->hw(0) * 2);
     A_(n->col, maxcol);
@@ -186,16 +184,10 @@ void conv_fwd(tbl_net *n, int id, const bf16 *x, int N, hipStream_t st)
     const Conv &c = n->L[id];
     const int h = n->H >> c.lvl, w = n->W >> c.lvl;
     const long P = static_cast<long>(N) * h * w;
-    const int kk = c.ks * c.ks * c.cin;
-    if (c.ks == 3) {
+    if (id == OUT)
+        out_fwd(P, x, n->wb + c.woff, n->w + c.boff, n->out, st);
+    else
         conv3x3(N, h, w, c.cin, c.cout, x, n->wp + c.wpoff, n->w + c.boff, n->act[id], c.relu, st);
-        return;
-    }
-    const bf16 *A = x;
-    float *Z = (id == OUT) ? n->out : n->z;
-    gemm(static_cast<int>(P), c.cout, kk, A, kk, 1, n->wb + c.woff, c.cout, 1, Z, c.cout, 1.f,
-         0.f, st);
-    bias_act(P, c.cout, Z, n->w + c.boff, id == OUT ? nullptr : n->act[id], c.relu, st);
 }
 
 // conv backward.  dy: fp32 gradient w.r.t. this conv's output; dx: fp32
@@ -349,7 +341,7 @@ extern "C" int tbl_net_destroy(tbl_net *n)
     fr(n->w); fr(n->g); fr(n->m); fr(n->v); fr(n->wb); fr(n->wp); fr(n->x_in); fr(n->d_xin);
     for (int i = 0; i < NCONV; ++i) { fr(n->act[i]); fr(n->d_act[i]); }
     for (int l = 0; l < 3; ++l) { fr(n->pool_out[l]); fr(n->d_pool[l]); fr(n->cat[l]); fr(n->d_cat[l]); }
-    fr(n->z); fr(n->out); fr(n->d_out); fr(n->col); fr(n->dcol); fr(n->dzb); fr(n->d_loss); fr(n->ws); fr(n->bs);
+    fr(n->out); fr(n->d_out); fr(n->col); fr(n->dcol); fr(n->dzb); fr(n->d_loss); fr(n->ws); fr(n->bs);
     if (n->own) (void)hipStreamDestroy(n->own);
     delete n;
     return TBL_OK;

@@ -16,7 +16,7 @@ void gemm(int M, int N, int K, const bf16 *A, long sam, long sak, const bf16 *B,
           long sbn, float *C, long ldc, float alpha, float beta, hipStream_t st, int splitk = 1);
 void im2col(int n, int h, int w, int c, const bf16 *x, bf16 *col, hipStream_t st);
 void col2im(int n, int h, int w, int c, const float *dcol, float *dx, int acc, hipStream_t st);
-void bias_act(long P, int c, float *z, const float *b, bf16 *y, int relu, hipStream_t st);
+void out_fwd(long P, const bf16 *x, const bf16 *w, const float *b, float *y, hipStream_t st);
 void relu_back(long n, const float *dy, const bf16 *y, bf16 *dz, int relu, hipStream_t st);
 void bias_grad(long P, int c, const bf16 *dz, float *db, hipStream_t st);
 void pool(int n, int h, int w, int c, const bf16 *x, bf16 *y, hipStream_t st);

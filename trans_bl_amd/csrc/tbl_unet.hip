@@ -850,17 +850,34 @@ __global__ void col2im_kernel(int Nn, int H, int W, int Cc, const float *dcol, f
 }
 
 // y = relu(z + b) -> bf16 (relu = 0: identity, fp32 output kept in z)
-__global__ void bias_act_kernel(long P, int Cc, float *z, const float *b, bf16 *y, int relu)
+// The output layer, 1x1 from 32 channels to 2, with bias: four lanes a pixel, 8
+// channels (16 bytes) each, fp32 sums.  A 64-wide GEMM tile has no use for two
+// columns, and its bias took a pass of its own: 64 images of 32x136 (20 MB)
+// 32 -> 5.6 us.
+__global__ void __launch_bounds__(256) out_kernel(unsigned P, const bf16 *__restrict__ x,
+                                                  const bf16 *__restrict__ w,
+                                                  const float *__restrict__ b, float *__restrict__ y)
 {
-    const long e = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-    if (e >= P * Cc) return;
-    float v = z[e] + b[e % Cc];
-    if (relu) v = fmaxf(v, 0.f);
-    z[e] = v;
-    if (y) y[e] = f2bf(v);
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const unsigned e = blockIdx.x * 256u + threadIdx.x, p = e / 4, q = e % 4;
+    if (p >= P) return;
+    const u4 v = *reinterpret_cast<const u4 *>(x + static_cast<size_t>(p) * 32 + 8 * q);
+    const u4 w0 = reinterpret_cast<const u4 *>(w)[2 * q], w1 = reinterpret_cast<const u4 *>(w)[2 * q + 1];
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const unsigned t = v[c / 2], u = c < 4 ? w0[c] : w1[c - 4];      // w[channel][output]
+        const float a = __uint_as_float(c % 2 ? t & 0xffff0000u : t << 16);
+        s0 = fmaf(a, __uint_as_float(u << 16), s0);
+        s1 = fmaf(a, __uint_as_float(u & 0xffff0000u), s1);
+    }
+    s0 += __shfl_xor(s0, 1, 4);
+    s1 += __shfl_xor(s1, 1, 4);
+    s0 += __shfl_xor(s0, 2, 4);
+    s1 += __shfl_xor(s1, 2, 4);
+    if (q < 2) y[2 * static_cast<size_t>(p) + q] = (q ? s1 : s0) + b[q];
 }
 
-// dZ = dY * (y > 0) (relu) or dY, written as bf16 for the GEMMs
 __global__ void relu_back_kernel(long n, const float *dY, const bf16 *y, bf16 *dZ, int relu)
 {
     const long e = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
@@ -886,22 +903,25 @@ __global__ void bias_grad_kernel(long P, int Cc, const bf16 *dZ, float *db)
     if (threadIdx.x == 0) db[c] = red[0];
 }
 
-// 2x2 average pooling, NHWC
-__global__ void pool_kernel(int Nn, int H, int W, int Cc, const bf16 *X, bf16 *Y)
+// 2x2 average pooling, NHWC, 8 channels a thread (total: outputs / 8)
+__global__ void __launch_bounds__(256) pool_kernel(unsigned total, unsigned H2, unsigned W2, unsigned G,
+                                                   const bf16 *__restrict__ X, bf16 *__restrict__ Y)
 {
-    const int h2 = H / 2, w2 = W / 2;
-    const long total = static_cast<long>(Nn) * h2 * w2 * Cc;
-    const long e = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const unsigned e = blockIdx.x * 256u + threadIdx.x;
     if (e >= total) return;
-    const int c = static_cast<int>(e % Cc);
-    long p = e / Cc;
-    const int w = static_cast<int>(p % w2), h = static_cast<int>((p / w2) % h2);
-    const int n = static_cast<int>(p / (static_cast<long>(w2) * h2));
-    auto at = [&](int hh, int ww) {
-        return bf2f(X[((static_cast<long>(n) * H + hh) * W + ww) * Cc + c]);
-    };
-    Y[e] = f2bf(0.25f * (at(2 * h, 2 * w) + at(2 * h, 2 * w + 1) + at(2 * h + 1, 2 * w) +
-                         at(2 * h + 1, 2 * w + 1)));
+    const unsigned p = e / G, g = e % G, r = p / W2, w = p % W2;         // r: image and row
+    const u4 *x = reinterpret_cast<const u4 *>(X) + ((static_cast<size_t>(2) * r * 2 * W2 + 2 * w) * G + g);
+    const u4 a = x[0], b = x[G], c = x[static_cast<size_t>(2) * W2 * G], d = x[(static_cast<size_t>(2) * W2 + 1) * G];
+    u4 y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        auto lo = [](unsigned v) { return __uint_as_float(v << 16); };
+        auto hi = [](unsigned v) { return __uint_as_float(v & 0xffff0000u); };
+        const unsigned l = f2bf(0.25f * (lo(a[i]) + lo(b[i]) + lo(c[i]) + lo(d[i])));
+        y[i] = l | static_cast<unsigned>(f2bf(0.25f * (hi(a[i]) + hi(b[i]) + hi(c[i]) + hi(d[i])))) << 16;
+    }
+    reinterpret_cast<u4 *>(Y)[e] = y;
 }
 
 __global__ void pool_back_kernel(int Nn, int H, int W, int Cc, const float *dY, float *dX, int accumulate)
@@ -918,24 +938,20 @@ __global__ void pool_back_kernel(int Nn, int H, int W, int Cc, const float *dY, 
 }
 
 // Y[:, :, :, 0:C1] = up2(A) (nearest), Y[:, :, :, C1:C1+C2] = Bskip
-// four channels (8 bytes) per thread; C1 and C2 are multiples of 4 and the
+// 8 channels (16 bytes) per thread; C1 and C2 are multiples of 8 and the
 // pixel count fits 32 bits
-__global__ void up_concat_kernel(int Nn, int H, int W, int C1, int C2, const bf16 *A, const bf16 *Bk,
-                                 bf16 *Y)
+__global__ void __launch_bounds__(256) up_concat_kernel(unsigned total, unsigned H, unsigned W, unsigned G1,
+                                                        unsigned G2, const bf16 *__restrict__ A,
+                                                        const bf16 *__restrict__ Bk, bf16 *__restrict__ Y)
 {
-    const int Ct = C1 + C2, G = Ct / 4;
-    const unsigned total = static_cast<unsigned>(Nn) * H * W * G;
-    const unsigned e = blockIdx.x * 256u + threadIdx.x;
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const unsigned G = G1 + G2, e = blockIdx.x * 256u + threadIdx.x;
     if (e >= total) return;
-    const int c = static_cast<int>(e % G) * 4;
-    const unsigned p = e / G;
-    const int w = static_cast<int>(p % W), h = static_cast<int>((p / W) % H);
-    const int n = static_cast<int>(p / (static_cast<unsigned>(W) * H));
-    const bf16 *src = (c < C1)
-        ? A + (static_cast<size_t>((n * (H / 2) + h / 2) * (W / 2) + w / 2) * C1 + c)
-        : Bk + (static_cast<size_t>(p) * C2 + (c - C1));
-    *reinterpret_cast<short4v *>(Y + static_cast<size_t>(p) * Ct + c) =
-        *reinterpret_cast<const short4v *>(src);
+    const unsigned g = e % G, p = e / G, r = p / W, w = p % W;           // r: image and row
+    const u4 *src = g < G1 ? reinterpret_cast<const u4 *>(A) +
+                                 (static_cast<size_t>((r / H * (H / 2) + r % H / 2) * (W / 2) + w / 2) * G1 + g)
+                           : reinterpret_cast<const u4 *>(Bk) + (static_cast<size_t>(p) * G2 + (g - G1));
+    reinterpret_cast<u4 *>(Y)[e] = *src;
 }
 
 // split the gradient of up_concat: dA (low res, sum of 4) and dB (skip)
@@ -1029,9 +1045,9 @@ void col2im(int n, int h, int w, int c, const float *dcol, float *dx, int acc, h
     const long t = static_cast<long>(n) * h * w * c;
     hipLaunchKernelGGL(col2im_kernel, dim3(nb(t)), dim3(256), 0, st, n, h, w, c, dcol, dx, acc);
 }
-void bias_act(long P, int c, float *z, const float *b, bf16 *y, int relu, hipStream_t st)
+void out_fwd(long P, const bf16 *x, const bf16 *w, const float *b, float *y, hipStream_t st)
 {
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nb(P * c)), dim3(256), 0, st, P, c, z, b, y, relu);
+    hipLaunchKernelGGL(out_kernel, dim3(nb(4 * P)), dim3(256), 0, st, static_cast<unsigned>(P), x, w, b, y);
 }
 void relu_back(long n, const float *dy, const bf16 *y, bf16 *dz, int relu, hipStream_t st)
 {
@@ -1043,19 +1059,19 @@ void bias_grad(long P, int c, const bf16 *dz, float *db, hipStream_t st)
 }
 void pool(int n, int h, int w, int c, const bf16 *x, bf16 *y, hipStream_t st)
 {
-    const long t = static_cast<long>(n) * (h / 2) * (w / 2) * c;
-    hipLaunchKernelGGL(pool_kernel, dim3(nb(t)), dim3(256), 0, st, n, h, w, c, x, y);
+    const long t = static_cast<long>(n) * (h / 2) * (w / 2) * (c / 8);
+    hipLaunchKernelGGL(pool_kernel, dim3(nb(t)), dim3(256), 0, st, static_cast<unsigned>(t), h / 2, w / 2, c / 8, x, y);
 }
 void pool_back(int n, int h, int w, int c, const float *dy, float *dx, int acc, hipStream_t st)
 {
     const long t = static_cast<long>(n) * h * w * c;
     hipLaunchKernelGGL(pool_back_kernel, dim3(nb(t)), dim3(256), 0, st, n, h, w, c, dy, dx, acc);
 }
-void up_concat(int n, int h, int w, int c1, int c2, const bf16 *a, const bf16 *b, bf16 *y,
-               hipStream_t st)
+void up_concat(int n, int h, int w, int c1, int c2, const bf16 *a, const bf16 *b, bf16 *y, hipStream_t st)
 {
-    const long t = static_cast<long>(n) * h * w * ((c1 + c2) / 4);
-    hipLaunchKernelGGL(up_concat_kernel, dim3(nb(t)), dim3(256), 0, st, n, h, w, c1, c2, a, b, y);
+    const long t = static_cast<long>(n) * h * w * ((c1 + c2) / 8);
+    hipLaunchKernelGGL(up_concat_kernel, dim3(nb(t)), dim3(256), 0, st, static_cast<unsigned>(t), h, w, c1 / 8, c2 / 8,
+                       a, b, y);
 }
 void up_concat_back(int n, int h, int w, int c1, int c2, const float *dy, float *da, float *db,
                     int acc_b, hipStream_t st)

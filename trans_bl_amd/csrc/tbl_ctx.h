@@ -27,7 +27,7 @@ struct tbl_ctx {
     std::vector<tbl::cx<float> *> E32, S32, R32, E32b;
     std::vector<double *> qdy2_d;
     std::vector<float *> qdy2_f;
-    std::vector<double *> lu_d;   // [K][2][5][ld] per level
+    std::vector<double *> lu_d;   // line-LU tables per level (tbl_kernels.h)
     std::vector<float *> lu_f;
     // inverse line matrices of the coarsest level (coarse_inv_size per mode and
     // centre/border), null where that form does not fit

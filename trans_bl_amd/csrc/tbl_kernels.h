@@ -10,6 +10,18 @@ namespace tbl {
 // -u1/pivot, -u2/pivot, 1/pivot
 constexpr int kLuFields = 8;
 
+// The line-LU tables of a level: [K][2][kLuFields][lus] by field and row, then
+// for each lane count the same factors as its lanes hold them: per (mode, kind)
+// line 16-byte chunks [chunk][lane], a lane's values field-major over its R
+// rows (l1, l2, u1, u2, -u1/p, -u2/p, 1/p and for FP64 p), so that a wavefront's
+// load is one contiguous run.
+constexpr int kLuLanes[3] = {16, 32, 64};
+constexpr int lu_pack_values(int esize) { return esize == 4 ? 7 : 8; }
+constexpr int lu_pack_chunks(int esize, int R) { return (lu_pack_values(esize) * R * esize + 15) / 16; }
+// elements of one line's packed table
+constexpr int lu_pack_line(int esize, int G, int R) { return lu_pack_chunks(esize, R) * G * (16 / esize); }
+size_t lu_pack_offset(int esize, int K, int ny, int lus, int G);   // G past the last: all elements
+
 // Per-level constants of the Poisson operator (poisson_par.f:229-793)
 template <typename T>
 struct LevelArgs {

@@ -572,6 +572,17 @@ int lu_stride(int ny)
     return (s + 7) / 8 * 8;
 }
 
+size_t lu_pack_offset(int esize, int K, int ny, int lus, int G)
+{
+    size_t o = static_cast<size_t>(K) * 2 * kLuFields * lus;
+    for (int g : kLuLanes) {
+        if (g == G) break;
+        const int R = line_rows_for(g, ny);
+        if (R > 0) o += static_cast<size_t>(K) * 2 * lu_pack_line(esize, g, R);
+    }
+    return o;
+}
+
 // G > 0: lanes per line with direct (lane-contiguous) global access;
 // G < 0: |G| lanes per line with the LDS-staged, coalesced kernel;
 // kStripShape < G < kXStagedShape: fused-sweep strips with G - kStripShape

@@ -169,24 +169,44 @@ __device__ __forceinline__ LineLU<T, R> load_line_lu_buf(__amdgpu_buffer_rsrc_t 
     return f;
 }
 
-// Same from a plain pointer to the line's padded table (stride lus).
-template <typename T, int R>
-__device__ __forceinline__ LineLU<T, R> load_line_lu_tbl(const T *__restrict__ lu, int lus, int j0)
+// Same factors from the packed tables of G lanes (rs: over them; off0: byte
+// offset of the line's): 16 bytes per lane and load, contiguous over the
+// lanes, instead of 8 R loads of one value at a stride of R values.  Where the
+// phases are bound by memory (1025x193x64 and up, finest level) that is worth
+// 0-2 %; where latency and address cycles count more: 385x97x8 FP64 solve 4.63 ->
+// 4.47 ms, the one-launch sweep of 513x97x64 FP32 32.8 -> 30.3 us, the mixed
+// solve of 1025x193x64 7.09 -> 6.86 ms.
+template <typename T, int G, int R>
+constexpr int kLuPackBytes = lu_pack_line(sizeof(T), G, R) * static_cast<int>(sizeof(T));
+template <typename T, int G, int R>
+__device__ __forceinline__ LineLU<T, R> load_line_lu_packed(__amdgpu_buffer_rsrc_t rs, unsigned off0,
+                                                           int lane)
 {
+    constexpr int NCH = lu_pack_chunks(sizeof(T), R), CV = 16 / sizeof(T);
+    T v[NCH * CV];
+#pragma unroll
+    for (int q = 0; q < NCH; ++q) {
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, off0 + lane * 16u, q * G * 16, 0);
+        __builtin_memcpy(v + q * CV, &x, sizeof(x));
+    }
     LineLU<T, R> f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int j = j0 + r;
-        f.l1[r] = lu[j];
-        f.l2[r] = lu[lus + j];
-        f.u1[r] = lu[2 * lus + j];
-        f.u2[r] = lu[3 * lus + j];
-        f.pv[r] = lu[4 * lus + j];
-        f.m1[r] = lu[5 * lus + j];
-        f.m2[r] = lu[6 * lus + j];
-        f.rp[r] = lu[7 * lus + j];
+        f.l1[r] = v[r];
+        f.l2[r] = v[R + r];
+        f.u1[r] = v[2 * R + r];
+        f.u2[r] = v[3 * R + r];
+        f.m1[r] = v[4 * R + r];
+        f.m2[r] = v[5 * R + r];
+        f.rp[r] = v[6 * R + r];
+        f.pv[r] = kIsF32<T> ? T(1) : v[7 * R + r];       // FP32 multiplies by 1 / p
     }
     return f;
+}
+template <typename T, int G, int R>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t lu_packed_rsrc(const T *pk, int K)
+{
+    return buf_rsrc(pk, static_cast<size_t>(K) * 2 * kLuPackBytes<T, G, R>);
 }
 
 // ---------------------------------------------------------------------------
@@ -456,11 +476,10 @@ __device__ __forceinline__ void relax_core(const LevelArgs<T> &L, const LineLU<T
 // one y-line relaxation on a column reached directly (global or LDS)
 template <typename T, int G, int R>
 __device__ __forceinline__ void relax_line(const LevelArgs<T> &L, cx<T> *col,
-                                           const cx<T> *__restrict__ Scol, const T *__restrict__ lu,
+                                           const cx<T> *__restrict__ Scol, const LineLU<T, R> &f,
                                            int side, T rf, int lane)
 {
     const int ny = L.ny, ld = L.ld;
-    const LineLU<T, R> f = load_line_lu_tbl<T, R>(lu, L.lus, line_j0(lane, R));
     relax_core<T, G, R>(
         L, f, rf, lane,
         [&](int j) { return xoff<T>(col, ld, j, side, side == 0 && j >= ny - 2); },

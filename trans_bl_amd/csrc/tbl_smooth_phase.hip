@@ -19,8 +19,9 @@ __global__ void __launch_bounds__(256) smooth_phase_kernel(LevelArgs<T> L, cx<T>
     const int i = phase_column(phase, c, L.nx);
     const int side = (phase == 0) ? (c == 0 ? -1 : 1) : 0;
     const size_t base = static_cast<size_t>(k) * L.plane + static_cast<size_t>(i) * L.ld;
-    const T *lut = lu + (static_cast<size_t>(k) * 2 + (side != 0)) * kLuFields * L.lus;
-    relax_line<T, G, R>(L, V + base, S + base, lut, side, rf, lane);
+    const LineLU<T, R> f = load_line_lu_packed<T, G, R>(
+        lu_packed_rsrc<T, G, R>(lu, L.K), (k * 2u + (side != 0)) * kLuPackBytes<T, G, R>, lane);
+    relax_line<T, G, R>(L, V + base, S + base, f, side, rf, lane);
 }
 
 constexpr int kStagedLines = 4;   // lines per workgroup of the staged smoother
@@ -156,11 +157,8 @@ __global__ void __launch_bounds__(256) smooth_staged_kernel(LevelArgs<T> L, cx<T
     }
     __syncthreads();
     if (live) {
-        const __amdgpu_buffer_rsrc_t lr =
-            buf_rsrc(lu, static_cast<size_t>(L.K) * 2 * kLuFields * L.lus * sizeof(T));
-        const unsigned lo = static_cast<unsigned>((static_cast<size_t>(k) * 2 + (side != 0)) *
-                                                  kLuFields * L.lus * sizeof(T));
-        const LineLU<T, R> f = load_line_lu_buf<T, R>(lr, lo, L.lus, line_j0(lane, R));
+        const LineLU<T, R> f = load_line_lu_packed<T, G, R>(
+            lu_packed_rsrc<T, G, R>(lu, L.K), (k * 2u + (side != 0)) * kLuPackBytes<T, G, R>, lane);
         if (FULL) {
             relax_core<T, G, R>(L, f, rf, lane, [&](int j) { return Xs[j]; },
                                 [&](int j) { return Vs[j]; }, [&](int j, int) { return Ss[j]; },
@@ -267,6 +265,7 @@ int phase_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, i
     G = form == 1 ? -G : form == 2 ? G - kXStagedShape : G;
     const int R = line_rows_for(G, L.ny);
     if (R < 0) return TBL_ERR_GRID;
+    lu += lu_pack_offset(sizeof(T), L.K, L.ny, L.lus, G);
     if (form == 1 && staged_lds<true>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
     if (form == 2 && staged_lds<false>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
     for (int it = 0; it < sweeps; ++it)

@@ -155,9 +155,8 @@ __device__ __forceinline__ void sweep_relax(const LevelArgs<T> &L, __amdgpu_buff
         }
     }
     wave_lds_sync();
-    const unsigned luo = static_cast<unsigned>((static_cast<size_t>(k) * 2 + (side != 0)) *
-                                               kLuFields * L.lus * sizeof(T));
-    const LineLU<T, R> f = load_line_lu_buf<T, R>(lr, luo, L.lus, line_j0(lane, R));
+    const LineLU<T, R> f =
+        load_line_lu_packed<T, G, R>(lr, (k * 2u + (side != 0)) * kLuPackBytes<T, G, R>, lane);
     relax_core<T, G, R>(L, f, rf, lane, [&](int j) { return Xs[j]; }, [&](int j) { return Vs[j]; },
                         [&](int j, int) { return Ss[j]; }, [&](int j, cx<T> v) { Vs[j] = v; });
     wave_lds_sync();
@@ -213,8 +212,7 @@ __global__ void __launch_bounds__(kSweepThreads) smooth_sweep_kernel(
     const unsigned ib = static_cast<unsigned>(in_half * half * ES);
     const unsigned ob = static_cast<unsigned>((1 - in_half) * half * ES);
     const __amdgpu_buffer_rsrc_t sr = buf_rsrc(S + poff, pbytes);
-    const __amdgpu_buffer_rsrc_t lr =
-        buf_rsrc(lu, static_cast<size_t>(L.K) * 2 * kLuFields * L.lus * sizeof(T));
+    const __amdgpu_buffer_rsrc_t lr = lu_packed_rsrc<T, G, R>(lu, L.K);
     cx<T> *outp = Vpair + (1 - in_half) * half + poff;
     cx<double> *upp = UPD ? vup + poff : nullptr;
     // boundary columns (Dirichlet data): copied by the strips owning the
@@ -336,6 +334,7 @@ int sweep_sweeps(const LevelArgs<T> &L, cx<T> *Va, cx<T> *Vb, const cx<T> *S, co
     if (vup && sizeof(T) != 4) return TBL_ERR_ARG;   // the update variant is FP32 only
     const int R = line_rows_for(G, L.ny);
     if (R < 0) return TBL_ERR_GRID;
+    lu += lu_pack_offset(sizeof(T), L.K, L.ny, L.lus, G);
     if (sweep_lds(L.ld, sizeof(cx<T>), G) > 160 * 1024) return TBL_ERR_GRID;
     const int width = sweep_strip_width(L.nx, L.K, wsel);
     int in_half = Va == pair ? 0 : 1;

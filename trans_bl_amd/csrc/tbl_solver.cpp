@@ -14,6 +14,27 @@
 using namespace tbl;
 
 namespace {
+
+// appends the lanes' form of the tables (tbl_kernels.h) to the rows' form
+template <typename T>
+void pack_lu(std::vector<T> &lu, int K, int ny, int lus)
+{
+    constexpr int es = sizeof(T), NF = lu_pack_values(es), CV = 16 / es;
+    static const int field[8] = {0, 1, 2, 3, 5, 6, 7, 4};
+    lu.resize(lu_pack_offset(es, K, ny, lus, 0), T(0));
+    for (int G : kLuLanes) {
+        const int R = line_rows_for(G, ny);
+        if (R <= 0) continue;
+        const size_t size = lu_pack_line(es, G, R);
+        for (int q = 0; q < 2 * K; ++q) {
+            const T *src = &lu[static_cast<size_t>(q) * kLuFields * lus];
+            T *dst = &lu[lu_pack_offset(es, K, ny, lus, G) + q * size];
+            for (int lane = 0; lane < G; ++lane)
+                for (int v = 0; v < NF * R; ++v)
+                    dst[(v / CV * G + lane) * CV + v % CV] = src[field[v / R] * lus + 1 + lane * R + v % R];
+        }
+    }
+}
 thread_local std::string g_last_error;
 }
 
@@ -165,6 +186,8 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
                 }
             }
         for (size_t e = 0; e < lu.size(); ++e) luf[e] = static_cast<float>(lu[e]);
+        pack_lu(lu, K, lv.ny, d);
+        pack_lu(luf, K, lv.ny, d);
         TRY(dalloc(&c->lu_d[l], lu.size()));
         TRY(dalloc(&c->lu_f[l], luf.size()));
         TBL_HIP(hipMemcpy(c->lu_d[l], lu.data(), sizeof(double) * lu.size(), hipMemcpyHostToDevice));

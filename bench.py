@@ -53,21 +53,22 @@ ROWS = (1, 2, 3, 4, 5, 6, 7, 9, 13, 17)
 
 def smoother_kernel(prec, lanes, ny):
     """Name of the smoother kernel a line shape runs in a plain sweep (as
-    rocprofv3 prints it): G direct, -G staged (x terms, v, S in LDS), 2000+G
-    staged (x terms only), 1000+G fused-sweep strip.  The staged kernel's
+    rocprofv3 prints it): G direct and 3000+G one-launch sweep, -G staged (x
+    terms, v, S in LDS), 2000+G staged (x terms only), 1000+G fused-sweep
+    strip.  The staged kernel's
     last template argument selects its updating form, which plain sweeps do
     not use.  A line's lanes hold its rows 1..ny-1 (row 0 is not relaxed)."""
-    g = lanes - 2000 if lanes > 2000 else lanes - 1000 if lanes > 1000 else abs(lanes)
+    g = (lanes - 3000) % 100 if lanes > 3000 else abs(lanes) % 1000
     need = -(-(ny - 1) // g)
     r = next(x for x in ROWS if x >= need)
     t = "float" if prec else "double"
-    if lanes > 2000:
+    if 3000 > lanes > 2000:
         return f"smooth_staged_kernel<{t}, {g}, {r}, false, false>"
-    if lanes > 1000:
+    if 2000 > lanes > 1000:
         return f"smooth_strip_kernel<{t}, {g}, {r}>"
     if lanes < 0:
         return f"smooth_staged_kernel<{t}, {g}, {r}, true, false>"
-    return f"smooth_phase_kernel<{t}, {g}, {r}>"
+    return f"smooth_sweep_kernel<{t}, {g}, {r}, false, false>"
 
 
 def measured_traffic(kernel):

@@ -329,14 +329,14 @@ int tbl_rk4_step_dev(tbl_ctx *ctx, double Re, double dt, int kphys, const tbl_ba
                      double *d_th, const tbl_solve_opts *opts, int *cycles, double *residual);
 
 /* Line-solve shape of one multigrid level's smoother: `lanes` (16, 32 or
-   64) lanes of a wavefront share one y-line; a negative value selects the
-   same shape with LDS-staged, coalesced loads and stores; 2000 + lanes
+   64) lanes of a wavefront share one y-line, a sweep in one launch; a negative
+   value selects colour phases with LDS-staged, coalesced loads and stores;
+   2000 + lanes
    stages only the x-direction terms in LDS and reads v and the source
    lane-contiguous; 1000 + lanes selects the fused-sweep strip smoother (a
    whole sweep per launch, one workgroup per strip of columns in LDS; not
    on the coarsest level).  On the coarsest level lanes = 1 (the default)
-   selects the sequential one-launch kernels and any lane form the G-lane
-   scan kernel; its FP32 shape is unused (that solve is FP64).
+   selects the inverse line matrices and any lane form the G-lane scan kernel.
    All forms give the same colour-ordered sweep.  prec 0 = FP64 smoother,
    1 = FP32 smoother.  Chosen by the autotuner; no reference counterpart
    (the reference solves each line sequentially, penta_par.f:367-404). */

@@ -48,19 +48,20 @@ constexpr int kDefBlock = sizeof(T) == 4 ? 8 : 2;
 
 // columns per strip: longer strips load fewer halo columns; the mixed
 // defect (FP64 in, FP32 out) was measured fastest at 64 on nx = 1025, the
-// others at 32.  Small levels take shorter strips, down to 2 columns, until
-// there are kDefWaves wavefronts (`waves` per strip): the march is a chain of
-// load latencies, one per block of columns (385x97x8 and its coarser levels,
-// FP64: 16.7 -> 4.7 us per launch of the plain form; the solve 5.03 -> 4.63 ms
-// with the one-pass form above).
-constexpr int kDefWaves = 1024;
+// others at 32.  Smaller levels take shorter strips (the march is a chain of load
+// latencies, one per block of columns): down to 4 columns until there are
+// kDefWaves wavefronts (`waves` per strip), 2 where that leaves less than a
+// quarter of them.  385x97x8 and its coarser levels, FP64: 16.7 -> 4.7 us per
+// launch of the plain form; a 1025x193x64 FP64 cycle 1.720 -> 1.677 ms with 4096
+// against 1024 wavefronts, 1.717 with 16384 (halo columns).
+constexpr int kDefWaves = 4096;
 template <typename T, typename TO>
 static int defect_strip(int nx, int waves)
 {
     int strip = sizeof(T) == 8 && sizeof(TO) == 4 && nx >= 1024 ? 64 : nx >= 512 ? 32 : 16;
-    while (strip > 2 && static_cast<long>(waves) * ((nx - 2 + strip - 1) / strip) < kDefWaves)
-        strip /= 2;
-    return strip;
+    auto all = [&](int w) { return static_cast<long>(waves) * ((nx - 2 + w - 1) / w); };
+    while (strip > 4 && all(strip) < kDefWaves) strip /= 2;
+    return strip == 4 && all(4) < kDefWaves / 4 ? 2 : strip;
 }
 
 // The restricting form (RS): the defect's full-weighting restriction onto

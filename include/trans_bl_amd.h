@@ -197,7 +197,8 @@ int tbl_deriv_dev(tbl_ctx *ctx, int kind, const double *d_fc, double *d_out);
 /* The four derivatives of one field in two passes over it (derparx,
    derparxx, dery, deryy of the same fc, as drv_gv calls them,
    main_par.f:1364-1377; derivs_par.f:80-129, 164-177).  Device pointers,
-   asynchronous on the context's stream; any output may be NULL. */
+   asynchronous on the context's stream; any output may be NULL, none may be
+   d_fc.  Where outputs of x and y overlap, the y-derivatives stand. */
 int tbl_derivs_dev(tbl_ctx *ctx, const double *d_fc, double *d_ddx, double *d_d2dx2,
                    double *d_ddy, double *d_d2dy2);
 

@@ -1,0 +1,56 @@
+"""Forms of a call whose route through the library depends on the grid: the
+result must not."""
+import numpy as np
+import pytest
+
+from trans_bl_amd import workload as wl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_mod(gpu_ready):
+    import torch
+    return torch
+
+
+def random_field(torch, g):
+    rng = np.random.default_rng(g.nx * g.ny)
+    return torch.from_numpy(rng.normal(size=(g.nmodes, g.ny, g.nx)) + 1j * rng.normal(size=(g.nmodes, g.ny, g.nx))).to("cuda")
+
+
+# the first three take all four derivatives in one launch where that may be, the last does not
+@pytest.mark.parametrize("nx, ny, nmodes", [(17, 9, 1), (129, 33, 4), (577, 143, 1), (641, 65, 2)], ids=lambda v: str(v))
+def test_derivatives_into_overlapping_outputs(torch_mod, nx, ny, nmodes):
+    """Outputs of the two directions in the same memory, whole or in part: the
+    y-derivatives, written last, stand; what they do not cover holds the
+    x-derivatives.  An output in the input's place is refused."""
+    torch = torch_mod
+    import trans_bl_amd as tb
+    g = wl.Grid(nx, ny, nmodes, 2, 0.02, 1e-3, 1.004, 0.0, 0.3)
+    f = random_field(torch, g)
+    n = f.numel()
+    with tb.Context(g) as ctx:
+        ref = [torch.zeros_like(f) for _ in range(4)]
+        p = [o.data_ptr() for o in ref]
+        ctx.derivs_dev(f.data_ptr(), p[0], p[1], 0, 0)
+        ctx.derivs_dev(f.data_ptr(), 0, 0, p[2], p[3])
+        ctx.synchronize()
+        a, b = torch.zeros_like(f), torch.zeros_like(f)
+        torch.cuda.synchronize()
+        ctx.derivs_dev(f.data_ptr(), a.data_ptr(), b.data_ptr(), a.data_ptr(), b.data_ptr())
+        ctx.synchronize()
+        assert torch.equal(a, ref[2]) and torch.equal(b, ref[3])
+        # d/dy starts half way into d/dx's memory
+        m = n // 2
+        buf, c = torch.zeros(n + m, dtype=f.dtype, device="cuda"), torch.zeros_like(f)
+        torch.cuda.synchronize()
+        ctx.derivs_dev(f.data_ptr(), buf.data_ptr(), b.data_ptr(), buf.data_ptr() + 16 * m, c.data_ptr())
+        ctx.synchronize()
+        assert torch.equal(buf[:m], ref[0].flatten()[:m]) and torch.equal(buf[m:], ref[2].flatten())
+        assert torch.equal(b, ref[1]) and torch.equal(c, ref[3])
+        for q in range(4):
+            out = [o.data_ptr() for o in (a, b, c, ref[3])]
+            out[q] = f.data_ptr()
+            with pytest.raises(tb.TblError):
+                ctx.derivs_dev(f.data_ptr(), *out)

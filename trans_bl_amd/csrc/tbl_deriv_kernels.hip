@@ -29,6 +29,8 @@
 // 230 -> 115 us, y 212 -> 160; of 2049x257x32 (809 MB): x 1526 -> 157, y 275 ->
 // 193.  x is bound by memory; y's rows of 128 bytes, mostly on two cache lines
 // each, keep it above that (three workgroups a CU instead of two: no faster).
+#include <cstdint>
+
 #include "tbl_deriv.h"
 
 namespace tbl {
@@ -395,12 +397,27 @@ static bool derivs_both(const DerivArgs &A, const C *f, C *dx, C *dxx, C *dy, C 
     return false;
 }
 
+// Where an output lies over the input or over one of the other direction, the
+// order counts (x, then y, which has read all of f it needs): two launches.
+static bool directions_apart(const DerivArgs &A, const double *f, const double *const (&x)[2],
+                             const double *const (&y)[2])
+{
+    const size_t n = static_cast<size_t>(A.nx) * A.ny * A.K * sizeof(C);
+    auto apart = [n](const double *p, const double *q) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+        return a + n <= b || b + n <= a;
+    };
+    for (const double *p : {x[0], x[1]})
+        if (!apart(p, f) || !apart(p, y[0]) || !apart(p, y[1])) return false;
+    return apart(y[0], f) && apart(y[1], f);
+}
+
 int derivs4(const DerivArgs &A, const double *f, double *dx, double *dxx, double *dy, double *dyy,
             hipStream_t st)
 {
     const C *fi = reinterpret_cast<const C *>(f);
     int rc = TBL_OK;
-    if (dx && dxx && dy && dyy &&
+    if (dx && dxx && dy && dyy && directions_apart(A, f, {dx, dxx}, {dy, dyy}) &&
         derivs_both(A, fi, reinterpret_cast<C *>(dx), reinterpret_cast<C *>(dxx),
                     reinterpret_cast<C *>(dy), reinterpret_cast<C *>(dyy), st))
         return TBL_OK;

@@ -54,3 +54,27 @@ def test_derivatives_into_overlapping_outputs(torch_mod, nx, ny, nmodes):
             out[q] = f.data_ptr()
             with pytest.raises(tb.TblError):
                 ctx.derivs_dev(f.data_ptr(), *out)
+
+
+def test_creating_a_context_of_many_modes(torch_mod):
+    """A mode costs a context its line factors, on the host, and their upload;
+    their other layouts are the device's work.  128 modes of a narrow tall grid
+    take 4 to 5 times as long as one mode with the factors alone, 16 to 20 times
+    with the layouts formed on the host: at most 8 (the quickest of seven each)."""
+    import time
+
+    import trans_bl_amd as tb
+
+    def create(nmodes):
+        g = wl.Grid(65, 257, nmodes, 3, 0.02, 2e-4, 1.012, 0.0, 0.1)
+        best = np.inf
+        for _ in range(7):
+            t = time.perf_counter()
+            ctx = tb.Context(g)
+            best = min(best, time.perf_counter() - t)
+            ctx.close()
+        return best
+
+    one, many = create(1), create(128)
+    print(f"creation: {1e3 * one:.2f} ms with 1 mode, {1e3 * many:.2f} with 128", flush=True)
+    assert many < 8 * one

@@ -370,47 +370,6 @@ void line_lu(const tbl_grid &g, const tbl_coefs &c, const Metrics &m, int lvl, i
     }
 }
 
-void coarse_inverse(const double *lu, int stride, int ny, const double *sp, const double *cp,
-                    double qx, int rows, int cols, double *out)
-{
-    const double *l1 = lu, *l2 = lu + stride, *u1 = lu + 2 * stride, *u2 = lu + 3 * stride,
-                 *pv = lu + 4 * stride;
-    double *g = out, *G = out + rows, *H = G + static_cast<size_t>(rows) * cols;
-    // the inverse, all columns of a row together
-    const int n = ny;
-    std::vector<double> X(static_cast<size_t>(n) * n, 0.0);
-    auto sub = [&](int j, double w, int i) {          // row j -= w row i
-        double *a = &X[static_cast<size_t>(j) * n];
-        const double *b = &X[static_cast<size_t>(i) * n];
-        for (int c = 0; c < n; ++c) a[c] -= w * b[c];
-    };
-    for (int j = 0; j < n; ++j) {
-        X[static_cast<size_t>(j) * n + j] = 1.0;
-        if (j >= 1) sub(j, l1[j], j - 1);
-        if (j >= 2) sub(j, l2[j], j - 2);
-    }
-    for (int j = n - 1; j >= 0; --j) {
-        if (j + 1 < n) sub(j, u1[j], j + 1);
-        if (j + 2 < n) sub(j, u2[j], j + 2);
-        for (int c = 0; c < n; ++c) X[static_cast<size_t>(j) * n + c] /= pv[j];
-    }
-    // H = qx G Bw: row j of Bw weighs X of rows j-1, j, j+1 (rhs_center); rows
-    // ny-2 and ny-1 take their own X
-    for (int r = 1; r < n; ++r) {
-        const double *x = &X[static_cast<size_t>(r) * n];
-        double *Gr = G + static_cast<size_t>(r - 1) * cols - 1, *Hr = H + static_cast<size_t>(r - 1) * cols - 1;
-        g[r - 1] = x[0];
-        for (int c = 1; c < n; ++c) Gr[c] = x[c];
-        Hr[1] += sp[1] * x[1];
-        Hr[2] += sp[2] * x[1];
-        for (int j = 2; j <= n - 3; ++j)
-            for (int q = 0; q < 3; ++q) Hr[j - 1 + q] += cp[q] * x[j];
-        Hr[n - 2] += x[n - 2];
-        Hr[n - 1] += x[n - 1];
-        for (int c = 1; c < n; ++c) Hr[c] *= qx;
-    }
-}
-
 // Thomas factors of a constant tridiagonal LHS (tridy 947-975): the forward
 // sweep's bet_j and gam_j depend only on the matrix.
 void thomas_factors(const std::vector<double> &a, const std::vector<double> &b,

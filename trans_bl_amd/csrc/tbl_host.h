@@ -23,11 +23,6 @@ void build_metrics(const tbl_grid &g, Metrics &m);
 int check_grid(const tbl_grid &g);
 void line_lu(const tbl_grid &g, const tbl_coefs &c, const Metrics &m, int lvl, int k,
              bool border, double *l1, double *l2, double *u1, double *u2, double *piv);
-// x = G S + g v_0 - H X of one line matrix from its factors (line_lu, fields
-// `stride` apart: l1, l2, u1, u2, pivot): out = g [rows], G [rows][cols], H
-// [rows][cols] over the matrix rows and columns 1..ny-1, zero-padded
-void coarse_inverse(const double *lu, int stride, int ny, const double *sp, const double *cp,
-                    double qx, int rows, int cols, double *out);
 void thomas_factors(const std::vector<double> &a, const std::vector<double> &b,
                     const std::vector<double> &c, std::vector<double> &gam,
                     std::vector<double> &bet);

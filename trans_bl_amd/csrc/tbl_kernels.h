@@ -21,6 +21,9 @@ constexpr int lu_pack_chunks(int esize, int R) { return (lu_pack_values(esize) *
 // elements of one line's packed table
 constexpr int lu_pack_line(int esize, int G, int R) { return lu_pack_chunks(esize, R) * G * (16 / esize); }
 size_t lu_pack_offset(int esize, int K, int ny, int lus, int G);   // G past the last: all elements
+// from the FP64 rows' form at the start of lu: the FP32 one, and the lanes' forms
+// of both
+void prepare_line_lu(double *lu, float *luf, int K, int ny, int lus, hipStream_t st);
 
 // Per-level constants of the Poisson operator (poisson_par.f:229-793)
 template <typename T>
@@ -145,6 +148,10 @@ template <typename T>
 int smooth_coarsest(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, const T *inv,
                     int sweeps, T rf, const int *active, int G, hipStream_t st);
 bool coarse_inv_fits(int nx, int ny);
+// the tables of that form in both precisions, from the level's factors in the
+// rows' form; sp, cp: its Poisson row weights
+void coarse_inverse(const double *lu, int K, int ny, int lus, const double *sp, const double *cp,
+                    double qx, double *inv, float *invf, hipStream_t st);
 template <typename T, typename TO>
 void defect(const LevelArgs<T> &L, const cx<T> *V, const cx<T> *S, cx<TO> *out, T si,
             const int *active, double *resmax, hipStream_t st);

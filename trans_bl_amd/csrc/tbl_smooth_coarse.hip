@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(512) smooth_coarsest_kernel(LevelArgs<T> L, cx
 // depends only on the mode and on centre/border (coef_center / coef_border,
 // poisson_par.f:229-340), so one relaxation of every line of a colour phase
 // is a product with two constant matrices formed at context creation
-// (coarse_inverse, tbl_host.cpp):
+// (coarse_inverse):
 //   x = A^-1 rhs = T - H X,  T = G S + g v_0,  G = (A^-1) rows 1.., H = qx G Bw
 // with X the line's off-diagonal x terms (xoff), S its source, Bw the compact
 // row weights and v_0 its wall value.  T does not change during the sweeps.
@@ -263,6 +263,68 @@ __global__ void __launch_bounds__(THREADS) smooth_coarsest_inv_kernel(LevelArgs<
     }
 }
 
+// The tables of one line matrix (coarse_inv_size): a wavefront per matrix, a
+// column of the inverse per lane, from the banded factors (l1, l2, u1, u2 and
+// the pivot); then H = qx G Bw, where row j of Bw weighs the x terms of rows
+// j-1, j, j+1 (rhs_center) and rows ny-2 and ny-1 take their own.
+constexpr int kInvMaxNy = 33;
+__global__ void __launch_bounds__(64) coarse_inverse_kernel(const double *__restrict__ lu, int lus,
+                                                            int n, double sp1, double sp2,
+                                                            double cp0, double cp1, double cp2,
+                                                            double qx, double *__restrict__ inv,
+                                                            float *__restrict__ invf)
+{
+    __shared__ double X[kInvMaxNy * kInvMaxNy];      // [row][column]
+    const double *l1 = lu + static_cast<size_t>(blockIdx.x) * kLuFields * lus, *l2 = l1 + lus,
+                 *u1 = l2 + lus, *u2 = u1 + lus, *pv = u2 + lus;
+    const int c = threadIdx.x;
+    if (c < n) {
+        double a = 0.0, b = 0.0;
+        for (int j = 0; j < n; ++j) {
+            double x = j == c ? 1.0 : 0.0;
+            if (j >= 1) x -= l1[j] * a;
+            if (j >= 2) x -= l2[j] * b;
+            X[j * n + c] = x;
+            b = a;
+            a = x;
+        }
+        a = b = 0.0;
+        for (int j = n - 1; j >= 0; --j) {
+            double x = X[j * n + c];
+            if (j + 1 < n) x -= u1[j] * a;
+            if (j + 2 < n) x -= u2[j] * b;
+            x /= pv[j];
+            X[j * n + c] = x;
+            b = a;
+            a = x;
+        }
+    }
+    __syncthreads();
+    const int cols = coarse_inv_cols(n), rows = coarse_inv_rows(n), size = rows * (1 + 2 * cols);
+    for (int e = threadIdx.x; e < size; e += 64) {
+        const int m = e < rows ? e : (e - rows) % (rows * cols);
+        const int r = 1 + (e < rows ? m : m / cols), k = e < rows ? 0 : 1 + m % cols;
+        double v = 0.0;
+        if (r < n && k < n) {
+            const double *x = X + r * n;
+            if (e < rows + rows * cols) {
+                v = x[k];
+            } else {
+                if (k == 1) v += sp1 * x[1];
+                if (k == 2) v += sp2 * x[1];
+                if (k >= 3 && k <= n - 2) v += cp2 * x[k - 1];
+                if (k >= 2 && k <= n - 3) v += cp1 * x[k];
+                if (k <= n - 4) v += cp0 * x[k + 1];
+                if (k >= n - 2) v += x[k];
+                v *= qx;
+            }
+        }
+        const size_t o = static_cast<size_t>(blockIdx.x) * size + e;
+        inv[o] = v;
+        invf[o] = static_cast<float>(v);
+    }
+}
+
 // k-steps of a level's row count
 inline int coarse_inv_steps(int ny) { return std::max(2, (ny + 2) / 4); }
 #define TBL_COARSE_KS(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
@@ -353,8 +415,15 @@ int coarse_kernel_attributes()
 // 15 wavefronts of lines and the part's v in LDS
 bool coarse_inv_fits(int nx, int ny)
 {
-    return ny - 1 <= 32 && (phase_lines(1, nx) + 15) / 16 < 16 &&
+    return ny <= kInvMaxNy && (phase_lines(1, nx) + 15) / 16 < 16 &&
            coarse_inv_lds<double>(nx, ny) <= 160 * 1024;
+}
+
+void coarse_inverse(const double *lu, int K, int ny, int lus, const double *sp, const double *cp,
+                    double qx, double *inv, float *invf, hipStream_t st)
+{
+    hipLaunchKernelGGL(coarse_inverse_kernel, dim3(2 * K), dim3(64), 0, st, lu, lus, ny, sp[1], sp[2],
+                       cp[0], cp[1], cp[2], qx, inv, invf);
 }
 
 template int smooth_coarsest<double>(const LevelArgs<double> &, cx<double> *, const cx<double> *,

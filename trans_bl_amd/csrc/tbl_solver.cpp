@@ -14,27 +14,6 @@
 using namespace tbl;
 
 namespace {
-
-// appends the lanes' form of the tables (tbl_kernels.h) to the rows' form
-template <typename T>
-void pack_lu(std::vector<T> &lu, int K, int ny, int lus)
-{
-    constexpr int es = sizeof(T), NF = lu_pack_values(es), CV = 16 / es;
-    static const int field[8] = {0, 1, 2, 3, 5, 6, 7, 4};
-    lu.resize(lu_pack_offset(es, K, ny, lus, 0), T(0));
-    for (int G : kLuLanes) {
-        const int R = line_rows_for(G, ny);
-        if (R <= 0) continue;
-        const size_t size = lu_pack_line(es, G, R);
-        for (int q = 0; q < 2 * K; ++q) {
-            const T *src = &lu[static_cast<size_t>(q) * kLuFields * lus];
-            T *dst = &lu[lu_pack_offset(es, K, ny, lus, G) + q * size];
-            for (int lane = 0; lane < G; ++lane)
-                for (int v = 0; v < NF * R; ++v)
-                    dst[(v / CV * G + lane) * CV + v % CV] = src[field[v / R] * lus + 1 + lane * R + v % R];
-        }
-    }
-}
 thread_local std::string g_last_error;
 }
 
@@ -175,7 +154,6 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
         const int d = lu_stride(lv.ny);
         const size_t per = static_cast<size_t>(kLuFields) * d;
         std::vector<double> lu(per * 2 * K, 0.0);
-        std::vector<float> luf(lu.size(), 0.0f);
         for (int k = 0; k < K; ++k)
             for (int t = 0; t < 2; ++t) {
                 double *b = &lu[(static_cast<size_t>(k) * 2 + t) * per];
@@ -193,26 +171,17 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
                     b[7 * d + j] = 1.0;
                 }
             }
-        for (size_t e = 0; e < lu.size(); ++e) luf[e] = static_cast<float>(lu[e]);
-        pack_lu(lu, K, lv.ny, d);
-        pack_lu(luf, K, lv.ny, d);
-        TRY(dalloc(&c->lu_d[l], lu.size()));
-        TRY(dalloc(&c->lu_f[l], luf.size()));
+        TRY(dalloc(&c->lu_d[l], lu_pack_offset(sizeof(double), K, lv.ny, d, 0)));
+        TRY(dalloc(&c->lu_f[l], lu_pack_offset(sizeof(float), K, lv.ny, d, 0)));
         TBL_HIP(hipMemcpy(c->lu_d[l], lu.data(), sizeof(double) * lu.size(), hipMemcpyHostToDevice));
-        TBL_HIP(hipMemcpy(c->lu_f[l], luf.data(), sizeof(float) * luf.size(), hipMemcpyHostToDevice));
+        prepare_line_lu(c->lu_d[l], c->lu_f[l], K, lv.ny, d, nullptr);
         // the coarsest level's inverse form, from the factors of each line matrix
         if (l == L - 1 && coarse_inv_fits(lv.nx, lv.ny)) {
-            const size_t sz = coarse_inv_size(lv.ny);
-            std::vector<double> inv(sz * 2 * K, 0.0);
-            for (int q = 0; q < 2 * K; ++q)
-                coarse_inverse(&lu[q * per], d, lv.ny, c->c.sp_poi[l], c->c.cp_poi[l],
-                               1.0 / (12.0 * c->m.dx2[l] * c->g.fac_y), coarse_inv_rows(lv.ny),
-                               coarse_inv_cols(lv.ny), &inv[q * sz]);
-            const std::vector<float> invf(inv.begin(), inv.end());
-            TRY(dalloc(&c->inv_d, inv.size()));
-            TRY(dalloc(&c->inv_f, invf.size()));
-            TBL_HIP(hipMemcpy(c->inv_d, inv.data(), sizeof(double) * inv.size(), hipMemcpyHostToDevice));
-            TBL_HIP(hipMemcpy(c->inv_f, invf.data(), sizeof(float) * invf.size(), hipMemcpyHostToDevice));
+            const size_t sz = coarse_inv_size(lv.ny) * 2 * K;
+            TRY(dalloc(&c->inv_d, sz));
+            TRY(dalloc(&c->inv_f, sz));
+            coarse_inverse(c->lu_d[l], K, lv.ny, d, c->c.sp_poi[l], c->c.cp_poi[l],
+                           1.0 / (12.0 * c->m.dx2[l] * c->g.fac_y), c->inv_d, c->inv_f, nullptr);
         }
         c->G64[l] = default_shape(lv, K, sizeof(cx<double>));
         c->G32[l] = default_shape(lv, K, sizeof(cx<float>));
@@ -323,6 +292,7 @@ static int create_impl(const tbl_grid *grid, const tbl_coefs *coefs, tbl_ctx *c)
     c->stream = c->own_stream;
     TBL_HIP(hipEventCreate(&c->ev0));
     TBL_HIP(hipEventCreate(&c->ev1));
+    TBL_HIP(hipGetLastError());
     TBL_HIP(hipDeviceSynchronize());
     return TBL_OK;
 }

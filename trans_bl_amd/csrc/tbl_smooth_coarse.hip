@@ -89,8 +89,8 @@ __global__ void __launch_bounds__(512) smooth_coarsest_kernel(LevelArgs<T> L, cx
 // takes one part (re or im: the operator is real) of one mode; a wavefront
 // owns 16 lines of each colour, their v and T in registers in the result
 // layout, and forms the operand X straight from the v columns in LDS; the two
-// border lines are one further wavefront's scalar products.  Per call, banded
-// substitution -> inverse form: FP64, 60 sweeps, 49x13x8 251 -> 70 us,
+// border lines are one further wavefront's scalar products.  Per call between
+// events, banded substitution -> inverse form: FP64, 60 sweeps, 49x13x8 251 -> 70 us,
 // 129x25x64 424 -> 160, 257x33x128 1774 -> 309, 129x24x20 (the lane scan) 1035
 // -> 159; FP32, 5 sweeps, 129x25x64 32 -> 22.
 // 16 NB rows and 4 KS columns hold the ny - 1 rows; THREADS bounds the
@@ -343,8 +343,9 @@ int smooth_coarsest(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu
                     int sweeps, T rf, const int *active, int G, hipStream_t st)
 {
     // shape kCoarseSeqShape: the inverse form where the context holds its
-    // tables (coarse_inv_fits: it was faster at every size that fits, 49x13 to
-    // 257x33); any other shape, or a level it does not fit, the G-lane scan
+    // tables (coarse_inv_fits: faster at every size class of 33x9 to 257x33, six
+    // FP64 sweeps 1.9-7.9 times, 33x33x16 29 against 54 us, 257x33x128 57 against
+    // 163); any other shape, or a level it does not fit, the G-lane scan
     if (G == kCoarseSeqShape && inv) {
         const int ks = coarse_inv_steps(L.ny);
         const unsigned waves = static_cast<unsigned>((phase_lines(1, L.nx) + 15) / 16) + 1;

@@ -275,7 +275,7 @@ typedef struct tbl_base {
 
 /* kphys 0: lterms_gv (nlterms_par.f:89-112, the reference's active call);
    otherwise nlterms_gv (115-180) with kphys points in z (a power of two,
-   >= 2 nmodes): a, b, c, d out. */
+   >= 2 nmodes, 4 to 1024): a, b, c, d out. */
 int tbl_terms_dev(tbl_ctx *ctx, int kphys, const tbl_base *base, const double *d_ux,
                   const double *d_uy, const double *d_uz, const double *d_wx,
                   const double *d_wy, const double *d_wz, double *d_a, double *d_b, double *d_c,
@@ -298,7 +298,7 @@ int tbl_drv_gv(tbl_ctx *ctx, double Re, int kphys, const double *uxb, const doub
 /* Flat-plate form (my_form 0, main_par.f:155-230).  kphys 0: lterms_fi
    (nlterms_par.f:6-38; base->uxb, uyb, wzb used); otherwise nlterms_fi
    (41-86, the reference's active call; base may be NULL) with kphys points
-   in z (a power of two, >= 2 nmodes): a, b, c out. */
+   in z (a power of two, >= 2 nmodes, 4 to 1024): a, b, c out. */
 int tbl_terms_fi_dev(tbl_ctx *ctx, int kphys, const tbl_base *base, const double *d_ux,
                      const double *d_uy, const double *d_uz, const double *d_wx,
                      const double *d_wy, const double *d_wz, double *d_a, double *d_b,

@@ -3,6 +3,7 @@ result must not."""
 import numpy as np
 import pytest
 
+import oracle
 from trans_bl_amd import workload as wl
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +79,34 @@ def test_creating_a_context_of_many_modes(torch_mod):
     one, many = create(1), create(128)
     print(f"creation: {1e3 * one:.2f} ms with 1 mode, {1e3 * many:.2f} with 128", flush=True)
     assert many < 8 * one
+
+
+@pytest.mark.parametrize("nmodes, kphys", [(256, 512), (43, 1024), (300, 1024), (512, 1024)])
+def test_nonlinear_terms_of_many_modes(torch_mod, nmodes, kphys):
+    """Every mode count up to kphys / 2 at the largest kphys, against the oracle
+    (1e-13 as at the other sizes; the oracle lies 8e-15 from numpy's FFT here)."""
+    torch = torch_mod
+    import trans_bl_amd as tb
+    g = wl.Grid(33, 17, nmodes, 2, 0.02, 1e-3, 1.02, 0.0, 0.3)
+    rng = np.random.default_rng(nmodes)
+    names = ("ux", "uy", "uz", "wx", "wy", "wz")
+    scale = dict(zip(names, (1.0, 1e-3, 0.1, 1e-2, 10.0, 1e-6)))
+    F = {k: scale[k] * (rng.normal(size=(nmodes, 17, 33)) + 1j * rng.normal(size=(nmodes, 17, 33))) for k in names}
+    base = {k: rng.normal(size=(17, 33)) for k in ("uxb", "uyb", "wzb", "varg", "dvargdx")}
+    p = oracle.make_params(g.nx, g.ny, g.nmodes, g.levels, g.dx, g.dy0, g.stf, g.alpha, g.beta)
+    with tb.Context(g) as ctx:
+        d = {k: torch.from_numpy(F[k]).to("cuda") for k in names}
+        db = {k: torch.from_numpy(base[k]).to("cuda") for k in base}
+        out = [torch.zeros_like(d["ux"]) for _ in range(4)]
+        ctx.terms_dev(kphys, {k: v.data_ptr() for k, v in db.items()}, *[d[k].data_ptr() for k in names],
+                      *[o.data_ptr() for o in out])
+        fi = [torch.zeros_like(d["ux"]) for _ in range(3)]
+        ctx.terms_fi_dev(kphys, None, *[d[k].data_ptr() for k in names], *[o.data_ptr() for o in fi])
+        ctx.synchronize()
+        for bad in (kphys + 2, kphys // 2 if 2 * nmodes > kphys // 2 else kphys + 2, 2048):
+            with pytest.raises(tb.TblError):
+                ctx.terms_dev(bad, {k: v.data_ptr() for k, v in db.items()}, *[d[k].data_ptr() for k in names],
+                              *[o.data_ptr() for o in out])
+    for o, ref in zip(out + fi, oracle.terms(p, kphys, base, F) + oracle.terms_fi(p, kphys, None, F)):
+        o = o.cpu().numpy()
+        assert np.max(np.abs(o - ref)) < 1e-13 * np.max(np.abs(ref))

@@ -38,7 +38,7 @@ struct RkArgs {
     int stage, nx, ny, K;
 };
 
-bool nlterms_fits(int K, int N);   // kphys values the nonlinear terms accept
+bool nlterms_fits(int N);   // kphys values the nonlinear terms accept
 int terms(const RhsArgs &r, int kphys, hipStream_t st);
 int drv_combine(const DrvArgs &r, hipStream_t st);
 // the derivatives and the combination in six launches (tbl_drv.hip); lin: the

@@ -289,6 +289,8 @@ __global__ void __launch_bounds__(256) nlterms_kernel(RhsArgs r)
     if (M > 1) put(m2, c2, n2);
 }
 
+// the kphys values (LDS: six half-length sequences and the twiddles, 72 KB at 1024
+// whatever the number of modes; 256 threads hold at most 1024 values)
 #define TBL_NL_SIZES(X) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
 
 // drv_gv's combination (main_par.f:1380-1397), rows 2..ny
@@ -355,11 +357,13 @@ __global__ void pert_kernel(cxd *uy, cxd *d2, const cxd *pu, const cxd *pd, int 
 
 }  // namespace
 
-bool nlterms_fits(int K, int N)
+bool nlterms_fits(int N)
 {
-    // the modes and values of 4 points and the twiddles within 160 KB of LDS
-    return sizeof(double) * (2 * 6 * 4 * static_cast<size_t>(K) + (4 * 4 + 2) * static_cast<size_t>(N)) <=
-           160 * 1024;
+#define X(NN) \
+    if (N == NN) return true;
+    TBL_NL_SIZES(X)
+#undef X
+    return false;
 }
 
 int terms(const RhsArgs &r, int kphys, hipStream_t st)

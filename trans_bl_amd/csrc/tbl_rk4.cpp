@@ -45,7 +45,7 @@ int check_kphys(const tbl_ctx *c, int kphys)
     if (kphys == 0) return TBL_OK;
     if (kphys < 4 || kphys < 2 * c->K || (kphys & (kphys - 1)))
         return fail("kphys must be 0 (linear terms) or a power of two >= max(4, 2 nmodes)");
-    if (!nlterms_fits(c->K, kphys)) return fail("kphys too large for the LDS");
+    if (!nlterms_fits(kphys)) return fail("kphys above 1024");
     return TBL_OK;
 }
 

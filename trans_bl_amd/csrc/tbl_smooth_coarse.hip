@@ -344,7 +344,7 @@ int smooth_coarsest(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu
 {
     // shape kCoarseSeqShape: the inverse form where the context holds its
     // tables (coarse_inv_fits: faster at every size class of 33x9 to 257x33, six
-    // FP64 sweeps 1.9-7.9 times, 33x33x16 29 against 54 us, 257x33x128 57 against
+    // FP64 sweeps 1.8 to 7.8 times, 33x33x16 29 against 54 us, 257x33x128 57 against
     // 163); any other shape, or a level it does not fit, the G-lane scan
     if (G == kCoarseSeqShape && inv) {
         const int ks = coarse_inv_steps(L.ny);

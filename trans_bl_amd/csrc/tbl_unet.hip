@@ -1171,7 +1171,9 @@ void conv3x3(int n, int h, int w, int cin, int cout, const bf16 *x, const bf16 *
 
 // ---- backward launchers ------------------------------------------------------
 constexpr size_t kBwdLds = 160 * 1024;
-// tiles of 32 input channels per workgroup (and 3 - nt pixel tiles a wavefront)
+// conv3x3_dx_kernel's forms: pixel tiles a wavefront, tiles of 32 input channels a
+// workgroup, output channels
+#define TBL_DX_SHAPES(X) X(2, 1, 32) X(2, 1, 64) X(1, 2, 64) X(1, 2, 128) X(1, 2, 256)
 static int dx_nt(int cin, int cout) { return cin % 64 == 0 && cout != 32 ? 2 : 1; }
 static size_t dx_lds(int px, int w, int ct, int cout)
 {
@@ -1192,9 +1194,12 @@ static int dw_chunks(int cout) { return cout % 128 == 0 ? 4 : cout % 64 == 0 ? 2
 bool conv3x3_back_fits(int w, int cin, int cout)
 {
     const int nc = dw_chunks(cout);
-    const bool co = cout == 32 || cout == 64 || cout == 128 || cout == 256;
     const int nt = dx_nt(cin, cout);
-    return co && cin % 4 == 0 && dw_lds(w, nc) <= kBwdLds &&
+    bool form = false;
+#define X(MT, NT, CO) form = form || (nt == NT && cout == CO);
+    TBL_DX_SHAPES(X)
+#undef X
+    return form && cin % 4 == 0 && dw_lds(w, nc) <= kBwdLds &&
            dx_lds(128 * (3 - nt), w, 32 * nt, cout) <= kBwdLds &&
            static_cast<long>(dw_rows(w, nc) + 3) * (w + 2) * (kWgRow / 4) < 65536;
 }
@@ -1222,7 +1227,6 @@ void conv3x3_dw(int n, int h, int w, int cin, int cout, const bf16 *x, const bf1
         hipLaunchKernelGGL(conv3x3_dw_kernel<1>, grid, dim3(256), lds, st, n * h, h, w, nr, ks, cin, cout, x, dz, ws);
 }
 
-#define TBL_DX_SHAPES(X) X(2, 1, 32) X(2, 1, 64) X(1, 2, 64) X(1, 2, 128) X(1, 2, 256) X(2, 1, 128) X(2, 1, 256)
 void conv3x3_dx(int n, int h, int w, int cin, int cout, const bf16 *dz, const bf16 *wb, float *dx,
                 hipStream_t st)
 {

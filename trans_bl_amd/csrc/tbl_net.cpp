@@ -15,7 +15,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <random>
 #include <string>
 #include <vector>
@@ -307,10 +306,8 @@ extern "C" int tbl_net_create(int H, int W, int max_batch, unsigned seed, tbl_ne
     n->H = H;
     n->W = W;
     n->nmax = max_batch;
-    static std::once_flag attr_once;
-    static int attr_rc = TBL_OK;
-    std::call_once(attr_once, [] { attr_rc = nn_kernel_attributes(); });
-    int rc = attr_rc;
+    // the attributes belong to the current device: set for every network
+    int rc = nn_kernel_attributes();
     if (rc == TBL_OK) rc = net_alloc(n);
     if (rc == TBL_OK) {
         std::vector<float> h;

@@ -21,7 +21,7 @@ ARCH = os.environ.get("TBL_OFFLOAD_ARCH", "gfx950")
 
 COMMON = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
-    # no fused multiply-add: FP64 results follow the reference's rounding
+    # no fused multiply-add but the written ones (__builtin_fma)
     "-ffp-contract=off",
     # packed FP32 instructions stay disabled
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

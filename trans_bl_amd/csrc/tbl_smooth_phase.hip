@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(256) smooth_staged_kernel(LevelArgs<T> L, cx<T
             const int j = 1 + lane + r * G;
             if (j < ny) {
                 cx<T> x;
-                // the sums of xoff in its order (multiply-adds in FP32)
+                // the sums of xoff in its order, as multiply-adds
                 if (side)
                     x = mac(T(-6), a3[r], mac(T(14), a2[r], mac(T(-4), a1[r], T(10) * a0[r])))
                         + a4[r];

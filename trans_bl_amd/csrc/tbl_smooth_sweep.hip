@@ -139,7 +139,7 @@ __device__ __forceinline__ void sweep_relax(const LevelArgs<T> &L, __amdgpu_buff
         const int j = 1 + lane + r * G;
         if (j < ny) {
             cx<T> x;
-            // the sums of xoff in its order (multiply-adds in FP32)
+            // the sums of xoff in its order, as multiply-adds
             if (side)
                 x = mac(T(-6), in.a3[r],
                         mac(T(14), in.a2[r], mac(T(-4), in.a1[r], T(10) * in.a0[r]))) +

@@ -849,7 +849,6 @@ __global__ void col2im_kernel(int Nn, int H, int W, int Cc, const float *dcol, f
     dX[e] = accumulate ? dX[e] + s : s;
 }
 
-// y = relu(z + b) -> bf16 (relu = 0: identity, fp32 output kept in z)
 // The output layer, 1x1 from 32 channels to 2, with bias: four lanes a pixel, 8
 // channels (16 bytes) each, fp32 sums.  A 64-wide GEMM tile has no use for two
 // columns, and its bias took a pass of its own: 64 images of 32x136 (20 MB)

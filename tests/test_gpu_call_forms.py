@@ -110,3 +110,26 @@ def test_nonlinear_terms_of_many_modes(torch_mod, nmodes, kphys):
     for o, ref in zip(out + fi, oracle.terms(p, kphys, base, F) + oracle.terms_fi(p, kphys, None, F)):
         o = o.cpu().numpy()
         assert np.max(np.abs(o - ref)) < 1e-13 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("nx, ny, nmodes", [(17, 9, 3), (33, 59, 1), (35, 59, 2), (65, 61, 5), (129, 121, 7), (1025, 193, 2)],
+                         ids=lambda v: str(v))
+def test_residual_maxima(torch_mod, nx, ny, nmodes):
+    """Each mode's largest residual is that of the field written (2 units in the
+    last place: a square root of a sum of squares against numpy's hypot), with
+    one to four wavefronts in a mode's last workgroup; the largest may lie in any
+    of them."""
+    torch = torch_mod
+    import trans_bl_amd as tb
+    g = wl.Grid(nx, ny, nmodes, 2 if ny % 2 else 1, 0.02, 1e-3, 1.004, 0.0, 0.3)
+    f = random_field(torch, g)
+    rng = np.random.default_rng(ny)
+    with tb.Context(g) as ctx:
+        v, out = torch.zeros_like(f), torch.zeros_like(f)
+        for _ in range(6):
+            k, j, i = rng.integers(nmodes), rng.integers(1, ny), rng.integers(1, nx - 1)
+            f[k, j, i] = 1e3 * (1 + 1j)
+            torch.cuda.synchronize()
+            res = ctx.residual_dev(0, f.data_ptr(), v.data_ptr(), out.data_ptr())
+            ref = np.abs(out.cpu().numpy()).max(axis=(1, 2))
+            assert ref[k] > 100 and np.all(np.abs(res - ref) <= 4.5e-16 * ref)

@@ -92,12 +92,23 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
                                                            CoarseOut<TO> co)
 {
     constexpr int kRows = RS ? kDefRowsRs : kDefRows, kHalo = RS ? 3 : 2;
-    constexpr bool kInj = RS && sizeof(T) == 8;
+    constexpr bool kInj = RS && sizeof(T) == 8, kMax = sizeof(T) == 8;
     const int lane = threadIdx.x & 63;
     const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int k = blockIdx.y;
-    if (item >= jchunks * nstrips) return;          // whole wavefront
     if (active && !active[k]) return;
+    __shared__ unsigned long long block_max;        // bits of the workgroup's largest |r|^2
+    __shared__ int block_left;                      // its wavefronts still at work
+    if constexpr (kMax) {
+        if (resmax) {
+            if (threadIdx.x == 0) {
+                block_max = 0;
+                block_left = min(4, jchunks * nstrips - static_cast<int>(blockIdx.x) * 4);
+            }
+            __syncthreads();
+        }
+    }
+    if (item >= jchunks * nstrips) return;          // whole wavefront
     const int nx = L.nx, ny = L.ny, ld = L.ld;
     const int jc = item % jchunks, sc = item / jchunks;
     const int j = 1 + jc * kRows - kHalo + lane;
@@ -236,7 +247,7 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
                 const cx<T> r = mac(si, lv, s_cur);   // s + si lv
                 rv = r;
                 if (!RS) out[o] = cx<TO>{static_cast<TO>(r.re), static_cast<TO>(r.im)};
-                if ((!RS || kInj) && resmax) {
+                if (kMax && resmax) {
                     // max of |r|^2; one square root per wavefront below
                     // (sqrt is monotone and correctly rounded: same maximum)
                     const double rr = static_cast<double>(r.re), ri = static_cast<double>(r.im);
@@ -277,9 +288,17 @@ __global__ void __launch_bounds__(256) defect_march_kernel(LevelArgs<T> L,
             sq[t] = ns[t];
         }
     }
-    if (resmax) {
-        for (int o = 32; o > 0; o >>= 1) amax = fmax(amax, __shfl_down(amax, o, 64));
-        if (lane == 0) atomic_max_nonneg<T>(resmax + k, sqrt(amax));
+    if constexpr (kMax) {
+        if (resmax) {
+            // one update per workgroup, by the wavefront that ends last (updates of
+            // one address queue: 1020 from the short strips of 1021x233x6 took 47 us)
+            for (int o = 32; o > 0; o >>= 1) amax = fmax(amax, __shfl_down(amax, o, 64));
+            if (lane == 0) {
+                atomicMax(&block_max, __double_as_longlong(amax));
+                if (__hip_atomic_fetch_sub(&block_left, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 1)
+                    atomic_max_nonneg<T>(resmax + k, sqrt(__longlong_as_double(atomicMax(&block_max, 0ull))));
+            }
+        }
     }
 }
 

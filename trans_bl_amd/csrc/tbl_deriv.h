@@ -344,8 +344,10 @@ __device__ __forceinline__ void y_solve(double (&a)[R], double (&b)[R], const do
 // wavefronts that hide the recurrences' latency)
 #define TBL_X_SHAPES(X) \
     X(2, 1) X(3, 1) X(5, 1) X(7, 1) X(9, 1) X(5, 2) X(7, 2) X(9, 2) X(7, 3) X(9, 3) X(7, 4) X(9, 4)
-// columns of a y workgroup's tile
+// columns of a y workgroup's tile, and the stride of a column's plane in it
 constexpr int kDerivYCols = 8;
+template <int TX>
+__host__ __device__ constexpr int y_stride(int rows) { return rows + 32 / TX; }
 // y shapes (G, R): the first that holds the rows; R odd (an even lane stride
 // puts the lanes of a column on few banks: 97 rows as 32 x 4 took 252 us for
 // both derivatives of 1025x97x128, as 16 x 7 149)

@@ -11,8 +11,8 @@
 //    derivs_par.f:80-113, 259-397, 775-858): a workgroup per x-line (j, k), W
 //    wavefronts per part, R consecutive points per lane.
 //  * y (dery/deryy/deryfv, rhsy/rhsyy/rhsyfv + tridy, derivs_par.f:116-177,
-//    400-611, 947-975): a workgroup holds a tile of 8 columns x all ny rows of
-//    one mode; G lanes per column and part, R rows per lane.
+//    400-611, 947-975): a workgroup holds a tile of 8 or 4 columns x all ny rows
+//    of one mode; G lanes per column and part, R rows per lane.
 // Results go back through LDS and out as coalesced rows.
 //
 // Thomas solve: u_j = r_j / bet_j - p_j u_{j-1} and x_j = u_j - g_j x_{j+1},
@@ -105,19 +105,24 @@ __global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
 }
 
 // y-lines: o1 = d/dy (fv: with the wall row forced, deryfv), o2 = d2/dy2 of f.
-// Workgroup: 8 columns x all rows of one mode, both parts, in LDS (column
-// stride LP, 4 past a multiple of 32 values: the 8 columns x 4 rows of half a
-// wavefront's tile accesses fall on different banks); G lanes per column and
-// part.  Interior rows: rhsy, rhsyy in the reference's sums, times the metric
+// Workgroup: TX columns x all rows of one mode, both parts, in LDS (column
+// stride LP, 32 / TX past a multiple of 32 values: the TX columns x 32 / TX rows of
+// half a wavefront's tile accesses fall on different banks); G lanes per column
+// and part.  Interior rows: rhsy, rhsyy in the reference's sums, times the metric
 // of the spacing the generator normalised to (v_qdy(j-2), v_qdy2(j-2, 1);
 // 1-based j) over the pivot; every row has its own table entry, at a constant
 // offset from the lane's first.  The stores do not stream: a row's 128 bytes
 // are rarely one cache line (with nt 8 of 9 sizes were up to 50 % slower).
+// 8 columns, 4 with 64 lanes each: 1024 threads are a CU's only workgroup, and its
+// load, solve and store phases overlap with nothing (us, one derivative and both:
+// 569x545x8 27.2, 38.8 with 8 columns, 21.9, 31.6 with 4; 1025x321x64 220, 368 and
+// 175, 281)
+__host__ __device__ constexpr int y_cols(int G) { return G == 64 ? 4 : kDerivYCols; }
 template <int G, int R, bool D1, bool D2>
 __device__ __forceinline__ void deriv_y_tile(const DerivArgs &A, int block, const C *f, C *o1, int fv,
                                              C *o2)
 {
-    constexpr int TX = kDerivYCols, NT = 2 * TX * G, N = (R + 1) / 2, M = G * R, LP = M + 4;
+    constexpr int TX = y_cols(G), NT = 2 * TX * G, N = (R + 1) / 2, M = G * R, LP = y_stride<TX>(M);
     constexpr int NTAB = 6 * M + 64;
     extern __shared__ double ylds[];
     double *planes = ylds, *tab = ylds + 2 * TX * LP;
@@ -149,7 +154,7 @@ __device__ __forceinline__ void deriv_y_tile(const DerivArgs &A, int block, cons
                 re[2 * G * q] = v[q].re;
                 im[2 * G * q] = v[q].im;
             }
-        if (t < 64) planes[t / 4 * LP + (t % 4 < 2 ? t % 4 : M + t % 4)] = 0.0;
+        if (t < 8 * TX) planes[t / 4 * LP + (t % 4 < 2 ? t % 4 : M + t % 4)] = 0.0;
         tc.store(tab, t);
     }
     __syncthreads();
@@ -177,7 +182,7 @@ __device__ __forceinline__ void deriv_y_tile(const DerivArgs &A, int block, cons
 }
 
 template <int G, int R, bool D1, bool D2>
-__global__ void __launch_bounds__(16 * G) deriv_y_kernel(DerivArgs A, const C *__restrict__ f,
+__global__ void __launch_bounds__(2 * y_cols(G) * G) deriv_y_kernel(DerivArgs A, const C *__restrict__ f,
                                                          C *__restrict__ o1, int fv,
                                                          C *__restrict__ o2)
 {
@@ -315,9 +320,10 @@ int deriv_y_rows(int ny, int *G, int *R)
 }
 
 // bytes of LDS of a y workgroup: the tile's planes and the tables
-static size_t y_lds(int rows)
+static size_t y_lds(int G, int rows)
 {
-    return (static_cast<size_t>(2 * kDerivYCols) * (rows + 4) + 6 * rows + 64) * sizeof(double);
+    const size_t tx = y_cols(G);
+    return (2 * tx * (rows + 32 / tx) + 6 * rows + 64) * sizeof(double);
 }
 
 static int deriv_y(const DerivArgs &A, const C *f, C *o1, int fv, C *o2, hipStream_t st)
@@ -330,12 +336,12 @@ static int deriv_y(const DerivArgs &A, const C *f, C *o1, int fv, C *o2, hipStre
         if (o2) hipLaunchKernelGGL(deriv_y_line_kernel, g2, dim3(64), 0, st, A, 3, f, o2);
         return TBL_OK;
     }
-    const int tiles = (A.nx + kDerivYCols - 1) / kDerivYCols * A.K;
+    const int tiles = (A.nx + y_cols(G) - 1) / y_cols(G) * A.K;
     const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8));
-    const size_t lds = y_lds(rows);
+    const size_t lds = y_lds(G, rows);
 #define X(GG, RR)                                                                               \
     if (G == GG && R == RR) {                                                                   \
-        const dim3 block(16 * GG);                                                              \
+        const dim3 block(2 * y_cols(GG) * GG);                                                              \
         if (o1 && o2)                                                                           \
             hipLaunchKernelGGL((deriv_y_kernel<GG, RR, true, true>), grid, block, lds, st, A,   \
                                f, o1, fv, o2);                                                  \
@@ -383,7 +389,7 @@ static bool derivs_both(const DerivArgs &A, const C *f, C *dx, C *dxx, C *dy, C 
     const long tiles = (A.nx + kDerivYCols - 1) / kDerivYCols * static_cast<long>(A.K);
     const long ybs = (tiles + 7) / 8 * 8, blocks = ybs + static_cast<long>(A.ny) * A.K;
     if (blocks > kBothBlocks) return false;
-    const size_t lds = y_lds(rows);
+    const size_t lds = y_lds(G, rows);
 #define XY(RRX, RRY)                                                                              \
     if (RX == RRX && RY == RRY) {                                                                 \
         hipLaunchKernelGGL((deriv_both_kernel<RRX, RRY>), dim3(static_cast<unsigned>(blocks)),    \

@@ -20,8 +20,9 @@
 // the host.  Each direction is a local solve from a zero state, a scan of the
 // lanes' affine maps and the homogeneous response of the incoming state.  The
 // interior rows' weights are constants (also in y: the grid's ratio is), so
-// the factors converge within 64 rows to the last bit or its neighbour and
-// every row beyond reads one entry: the tables (kTriRows entries) sit in LDS.
+// the factors converge within 64 rows to the last bit or its neighbour: in x
+// every row beyond reads one entry (kTriRows in all), in y, where a row has its
+// own metric, each its own.  The tables sit in LDS.
 // (Read from global memory, as 6 lane-segmented loads per row or 3 of the
 // short tables, the address and data units were 85-98 % busy.)
 //

@@ -162,7 +162,9 @@ __device__ __forceinline__ void nl_up(cxd *x, const cxd *tw)
 // registers.  A thread keeps the modes m and M - m of a point from the load to
 // the base-flow terms.  As a direct DFT (O(K N) per point, 65 GFLOP at
 // 1025x193x64 with N = 128) this kernel was bound by FP64 arithmetic: 3466 us;
-// as FFTs by its LDS passes and memory (10 fields of 203 MB): 619 us.
+// as FFTs by its LDS passes and memory (10 fields of 203 MB): 619 us.  From N = 512
+// a workgroup's two points, or one, read 32 or 16 bytes of each cache line: 513x97x200
+// with N = 512 688 us for 305 of bytes (direct 16100), 513x97x42 with 1024 1320 (7370).
 template <int N, bool FI>
 __global__ void __launch_bounds__(256) nlterms_kernel(RhsArgs r)
 {

@@ -133,3 +133,52 @@ def test_residual_maxima(torch_mod, nx, ny, nmodes):
             res = ctx.residual_dev(0, f.data_ptr(), v.data_ptr(), out.data_ptr())
             ref = np.abs(out.cpu().numpy()).max(axis=(1, 2))
             assert ref[k] > 100 and np.all(np.abs(res - ref) <= 4.5e-16 * ref)
+
+
+@pytest.mark.parametrize("shape", [0, 64], ids=["default", "direct"])
+def test_line_factors_past_4_gigabytes(torch_mod, shape):
+    """58400 modes of 545 rows: the FP64 factors of 64 lanes take 4.3 GB, past what
+    one buffer resource reaches.  Two cycles of the last modes, staged (the
+    default) and direct, against a context of two modes with the same kz (1e-12, as
+    other forms of one sweep)."""
+    torch = torch_mod
+    import trans_bl_amd as tb
+    if torch.cuda.mem_get_info()[0] < 140 << 30:
+        pytest.skip("needs 140 GiB of device memory")
+    nx, ny, K, beta = 15, 545, 58400, 1e-4
+    rng = np.random.default_rng(5)
+    one = torch.from_numpy(rng.normal(size=(1, ny, nx)) + 1j * rng.normal(size=(1, ny, nx))).to("cuda")
+
+    def solve(nmodes, b, want):
+        with tb.Context(wl.Grid(nx, ny, nmodes, 2, 0.02, 1e-3, 1.002, 0.0, b)) as ctx:
+            if shape:
+                ctx.set_line_shape(0, 1, shape)
+            f = one.expand(nmodes, ny, nx).contiguous()
+            v = torch.zeros_like(f)
+            torch.cuda.synchronize()
+            ctx.solve_rhs_dev(f.data_ptr(), v.data_ptr(), 0.0, precision=0, max_cycles=2, guess=1)
+            return [v[k].cpu().numpy() for k in want]
+
+    modes = (1, K // 2, K - 2, K - 1)
+    for k, got in zip(modes, solve(K, beta, modes)):
+        ref = solve(2, k * beta, (1,))[0]
+        assert np.max(np.abs(got - ref)) < 1e-12 * np.max(np.abs(ref)), k
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "fp32"])
+def test_colour_phases_of_a_large_coarsest_level(torch_mod, precision):
+    """A coarsest level past the LDS takes a launch per colour phase: direct with
+    16, 32 and 64 lanes (a wavefront's lines of two modes and kinds) and staged, the
+    iterates after two cycles to rounding (1e-12; FP32 corrections 1e-5)."""
+    import trans_bl_amd as tb
+    g = wl.Grid(257, 161, 3, 2, 0.02, 5e-4, 1.01, 0.0, 0.3)        # coarsest 129x81
+    f = wl.wavepacket_rhs(g, tag="phases")
+    u = 0.01 * wl.wavepacket_rhs(g, tag="start")
+    out = []
+    with tb.Context(g) as ctx:
+        for shape in (16, 32, 64, -16, 2032):
+            ctx.set_line_shape(precision, 2, shape)
+            out.append(ctx.poi_uy(None, -f, u, 0.0, precision=precision, max_cycles=2)[0])
+    for o in out[1:]:
+        assert np.max(np.abs(o - out[0])) < (1e-12 if precision == 0 else 1e-5) * np.max(np.abs(out[0]))

@@ -167,17 +167,9 @@ __device__ __forceinline__ LineLU<T, R> load_line_lu_buf(__amdgpu_buffer_rsrc_t 
 // solve of 1025x193x64 7.09 -> 6.86 ms.
 template <typename T, int G, int R>
 constexpr int kLuPackBytes = lu_pack_line(sizeof(T), G, R) * static_cast<int>(sizeof(T));
-template <typename T, int G, int R>
-__device__ __forceinline__ LineLU<T, R> load_line_lu_packed(__amdgpu_buffer_rsrc_t rs, unsigned off0,
-                                                           int lane)
+template <typename T, int R>
+__device__ __forceinline__ LineLU<T, R> unpack_line_lu(const T *v)
 {
-    constexpr int NCH = lu_pack_chunks(sizeof(T), R), CV = 16 / sizeof(T);
-    T v[NCH * CV];
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, off0 + lane * 16u, q * G * 16, 0);
-        __builtin_memcpy(v + q * CV, &x, sizeof(x));
-    }
     LineLU<T, R> f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -191,6 +183,32 @@ __device__ __forceinline__ LineLU<T, R> load_line_lu_packed(__amdgpu_buffer_rsrc
         f.pv[r] = kIsF32<T> ? T(1) : v[7 * R + r];       // FP32 multiplies by 1 / p
     }
     return f;
+}
+template <typename T, int G, int R>
+__device__ __forceinline__ LineLU<T, R> load_line_lu_packed(__amdgpu_buffer_rsrc_t rs, unsigned off0,
+                                                           int lane)
+{
+    constexpr int NCH = lu_pack_chunks(sizeof(T), R), CV = 16 / sizeof(T);
+    T v[NCH * CV];
+#pragma unroll
+    for (int q = 0; q < NCH; ++q) {
+        const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rs, off0 + lane * 16u, q * G * 16, 0);
+        __builtin_memcpy(v + q * CV, &x, sizeof(x));
+    }
+    return unpack_line_lu<T, R>(v);
+}
+// from a pointer to the line's table, for tables past a resource's 4 GB
+template <typename T, int G, int R>
+__device__ __forceinline__ LineLU<T, R> load_line_lu_packed(const T *__restrict__ line, int lane)
+{
+    constexpr int NCH = lu_pack_chunks(sizeof(T), R), CV = 16 / sizeof(T);
+    T v[NCH * CV];
+#pragma unroll
+    for (int q = 0; q < NCH; ++q) {
+        const u32x4 x = reinterpret_cast<const u32x4 *>(line)[q * G + lane];
+        __builtin_memcpy(v + q * CV, &x, sizeof(x));
+    }
+    return unpack_line_lu<T, R>(v);
 }
 template <typename T, int G, int R>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t lu_packed_rsrc(const T *pk, int K)

@@ -20,7 +20,7 @@ __global__ void __launch_bounds__(256) smooth_phase_kernel(LevelArgs<T> L, cx<T>
     const int side = (phase == 0) ? (c == 0 ? -1 : 1) : 0;
     const size_t base = static_cast<size_t>(k) * L.plane + static_cast<size_t>(i) * L.ld;
     const LineLU<T, R> f = load_line_lu_packed<T, G, R>(
-        lu_packed_rsrc<T, G, R>(lu, L.K), (k * 2u + (side != 0)) * kLuPackBytes<T, G, R>, lane);
+        lu + (static_cast<size_t>(k) * 2 + (side != 0)) * lu_pack_line(sizeof(T), G, R), lane);
     relax_line<T, G, R>(L, V + base, S + base, f, side, rf, lane);
 }
 
@@ -259,13 +259,17 @@ template <typename T>
 int phase_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps, T rf,
                  const int *active, int G, hipStream_t st, bool zero_start, cx<double> *vup)
 {
-    const int form = G < 0 ? 1 : G > kXStagedShape ? 2 : 0;
+    int form = G < 0 ? 1 : G > kXStagedShape ? 2 : 0;
     if ((zero_start || vup) && form != 1) return TBL_ERR_ARG;
     if (vup && sizeof(T) != 4) return TBL_ERR_ARG;   // the update variant is FP32 only
     G = form == 1 ? -G : form == 2 ? G - kXStagedShape : G;
     const int R = line_rows_for(G, L.ny);
     if (R < 0) return TBL_ERR_GRID;
     lu += lu_pack_offset(sizeof(T), L.K, L.ny, L.lus, G);
+    // the staged forms read the factors through one buffer resource (FP64 past 4 GB
+    // from 40000 modes of 833 rows; FP32 tables stay below)
+    if (sizeof(T) == 8 && sizeof(T) * 2 * L.K * static_cast<size_t>(lu_pack_line(sizeof(T), G, R)) >= size_t{1} << 32)
+        form = 0;
     if (form == 1 && staged_lds<true>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
     if (form == 2 && staged_lds<false>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
     for (int it = 0; it < sweeps; ++it)

@@ -166,6 +166,33 @@ def test_line_factors_past_4_gigabytes(torch_mod, shape):
     torch.cuda.empty_cache()
 
 
+def test_x_derivatives_of_many_lines(torch_mod):
+    """35 million x-lines, whose threads are past 2^32: every mode of a field of
+    equal modes has the first one's derivatives."""
+    torch = torch_mod
+    import trans_bl_amd as tb
+    if torch.cuda.mem_get_info()[0] < 140 << 30:
+        pytest.skip("needs 140 GiB of device memory")
+    nx, ny, K = 15, 545, 64000
+    rng = np.random.default_rng(6)
+    one = torch.from_numpy(rng.normal(size=(1, ny, nx)) + 1j * rng.normal(size=(1, ny, nx))).to("cuda")
+    f = one.expand(K, ny, nx).contiguous()
+    a, b = torch.zeros_like(f), torch.zeros_like(f)
+    with tb.Context(wl.Grid(nx, ny, K, 2, 0.02, 1e-3, 1.002, 0.0, 1e-4)) as ctx:
+        torch.cuda.synchronize()
+        ctx.derivs_dev(f.data_ptr(), a.data_ptr(), b.data_ptr(), 0, 0)
+        ctx.synchronize()
+        for o in (a, b):
+            assert torch.any(o[0] != 0) and all(torch.equal(o[k], o[0]) for k in range(0, K, 777))
+        a.zero_()
+        torch.cuda.synchronize()
+        ctx.deriv_dev(tb.DERIV_KINDS["x"], f.data_ptr(), a.data_ptr())
+        ctx.synchronize()
+        assert torch.any(a[0] != 0) and all(torch.equal(a[k], a[0]) for k in range(0, K, 777))
+    del f, a, b
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "fp32"])
 def test_colour_phases_of_a_large_coarsest_level(torch_mod, precision):
     """A coarsest level past the LDS takes a launch per colour phase: direct with

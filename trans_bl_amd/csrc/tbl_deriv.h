@@ -354,6 +354,15 @@ __host__ __device__ constexpr int y_stride(int rows) { return rows + 32 / TX; }
 #define TBL_Y_SHAPES(X) \
     X(16, 3) X(16, 5) X(16, 7) X(16, 9) X(32, 5) X(32, 7) X(32, 9) X(64, 5) X(64, 7) X(64, 9)
 
+// workgroups, one per x-line: a dimension's threads are counted in 32 bits, so from
+// 2^20 lines on in rows of that many
+inline dim3 line_grid(size_t lines)
+{
+    const size_t row = lines < (size_t{1} << 20) ? lines : size_t{1} << 20;
+    return dim3(static_cast<unsigned>(row), static_cast<unsigned>((lines + row - 1) / row));
+}
+__device__ __forceinline__ unsigned line_index() { return (blockIdx.y << 20) + blockIdx.x; }
+
 // longest x-line accepted (ptsx), below the 64 * 9 * 4 points the shapes hold
 constexpr int kDerivMaxNx = 2112;
 inline bool x_shape(int nx, int *R, int *W)

@@ -46,7 +46,7 @@ namespace tbl {
 // From 3 wavefronts per part the registers are held to 4 wavefronts a SIMD: two
 // workgroups a CU (2049x257x32: 276 -> 198 us; below that it only spilled).
 template <int R, int W, bool D1, bool D2>
-__device__ __forceinline__ void deriv_x_line(const DerivArgs &A, int block, const C *f, C *o1, C *o2)
+__device__ __forceinline__ void deriv_x_line(const DerivArgs &A, unsigned block, const C *f, C *o1, C *o2)
 {
     constexpr int NT = 128 * W, N = (R + 1) / 2, LP = 64 * R * W + 4;
     __shared__ double planes[2 * LP], maps[16 * W], tab[kXTab];
@@ -102,7 +102,8 @@ template <int R, int W, bool D1, bool D2>
 __global__ void __launch_bounds__(128 * W, W >= 3 ? 4 : 1)
     deriv_x_kernel(DerivArgs A, const C *__restrict__ f, C *__restrict__ o1, C *__restrict__ o2)
 {
-    deriv_x_line<R, W, D1, D2>(A, static_cast<int>(blockIdx.x), f, o1, o2);
+    const unsigned line = line_index();
+    if (line < static_cast<unsigned>(A.ny) * A.K) deriv_x_line<R, W, D1, D2>(A, line, f, o1, o2);
 }
 
 // y-lines: o1 = d/dy (fv: with the wall row forced, deryfv), o2 = d2/dy2 of f.
@@ -286,7 +287,7 @@ static int deriv_x(const DerivArgs &A, const C *f, C *o1, C *o2, hipStream_t st)
 {
     int R = 0, W = 0;
     if (!x_shape(A.nx, &R, &W)) return TBL_ERR_GRID;
-    const dim3 grid(static_cast<unsigned>(A.ny) * static_cast<unsigned>(A.K));
+    const dim3 grid = line_grid(static_cast<size_t>(A.ny) * A.K);
 #define X(RR, WW)                                                                              \
     if (R == RR && W == WW) {                                                                  \
         const dim3 block(128 * WW);                                                            \

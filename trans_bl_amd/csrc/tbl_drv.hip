@@ -121,8 +121,8 @@ __global__ void __launch_bounds__(128 * W, W >= 2 ? 4 : 1) drv_x_kernel(DerivArg
     const int t = threadIdx.x, lane = t & 63;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int part = wv / W, w = wv % W;
-    const int nx = A.nx, rows = A.ny - 1;
-    const int k = static_cast<int>(blockIdx.x) / rows, j = 1 + static_cast<int>(blockIdx.x) % rows;
+    const int nx = A.nx, rows = A.ny - 1, m = static_cast<int>(line_index()), k = m / rows, j = 1 + m % rows;
+    if (k >= A.K) return;
     const size_t line = (static_cast<size_t>(k) * A.ny + j) * nx, line2 = static_cast<size_t>(j) * nx;
     auto load = [&](const C *p, C (&v)[N]) {
         const __amdgpu_buffer_rsrc_t s = buf_rsrc(p + line, static_cast<size_t>(nx) * sizeof(C));
@@ -288,7 +288,7 @@ void launch_x(const DerivArgs &A, const DrvArgs &r, hipStream_t st)
 {
     int R = 0, W = 0;
     x_shape(A.nx, &R, &W);
-    const dim3 grid(static_cast<unsigned>(A.ny - 1) * static_cast<unsigned>(A.K));
+    const dim3 grid = line_grid(static_cast<size_t>(A.ny - 1) * A.K);
 #define X(RR, WW)           \
     if (R == RR && W == WW) \
         hipLaunchKernelGGL((drv_x_kernel<RR, WW, Q, LIN>), grid, dim3(128 * WW), 0, st, A, r);

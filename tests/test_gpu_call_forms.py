@@ -166,6 +166,40 @@ def test_line_factors_past_4_gigabytes(torch_mod, shape):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("shape,precision,nx,ny,K", [
+    (-64, 0, 15, 17, 1300000), (-64, 1, 15, 17, 1300000), (2064, 0, 15, 17, 1300000),
+    (1064, 0, 15, 17, 1300000), (1064, 1, 15, 17, 1300000)])
+def test_line_factors_of_a_million_modes(torch_mod, shape, precision, nx, ny, K):
+    """Lines of 64 lanes whose factors, 8 kB a mode in FP64 and 3.6 to 4 in FP32, take
+    two or three ranges of modes a sweep: staged and strips.  Two cycles
+    of modes in and next to the ranges against a context of two modes with the
+    same kz (1e-12; FP32 corrections 1e-5)."""
+    torch = torch_mod
+    import trans_bl_amd as tb
+    if torch.cuda.mem_get_info()[0] < 200 << 30:
+        pytest.skip("needs 200 GiB of device memory")
+    beta = 1e-5
+    rng = np.random.default_rng(7)
+    one = torch.from_numpy(rng.normal(size=(1, ny, nx)) + 1j * rng.normal(size=(1, ny, nx))).to("cuda")
+
+    def solve(nmodes, b, want):
+        with tb.Context(wl.Grid(nx, ny, nmodes, 2, 0.02, 1e-2, 1.02, 0.0, b)) as ctx:
+            ctx.set_line_shape(precision, 1, shape)
+            f = one.expand(nmodes, ny, nx).contiguous()
+            v = torch.zeros_like(f)
+            torch.cuda.synchronize()
+            ctx.solve_rhs_dev(f.data_ptr(), v.data_ptr(), 0.0, precision=precision, max_cycles=2, guess=1)
+            return [v[k].cpu().numpy() for k in want]
+
+    each = 4096 if precision and shape > 1000 else 3584 if precision else 8192   # bytes a mode
+    most = (2 ** 32 - 1) // each
+    modes = (1, most - 1, most, most + 1, K // 2 + 1, K - 2, K - 1)
+    for k, got in zip(modes, solve(K, beta, modes)):
+        ref = solve(2, k * beta, (1,))[0]
+        assert np.max(np.abs(got - ref)) < (1e-12 if precision == 0 else 1e-5) * np.max(np.abs(ref)), k
+    torch.cuda.empty_cache()
+
+
 def test_x_derivatives_of_many_lines(torch_mod):
     """35 million x-lines, whose threads are past 2^32: every mode of a field of
     equal modes has the first one's derivatives."""

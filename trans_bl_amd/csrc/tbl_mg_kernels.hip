@@ -517,11 +517,11 @@ __global__ void fill_int_kernel(int *p, int n, int v)
 
 __global__ void __launch_bounds__(256) narrow_kernel(const double *__restrict__ a, float *__restrict__ b, size_t n)
 {
-    const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i < n) b[i] = static_cast<float>(a[i]);
+    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * 256)
+        b[i] = static_cast<float>(a[i]);
 }
 
-// The packed tables of G lanes with R rows each, one value per thread.  (As a
+// The packed tables of G lanes with R rows each, a value per thread and step.  (As a
 // loop on the host, with four times the bytes to upload, this was most of a
 // context's creation: 2049x257x128 18 ms, 4.9 here, 4.6 with the rows' form alone;
 // 65x257x128 14, 3.1 and 2.9.)
@@ -530,13 +530,13 @@ __global__ void __launch_bounds__(256) pack_line_lu_kernel(const T *__restrict__
                                                            size_t n, int lus, int G, int R)
 {
     constexpr int NF = lu_pack_values(sizeof(T)), CV = 16 / sizeof(T);
-    const size_t e = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (e >= n) return;
     const int size = lu_pack_line(sizeof(T), G, R);
-    const int x = static_cast<int>(e % size), lane = x / CV % G, v = x / (CV * G) * CV + x % CV;
-    // value v / R: l1, l2, u1, u2, -u1/p, -u2/p, 1/p, p
-    const int q = v / R, field = q < 4 ? q : q < 7 ? q + 1 : 4;
-    pk[e] = q < NF ? rows[(e / size * kLuFields + field) * lus + 1 + lane * R + v % R] : T(0);
+    for (size_t e = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; e < n; e += static_cast<size_t>(gridDim.x) * 256) {
+        const int x = static_cast<int>(e % size), lane = x / CV % G, v = x / (CV * G) * CV + x % CV;
+        // value v / R: l1, l2, u1, u2, -u1/p, -u2/p, 1/p, p
+        const int q = v / R, field = q < 4 ? q : q < 7 ? q + 1 : 4;
+        pk[e] = q < NF ? rows[(e / size * kLuFields + field) * lus + 1 + lane * R + v % R] : T(0);
+    }
 }
 
 // dst = src on the modes whose activity is `want`
@@ -636,6 +636,7 @@ size_t lu_pack_offset(int esize, int K, int ny, int lus, int G)
     return o;
 }
 
+static unsigned table_blocks(size_t n) { return static_cast<unsigned>(n < (size_t{1} << 28) ? (n + 255) / 256 : 1u << 20); }
 template <typename T>
 static void pack_line_lu(T *lu, int K, int ny, int lus, hipStream_t st)
 {
@@ -643,14 +644,14 @@ static void pack_line_lu(T *lu, int K, int ny, int lus, hipStream_t st)
         const int R = line_rows_for(G, ny);
         if (R <= 0) continue;
         const size_t n = static_cast<size_t>(K) * 2 * lu_pack_line(sizeof(T), G, R);
-        hipLaunchKernelGGL((pack_line_lu_kernel<T>), dim3(nblk(n)), dim3(256), 0, st, lu,
+        hipLaunchKernelGGL((pack_line_lu_kernel<T>), dim3(table_blocks(n)), dim3(256), 0, st, lu,
                            lu + lu_pack_offset(sizeof(T), K, ny, lus, G), n, lus, G, R);
     }
 }
 void prepare_line_lu(double *lu, float *luf, int K, int ny, int lus, hipStream_t st)
 {
     const size_t n = static_cast<size_t>(K) * 2 * kLuFields * lus;
-    hipLaunchKernelGGL(narrow_kernel, dim3(nblk(n)), dim3(256), 0, st, lu, luf, n);
+    hipLaunchKernelGGL(narrow_kernel, dim3(table_blocks(n)), dim3(256), 0, st, lu, luf, n);
     pack_line_lu(lu, K, ny, lus, st);
     pack_line_lu(luf, K, ny, lus, st);
 }

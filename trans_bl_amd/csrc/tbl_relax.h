@@ -210,6 +210,23 @@ __device__ __forceinline__ LineLU<T, R> load_line_lu_packed(const T *__restrict_
     }
     return unpack_line_lu<T, R>(v);
 }
+// The smoothers that read the factors through one buffer resource run over as many
+// modes at a time as its 4 GB hold: `each` bytes a mode (FP64, 545 rows: 58200 modes).
+// One-launch sweeps need no ranges: their two buffers stay below 2 GB, and on the
+// smallest grid, 15x9, the factors are then 2.3 GB.
+inline int modes_of_resource(int K, size_t each)
+{
+    const size_t most = ((size_t{1} << 32) - 1) / each;
+    return static_cast<size_t>(K) > most ? static_cast<int>(most) : K;
+}
+// the modes from k0 on
+template <typename T>
+LevelArgs<T> mode_range(const LevelArgs<T> &L, int k0, int modes)
+{
+    LevelArgs<T> part = L;
+    part.K = L.K - k0 < modes ? L.K - k0 : modes;
+    return part;
+}
 template <typename T, int G, int R>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t lu_packed_rsrc(const T *pk, int K)
 {

@@ -251,27 +251,12 @@ static void launch_full(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T
     launch_staged<T, G, R, true>(L, V, S, lu, phase, rf, active, st, zs, nullptr);
 }
 
-// One colour phase per launch.  G > 0: lanes per line with direct
-// (lane-contiguous) global access; G < 0: |G| lanes per line, x terms, v
-// and S staged in LDS; G > kXStagedShape: G - kXStagedShape lanes per line,
-// only the x terms staged.
+// the sweeps of phase_sweeps on one range of modes, lu their packed factors
 template <typename T>
-int phase_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps, T rf,
-                 const int *active, int G, hipStream_t st, bool zero_start, cx<double> *vup)
+static int phase_sweeps_part(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps,
+                             T rf, const int *active, int G, int R, int form, hipStream_t st,
+                             bool zero_start, cx<double> *vup)
 {
-    int form = G < 0 ? 1 : G > kXStagedShape ? 2 : 0;
-    if ((zero_start || vup) && form != 1) return TBL_ERR_ARG;
-    if (vup && sizeof(T) != 4) return TBL_ERR_ARG;   // the update variant is FP32 only
-    G = form == 1 ? -G : form == 2 ? G - kXStagedShape : G;
-    const int R = line_rows_for(G, L.ny);
-    if (R < 0) return TBL_ERR_GRID;
-    lu += lu_pack_offset(sizeof(T), L.K, L.ny, L.lus, G);
-    // the staged forms read the factors through one buffer resource (FP64 past 4 GB
-    // from 40000 modes of 833 rows; FP32 tables stay below)
-    if (sizeof(T) == 8 && sizeof(T) * 2 * L.K * static_cast<size_t>(lu_pack_line(sizeof(T), G, R)) >= size_t{1} << 32)
-        form = 0;
-    if (form == 1 && staged_lds<true>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
-    if (form == 2 && staged_lds<false>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
     for (int it = 0; it < sweeps; ++it)
         for (int ph = 0; ph < 4; ++ph) {
             bool done = false;
@@ -288,6 +273,36 @@ int phase_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, i
 #undef X
             if (!done) return TBL_ERR_GRID;
         }
+    return TBL_OK;
+}
+
+// One colour phase per launch.  G > 0: lanes per line with direct
+// (lane-contiguous) global access; G < 0: |G| lanes per line, x terms, v
+// and S staged in LDS; G > kXStagedShape: G - kXStagedShape lanes per line,
+// only the x terms staged.
+template <typename T>
+int phase_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, int sweeps, T rf,
+                 const int *active, int G, hipStream_t st, bool zero_start, cx<double> *vup)
+{
+    const int form = G < 0 ? 1 : G > kXStagedShape ? 2 : 0;
+    if ((zero_start || vup) && form != 1) return TBL_ERR_ARG;
+    if (vup && sizeof(T) != 4) return TBL_ERR_ARG;   // the update variant is FP32 only
+    G = form == 1 ? -G : form == 2 ? G - kXStagedShape : G;
+    const int R = line_rows_for(G, L.ny);
+    if (R < 0) return TBL_ERR_GRID;
+    if (form == 1 && staged_lds<true>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
+    if (form == 2 && staged_lds<false>(L.ld, sizeof(cx<T>)) > 160 * 1024) return TBL_ERR_GRID;
+    lu += lu_pack_offset(sizeof(T), L.K, L.ny, L.lus, G);
+    // the direct form reads the factors through a pointer
+    const size_t mode_lu = 2 * static_cast<size_t>(lu_pack_line(sizeof(T), G, R));
+    const int modes = form ? modes_of_resource(L.K, mode_lu * sizeof(T)) : L.K;
+    for (int k0 = 0; k0 < L.K; k0 += modes) {
+        const size_t at = k0 * L.plane;
+        const int rc = phase_sweeps_part<T>(mode_range(L, k0, modes), V + at, S + at, lu + k0 * mode_lu,
+                                            sweeps, rf, active ? active + k0 : nullptr, G, R, form, st,
+                                            zero_start, vup ? vup + at : nullptr);
+        if (rc != TBL_OK) return rc;
+    }
     return TBL_OK;
 }
 

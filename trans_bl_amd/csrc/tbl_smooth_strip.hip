@@ -191,11 +191,17 @@ int strip_sweeps(const LevelArgs<T> &L, cx<T> *V, const cx<T> *S, const T *lu, i
     const int R = line_rows_for(G, L.ny);
     const StripGeom sg = strip_geom(L.nx, L.ny, L.K, sizeof(T));
     if (R < 0 || sg.nstrips < 1 || (sg.nstrips > 1 && !halo)) return TBL_ERR_GRID;
+    const size_t mode_lu = size_t{2} * kLuFields * L.lus;
+    const int modes = modes_of_resource(L.K, mode_lu * sizeof(T));
     for (int it = 0; it < sweeps; ++it) {
         bool done = false;
 #define X(GG, RR)                                                                       \
     if (!done && G == GG && R == RR) {                                                  \
-        launch_strip<T, GG, RR>(L, V, S, lu, halo, sg, rf, active, st);                 \
+        for (int k0 = 0; k0 < L.K; k0 += modes) {                                       \
+            const size_t at = k0 * L.plane;                                             \
+            launch_strip<T, GG, RR>(mode_range(L, k0, modes), V + at, S + at, lu + k0 * mode_lu, halo, \
+                                    sg, rf, active ? active + k0 : nullptr, st);        \
+        }                                                                               \
         done = true;                                                                    \
     }
         TBL_LINE_SHAPES(X)
